@@ -31,6 +31,9 @@ __device__ __forceinline__ uint32_t deq_pair(uint32_t bits, half2_t d2) {
     return __builtin_bit_cast(uint32_t, (magic - off) * d2);
 }
 
+// Any K % 32 == 0, no workspace: what a product that fits neither panel kernel runs on -- a K that is no multiple of 256 (or
+// weights that are not 16-byte aligned) while a graph is captured and the workspace is still too small, or operands past
+// 32-bit panel offsets (77 x 3200 x 8640: 93 us against 19.8 us on the skinny kernel).
 __global__ __launch_bounds__(256) void gemm_q4_0_mfma_v1(const uint8_t *__restrict__ W, const float *__restrict__ X,
                                                           float *__restrict__ Y, int K, int N, int M) {
     __shared__ __attribute__((aligned(16))) _Float16 As[TM * LDS_STRIDE];
@@ -164,22 +167,22 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 // at ((m16 * K/32) + kb) * 1 KB, and inside a tile the 16-byte run k = kb*32 + kg*8 .. +7 of row
 // m16*16 + r at (kg * 16 + r) * 16 bytes.  Lane l = kg * 16 + r of a wave owns exactly that run in
 // v_mfma_f32_16x16x32_f16, so a fragment load is 64 consecutive 16-byte pieces: one contiguous KB.
-// Rows past M (the last tile of a ragged M) are written as zeros.
+// Rows past M (the last tile of a ragged M) are written as zeros, and so are the k-blocks past K of a panel whose rows are
+// kblocks long (a K that is no multiple of the kernels' pieces).
 // SWIGLU: the panel receives silu(x) * up instead of x (silu_f32 then mul_f32, unary.cu:1-10, mul.cu:3-12, with the
 // arithmetic of galois_hip_silu_mul_f32), so that a down projection needs neither that launch nor the conversion.
 template <bool SWIGLU>
 __global__ __launch_bounds__(256) void f32_to_f16_tiles(const float *__restrict__ x, const float *__restrict__ up,
-                                                        _Float16 *__restrict__ y, int M, int K, int64_t nchunks) {
+                                                        _Float16 *__restrict__ y, int M, int K, int kblocks, int64_t nchunks) {
     const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;  // 16-byte output chunk
     if (o >= nchunks) return;
     const int64_t tile = o >> 6;
     const int c = (int)(o & 63), kg = c >> 4, r = c & 15;
-    const int kblocks = K / 32;
     const int64_t m16 = tile / kblocks;
     const int kb = (int)(tile - m16 * kblocks);
     const int64_t m = m16 * 16 + r;
     uint4 out = make_uint4(0, 0, 0, 0);
-    if (m < M) {
+    if (m < M && kb * 32 < K) {
         const float4 *src = reinterpret_cast<const float4 *>(x + m * K + kb * 32 + kg * 8);
         float4 a = src[0], b = src[1];
         if (SWIGLU) {
@@ -751,6 +754,12 @@ int32_t gemm_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *
     return GALOIS_HIP_OK;
 }
 
+}  // namespace
+
+#include "gemm_q4_0_skinny.h"
+
+namespace {
+
 // Tile width by how many workgroups it gives the device.  Cost model: rounds of workgroups over the CUs
 // times the relative cost of a k-stage (a 48-column stage has half the matrix instructions and half
 // the dequantisation of a 96-column one but the same barriers and A requests: ~0.65).
@@ -766,6 +775,7 @@ void gemm_concat(gemm_mats &mats, int n_mats) {
 
 int32_t gemm_launch_any(galois_hip_ctx *ctx, gemm_mats mats, int n_mats, const _Float16 *Xh, int K, int M) {
     gemm_concat(mats, n_mats);
+    if (M <= SK_MAX_ROWS) return skinny_launch_any(ctx, mats, Xh, K, K / 32, M, true);
     const int64_t cols = mats.n_total;
     const int64_t m_tiles = (M + GM - 1) / GM;
     const int64_t wg96 = (cols + 95) / 96 * m_tiles, wg48 = (cols + 47) / 48 * m_tiles;
@@ -778,14 +788,14 @@ int32_t gemm_launch_any(galois_hip_ctx *ctx, gemm_mats mats, int n_mats, const _
 // whose byte offsets fit 32 bits.
 bool gemm_panel_shape_ok(int64_t K, int64_t M) { return K > 0 && M > 0 && K % 256 == 0 && (M + 16) * K * 2 < ((int64_t)1 << 32); }
 
-int32_t launch_to_panel(galois_hip_ctx *ctx, const float *x, const float *up, _Float16 *panel, int K, int M, bool swiglu) {
+int32_t launch_to_panel(galois_hip_ctx *ctx, const float *x, const float *up, _Float16 *panel, int K, int kblocks, int M, bool swiglu) {
     const int64_t m_pad = ((int64_t)M + 15) / 16 * 16;
-    const int64_t nchunks = m_pad * K / 8;
+    const int64_t nchunks = m_pad * kblocks * 4;
     const dim3 grid((unsigned)((nchunks + 255) / 256)), block(256);
     if (swiglu)
-        hipLaunchKernelGGL(f32_to_f16_tiles<true>, grid, block, 0, ctx->stream, x, up, panel, M, K, nchunks);
+        hipLaunchKernelGGL(f32_to_f16_tiles<true>, grid, block, 0, ctx->stream, x, up, panel, M, K, kblocks, nchunks);
     else
-        hipLaunchKernelGGL(f32_to_f16_tiles<false>, grid, block, 0, ctx->stream, x, up, panel, M, K, nchunks);
+        hipLaunchKernelGGL(f32_to_f16_tiles<false>, grid, block, 0, ctx->stream, x, up, panel, M, K, kblocks, nchunks);
     return GALOIS_HIP_OK;
 }
 
@@ -804,6 +814,7 @@ bool gemm_two_shares_pay(const galois_hip_ctx *ctx, int K, int N, int M, double 
     const int64_t m_tiles = (M + GM - 1) / GM, cus = ctx->n_cu > 0 ? ctx->n_cu : 256, stages = K / 64;
     const int64_t wg96 = ((int64_t)N + 95) / 96 * m_tiles, wg48 = ((int64_t)N + 47) / 48 * m_tiles, wg64x2 = ((int64_t)N + 63) / 64 * m_tiles * 2;
     const int64_t mn = (int64_t)M * N;
+    if (M <= SK_MAX_ROWS) return false;
     const double c96 = (double)((wg96 + cus - 1) / cus) * stages, c48 = 0.65 * (double)((wg48 + cus - 1) / cus) * stages;
     const double c64x2 = 0.75 * (double)((wg64x2 + cus - 1) / cus) * (stages / 2 + 2) + 14.0 * (double)mn / (double)(1 << 21);
     return K >= 512 && mn % 4 == 0 && margin * c64x2 < c96 && margin * c64x2 < c48 && c96 >= min_cost && c48 >= min_cost;
@@ -829,29 +840,50 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
     GH_REQUIRE(ctx, gh_aligned(W, 2) && gh_aligned(X, 16) && gh_aligned(Y, 4), GALOIS_HIP_E_ALIGN,
                "mul_mat_q4_0_f32: W 2-byte, X 16-byte, Y 4-byte aligned");
     GH_BIND(ctx);
-    if (gemm_panel_shape_ok(K, M) && gh_aligned(W, 16)) {
-        // fp16 copy of X, tiled for the A fragments, in the context's workspace (grown on demand); behind it, for a
-        // matrix that is clearly better multiplied as two shares of k (512 x 11008 x 4096: 65 -> 47 us + a 5.7 us adding
-        // pass), room for the two partial results
-        const int64_t m_pad = ((int64_t)M + 15) / 16 * 16, mn = (int64_t)M * N;
-        const size_t panel_bytes = ((size_t)m_pad * K * sizeof(_Float16) + 255) & ~(size_t)255;
-        const bool shares = mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_two_shares_pay(ctx, K, N, M, 1.1, 64.0);
-        const size_t need = panel_bytes + (shares ? 2 * (size_t)mn * sizeof(float) : 0);
-        if (ctx->ws_bytes < need) {
+    // fp16 copy of X, tiled for the activation fragments, in the context's workspace (grown on demand), its rows padded
+    // with zeros to whole pieces of 256; behind it, for a matrix that is clearly better multiplied as two shares of k
+    // (512 x 11008 x 4096: 65 -> 47 us + a 5.7 us adding pass), room for the two partial results
+    const int64_t m_pad = ((int64_t)M + 15) / 16 * 16, k_pad = ((int64_t)K + 255) / 256 * 256, mn = (int64_t)M * N;
+    const size_t panel_bytes = ((size_t)m_pad * k_pad * sizeof(_Float16) + 255) & ~(size_t)255;
+    const bool wide = K == k_pad && gh_aligned(W, 16);  // what the 256-row kernel asks of the weights
+    const bool skinny = !wide || M <= SK_MAX_ROWS;
+    const bool shares = !skinny && mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_two_shares_pay(ctx, K, N, M, 1.1, 64.0);
+    const size_t need = panel_bytes + (shares ? 2 * (size_t)mn * sizeof(float) : 0);
+    bool panel = gemm_panel_shape_ok((int32_t)k_pad, M);
+    if (panel && ctx->ws_bytes < need) {
+        // weights that are not laid out in pieces of 256 have a kernel that needs no workspace: while a graph is being
+        // captured they run on it rather than fail
+        if (!wide && ctx->capturing) {
+            panel = false;
+        } else {
             GH_NOT_CAPTURING(ctx, "mul_mat_q4_0_f32: growing the workspace");
             // The outgrown block is kept until the context dies: work already queued, or a graph captured earlier,
             // has its address baked in.  Growing by at least half bounds what the retired blocks add up to.
             const size_t bytes = need > ctx->ws_bytes + ctx->ws_bytes / 2 ? need : ctx->ws_bytes + ctx->ws_bytes / 2;
             void *grown = nullptr;
             const hipError_t e = hipMalloc(&grown, bytes);
-            if (e != hipSuccess) return gh_hip(ctx, e, "hipMalloc(workspace)");
-            if (ctx->ws) ctx->ws_retired.push_back(ctx->ws);
-            ctx->ws = grown;
-            ctx->ws_bytes = bytes;
+            if (e == hipSuccess) {
+                if (ctx->ws) ctx->ws_retired.push_back(ctx->ws);
+                ctx->ws = grown;
+                ctx->ws_bytes = bytes;
+            } else if (wide) {
+                return gh_hip(ctx, e, "hipMalloc(workspace)");
+            } else {
+                (void)hipGetLastError();
+                panel = false;
+            }
         }
+    }
+    if (panel) {
         _Float16 *Xh = (_Float16 *)ctx->ws;
-        launch_to_panel(ctx, X, nullptr, Xh, K, M, false);
-        if (shares) {
+        launch_to_panel(ctx, X, nullptr, Xh, K, (int)(k_pad / 32), M, false);
+        if (skinny) {
+            gemm_mats mats = {};
+            mats.W[0] = (const uint8_t *)W, mats.Y[0] = Y, mats.N[0] = N;
+            gemm_concat(mats, 1);
+            const int32_t st = skinny_launch_any(ctx, mats, Xh, K, (int)(k_pad / 32), M, K % 64 == 0 && gh_aligned(W, 4));
+            if (st != GALOIS_HIP_OK) return st;
+        } else if (shares) {
             float *parts = reinterpret_cast<float *>(static_cast<unsigned char *>(ctx->ws) + panel_bytes);
             const int32_t st = gemm_launch_shares(ctx, W, Xh, parts, K, N, M, 2);
             if (st != GALOIS_HIP_OK) return st;
@@ -894,7 +926,7 @@ extern "C" int32_t galois_hip_f32_to_f16_panel(galois_hip_ctx *ctx, const float 
     const int32_t st = panel_args(ctx, x, x, panel, ncols, nrows, "f32_to_f16_panel");
     if (st != GALOIS_HIP_OK) return st;
     GH_BIND(ctx);
-    launch_to_panel(ctx, x, nullptr, (_Float16 *)panel, ncols, nrows, false);
+    launch_to_panel(ctx, x, nullptr, (_Float16 *)panel, ncols, ncols / 32, nrows, false);
     GH_LAUNCH_CHECK(ctx, "f32_to_f16_panel launch");
 }
 
@@ -903,7 +935,7 @@ extern "C" int32_t galois_hip_silu_mul_f16_panel(galois_hip_ctx *ctx, const floa
     const int32_t st = panel_args(ctx, gate, up, panel, ncols, nrows, "silu_mul_f16_panel");
     if (st != GALOIS_HIP_OK) return st;
     GH_BIND(ctx);
-    launch_to_panel(ctx, gate, up, (_Float16 *)panel, ncols, nrows, true);
+    launch_to_panel(ctx, gate, up, (_Float16 *)panel, ncols, ncols / 32, nrows, true);
     GH_LAUNCH_CHECK(ctx, "silu_mul_f16_panel launch");
 }
 
@@ -1055,7 +1087,8 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_swiglu_f16_panel(galois_hip_ctx *ctx,
     for (int j = 0; j < GEMM_MAX_MATS; j++) mats.col0[j] = 0x7FFFFFFF;
     mats.n_total = 96 * ((N + 47) / 48);
     mats.swiglu_out = static_cast<_Float16 *>(panel_out);
-    const int32_t st = gemm_launch<96>(ctx, mats, (const _Float16 *)panel, K, M);
+    const int32_t st = M <= SK_MAX_ROWS ? skinny_launch_any(ctx, mats, (const _Float16 *)panel, K, K / 32, M, true)
+                                        : gemm_launch<96>(ctx, mats, (const _Float16 *)panel, K, M);
     if (st != GALOIS_HIP_OK) return st;
     GH_LAUNCH_CHECK(ctx, "mul_mat_q4_0_swiglu_f16_panel launch");
 }

@@ -1,0 +1,328 @@
+// Q4_0 matrices against a panel of few activation rows (part of gemm_q4_0.hip).
+//
+// What bounds it.  Up to about a hundred rows the weights' bytes do (512 flops a byte of HBM before the matrix pipe is
+// the limit), so the 256-row tile of the main kernel multiplies padding and its producer waves dequantise at the pace of
+// a tile that is never full.  Here every wave dequantises its own operand in registers and no barrier stands between
+// the weight stream and the matrix instructions:
+//   - A wave owns NT tiles of 16 weight rows and MT tiles of 16 activation rows; a workgroup's KS waves own the same tiles
+//     and take every KS-th piece of 256 k each; their sums meet in LDS at the end, in a fixed order.
+//   - v_mfma_f32_16x16x32_f16 adds over k in any order as long as both operands agree on it.  Lane (r, kg) of the
+//     weight operand therefore takes the whole 36-byte slot kg of the piece (two blocks of row r, as the
+//     decode kernel's lanes do): one piece = eight instructions, instruction (b, c) of which multiplies the eight weights k
+//     = 8c .. 8c+7 of block b of each lane's slot.  No shuffle, no LDS round trip, the block's scale is in the lane.
+//   - The activation operand is then the 16-byte run c of row r in panel tile 2 kg + b: four contiguous 256-byte pieces a
+//     request, from L2 (every workgroup reads the whole panel: NT rows of tiles share a fragment).
+//   - The result tile has the weight rows down its registers: a lane holds four consecutive columns of Y.
+// Measured (MI355X, us, weights from HBM, against the 256-row tile): see SK_MAX_ROWS.  77 rows of a 3200 x 8640 matrix through
+// the f32 entry point 93 -> 19.8 (the generic kernel before), a prefill of 23 tokens through 32 layers 4705 -> 2871.
+// Weights are rounded exactly as in the main kernel ((q - 8) * d, once, to fp16), sums are f32.
+#pragma once
+
+namespace {
+
+constexpr int SK_MAX_MT = 5;  // row tiles per wave: more would take the registers of the second wave per SIMD
+
+// A lane's share of a piece: two blocks, as they lie in memory.
+template <bool ALIGNED>
+struct sk_raw;
+
+template <>
+struct sk_raw<true> {  // K % 64 == 0 and W 4-byte aligned: one 36-byte slot
+    uint32_t w[9];
+};
+template <>
+struct sk_raw<false> {  // any 2-byte aligned block: its four aligned dwords and the two bytes before or behind them
+    uint32_t w[2][4];
+    uint32_t h[2];
+};
+
+// block: index of the lane's first block in its row (even); nblocks: blocks of the row.  Blocks past the end are
+// loaded from the row's last ones and given a zero scale by sk_blocks.
+__device__ __forceinline__ void sk_load(sk_raw<true> &q, const uint8_t *row, int block, int nblocks) {
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(row + (size_t)min(block, nblocks - 2) * 18);
+#pragma unroll
+    for (int i = 0; i < 9; i++) q.w[i] = p[i];
+}
+__device__ __forceinline__ void sk_load(sk_raw<false> &q, const uint8_t *row, int block, int nblocks) {
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const uint8_t *p = row + (size_t)min(block + b, nblocks - 1) * 18;
+        const bool odd = ((uintptr_t)p & 2) != 0;  // the block's d lies in front of an aligned dword: its qs are aligned
+        const uint32_t *w = reinterpret_cast<const uint32_t *>(odd ? p + 2 : p);
+#pragma unroll
+        for (int i = 0; i < 4; i++) q.w[b][i] = w[i];
+        q.h[b] = *reinterpret_cast<const uint16_t *>(odd ? p : p + 16);
+    }
+}
+
+struct sk_blocks {
+    uint32_t q[2][4];  // the nibble dwords of both blocks
+    half2_t d[2];
+};
+__device__ __forceinline__ void sk_unpack(sk_blocks &o, const sk_raw<true> &r, const uint8_t *, int block, int nblocks) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        o.q[0][i] = __builtin_amdgcn_alignbit(r.w[i + 1], r.w[i], 16);
+        o.q[1][i] = r.w[5 + i];
+    }
+    const bool in = block < nblocks;
+    const _Float16 a = __builtin_bit_cast(_Float16, (uint16_t)(in ? r.w[0] & 0xFFFFu : 0u));
+    const _Float16 b = __builtin_bit_cast(_Float16, (uint16_t)(in ? r.w[4] >> 16 : 0u));
+    o.d[0] = half2_t{a, a}, o.d[1] = half2_t{b, b};
+}
+__device__ __forceinline__ void sk_unpack(sk_blocks &o, const sk_raw<false> &r, const uint8_t *row, int block, int nblocks) {
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const bool odd = ((uintptr_t)(row + (size_t)min(block + b, nblocks - 1) * 18) & 2) != 0;
+        const uint32_t next[4] = {r.w[b][1], r.w[b][2], r.w[b][3], r.h[b]};
+#pragma unroll
+        for (int i = 0; i < 4; i++) o.q[b][i] = odd ? r.w[b][i] : __builtin_amdgcn_alignbit(next[i], r.w[b][i], 16);
+        const uint32_t bits = odd ? r.h[b] : r.w[b][0] & 0xFFFFu;
+        const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)(block + b < nblocks ? bits : 0u));
+        o.d[b] = half2_t{d, d};
+    }
+}
+
+// Weights k = 8c .. 8c+7 of a block as fp16: the low (c < 2) or high nibbles of the dwords 2 (c % 2) and 2 (c % 2) + 1.
+template <int C>
+__device__ __forceinline__ half8_t sk_operand(const uint32_t (&q)[4], half2_t d) {
+    const half2_t off = {(_Float16)1032.0f, (_Float16)1032.0f};
+    uint4 o;
+    uint32_t *ov = &o.x;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t v = q[2 * (C & 1) + i];
+        const uint32_t n = (C < 2 ? v : v >> 4) & 0x0F0F0F0Fu;
+        // 0x64nn is 1024 + nn: minus 1032 the exact integer n - 8, rounded once by the product with d
+        const half2_t a = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, n, 0x04010400u));
+        const half2_t b = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, n, 0x04030402u));
+        ov[2 * i] = __builtin_bit_cast(uint32_t, (a - off) * d);
+        ov[2 * i + 1] = __builtin_bit_cast(uint32_t, (b - off) * d);
+    }
+    return __builtin_bit_cast(half8_t, o);
+}
+
+// Instructions of a piece whose activation fragments are requested together: about eight fragments in flight a wave.
+constexpr int sk_steps(int mt) { return mt <= 1 ? 4 : mt <= 4 ? 2 : 1; }
+// Waves per SIMD the registers are kept to: four hide the requests' latency where the tiles allow it (2 x 2 tiles: 138 -> 110
+// registers, gate | up at 23 rows 21.4 -> 20.3 us).
+constexpr int sk_occ(int nt, int mt) {
+    const int regs = 4 * nt * mt + 8 * sk_steps(mt) * mt + 19 * nt + 40;
+    return regs <= 138 ? 4 : regs <= 175 ? 3 : 2;
+}
+
+// Where four consecutive columns of row m go: n is a column of the concatenated matrices.
+__device__ __forceinline__ void sk_store4(const gemm_mats &mats, int n, int m, float4_t v) {
+    if (n >= mats.n_total) return;
+    float *Y = mats.Y[0];
+    int N = mats.N[0], first = 0;
+#pragma unroll
+    for (int t = 1; t < GEMM_MAX_MATS; t++) {
+        const bool ge = n >= mats.col0[t];
+        Y = ge ? mats.Y[t] : Y, N = ge ? mats.N[t] : N, first = ge ? mats.col0[t] : first;
+    }
+    float *dst = Y + (size_t)m * N + (n - first);
+    if (n - first + 4 <= N && ((uintptr_t)dst & 15) == 0) {
+        *reinterpret_cast<float4_t *>(dst) = v;
+        return;
+    }
+    for (int e = 0; e < 4; e++) {  // a ragged or unaligned result, or four columns that go on in the next matrix
+        const int ne = n + e;
+        if (ne >= mats.n_total) return;
+        Y = mats.Y[0], N = mats.N[0], first = 0;
+        for (int t = 1; t < GEMM_MAX_MATS; t++)
+            if (ne >= mats.col0[t]) Y = mats.Y[t], N = mats.N[t], first = mats.col0[t];
+        Y[(size_t)m * N + (ne - first)] = v[e];
+    }
+}
+
+// K: the rows' true length (a multiple of 32); kp_blocks: 32-k blocks of a panel row, a multiple of 8, zeros past K.
+// With mats.swiglu_out the first NT / 2 tiles are gate rows and the others the same rows of the up matrix.
+template <int NT, int MT, int KS, bool ALIGNED>
+__global__ __launch_bounds__(KS * 64, sk_occ(NT, MT)) void gemm_q4_0_skinny(const gemm_mats mats, const _Float16 *__restrict__ Xh, int K,
+                                                            int kp_blocks, int M, int n_tiles, int m_blocks) {
+    constexpr int SG = sk_steps(MT), GROUPS = 8 / SG;  // an even number of groups a piece
+    __shared__ __attribute__((aligned(16))) float4_t part[KS][KS][64];
+    // blockIdx % 8 is the XCD: the row blocks of one weight tile follow one another on it, so the second reads its
+    // weights from that XCD's L2
+    const int idx = blockIdx.x >> 3;
+    const int nt0 = (idx / m_blocks) * 8 + (blockIdx.x & 7), mb = idx % m_blocks;
+    if (nt0 >= n_tiles) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, kg = lane >> 4;
+    const bool swiglu = mats.swiglu_out != nullptr;
+    const int nblocks = K / 32, npieces = kp_blocks / 8;
+    const size_t wrow_bytes = (size_t)nblocks * 18;
+
+    const uint8_t *row[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        if (NT > 1 && swiglu)
+            row[t] = mats.W[t >= NT / 2] + (size_t)min(nt0 * (NT / 2 * 16) + (t % (NT / 2 > 0 ? NT / 2 : 1)) * 16 + r, mats.N[0] - 1) * wrow_bytes;
+        else
+            row[t] = gemm_w_row(mats, nt0 * (NT * 16) + t * 16 + r, wrow_bytes);
+    }
+    // fragment (b, c) of row tile i, piece p: byte fo[i] + p * 8 KB + b * 1 KB + c * 256 of the panel
+    const int m16_last = (M + 15) / 16 - 1;
+    uint32_t fo[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) fo[i] = (uint32_t)min(mb * MT + i, m16_last) * (uint32_t)kp_blocks * 1024u + kg * 2048u + r * 16u;
+
+    float4_t acc[NT][MT];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[t][i] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    const unsigned char *xb = reinterpret_cast<const unsigned char *>(Xh);
+    half8_t f[2][SG][MT];
+    auto frags = [&](half8_t(&dst)[SG][MT], int piece, int g) {
+#pragma unroll
+        for (int j = 0; j < SG; j++)
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+                dst[j][i] = *reinterpret_cast<const half8_t *>(xb + (size_t)piece * 8192 + fo[i] + (g * SG + j) / 4 * 1024 + (g * SG + j) % 4 * 256);
+    };
+    sk_raw<ALIGNED> raw[NT];
+    int piece = wave;
+    if (piece < npieces) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) sk_load(raw[t], row[t], piece * 8 + kg * 2, nblocks);
+        frags(f[0], piece, 0);
+    }
+    for (; piece < npieces; piece += KS) {
+        const int next = min(piece + KS, npieces - 1);  // the last round requests a piece again, unused
+        sk_blocks blk[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) sk_unpack(blk[t], raw[t], row[t], piece * 8 + kg * 2, nblocks);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < NT; t++) sk_load(raw[t], row[t], next * 8 + kg * 2, nblocks);
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            frags(f[(g + 1) & 1], g + 1 < GROUPS ? piece : next, (g + 1) % GROUPS);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < SG; j++) {
+                const int step = g * SG + j, b = step / 4;
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const half8_t w = step % 4 == 0   ? sk_operand<0>(blk[t].q[b], blk[t].d[b])
+                                      : step % 4 == 1 ? sk_operand<1>(blk[t].q[b], blk[t].d[b])
+                                      : step % 4 == 2 ? sk_operand<2>(blk[t].q[b], blk[t].d[b])
+                                                      : sk_operand<3>(blk[t].q[b], blk[t].d[b]);
+#pragma unroll
+                    for (int i = 0; i < MT; i++) acc[t][i] = GEMM_MFMA(w, f[g & 1][j][i], acc[t][i]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    // The waves' sums, KS tiles at a time: every wave parks its own, then adds up one of them.  Tiles go in the order
+    // (i, t), for a SwiGLU with the gate and the up tile of an output next to each other.
+    constexpr int TILES = NT * MT;
+#pragma unroll
+    for (int c0 = 0; c0 < TILES; c0 += KS) {
+        if (c0) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KS; j++) {
+            constexpr int H = NT / 2 > 0 ? NT / 2 : 1;
+            if (c0 + j < TILES) {
+                const int i = (c0 + j) / NT, o = (c0 + j) % NT;
+                const int t_pair = (o & 1) * H + (o >> 1);  // gate 0, up 0, gate 1, up 1 ..
+                part[j][wave][lane] = NT > 1 && swiglu ? acc[t_pair][i] : acc[o][i];
+            }
+        }
+        __syncthreads();
+        const int j = wave;
+        const int tile = c0 + j;
+        const int i = tile / NT, o = tile % NT;
+        const int m = (mb * MT + i) * 16 + r;
+        if (tile >= TILES) continue;
+        float4_t v = part[j][0][lane];
+#pragma unroll
+        for (int w = 1; w < KS; w++) v += part[j][w][lane];
+        if (NT > 1 && swiglu) {
+            if (o & 1) continue;  // the up tile is read by the wave of its gate tile
+            float4_t u = part[j + 1 < KS ? j + 1 : j][0][lane];
+#pragma unroll
+            for (int w = 1; w < KS; w++) u += part[j + 1 < KS ? j + 1 : j][w][lane];
+            const int n = nt0 * (NT / 2 * 16) + (o >> 1) * 16 + 4 * kg;
+            const int N = mats.N[0];
+            if (m < ((M + 15) & ~15) && n < N) {  // rows past M are zeros in the input panel, hence here
+                float s[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[e] * -1.44269504088896340736f));
+                    s[e] = (v[e] * sig) * u[e];
+                }
+                unsigned char *out = reinterpret_cast<unsigned char *>(mats.swiglu_out) + (size_t)(m >> 4) * (size_t)(N >> 5) * 1024 +
+                                     (size_t)(n >> 5) * 1024 + (size_t)((n & 31) >> 3) * 256 + (size_t)(m & 15) * 16 + (size_t)(n & 7) * 2;
+                *reinterpret_cast<uint2 *>(out) = make_uint2(pack_h2(s[0], s[1]), pack_h2(s[2], s[3]));
+            }
+        } else if (m < M) {
+            sk_store4(mats, nt0 * (NT * 16) + o * 16 + 4 * kg, m, v);
+        }
+    }
+}
+
+template <int NT, int MT, int KS, bool ALIGNED>
+int32_t skinny_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M) {
+    const int cols_per_tile = mats.swiglu_out ? NT / 2 * 16 : NT * 16;
+    const int cols = mats.swiglu_out ? mats.N[0] : mats.n_total;
+    const int n_tiles = (cols + cols_per_tile - 1) / cols_per_tile, m_blocks = ((M + 15) / 16 + MT - 1) / MT;
+    const dim3 grid((unsigned)((n_tiles + 7) / 8 * 8 * m_blocks));
+    hipLaunchKernelGGL((gemm_q4_0_skinny<NT, MT, KS, ALIGNED>), grid, dim3(KS * 64), 0, ctx->stream, mats, Xh, K, kp_blocks, M,
+                       n_tiles, m_blocks);
+    return GALOIS_HIP_OK;
+}
+
+// Rows up to which the panel calls run here rather than on the 256-row kernel.  Measured (us, this kernel / that one, weights
+// from HBM): q | k | v of 4096 (12288 x 4096) 14.1 / 25.3 at 23 rows, 19.8 / 28.0 at 77, 27.3 / 30.6 at 128, 30.0 / 28.2 at
+// 150; gate | up + SwiGLU (2 x 11008 x 4096) 20.3 / 41.1, 31.6 / 43.9, 40.0 / 43.9, 55 / 43.4; 4096 x 11008 14.7 / 52.8,
+// 20.3 / 53.3, 24.1 / 54.4; 4096 x 4096 7.1 / 23.0, 10.2 / 23.2, 11.9 / 22.7.  A result's sum order depends on K and
+// on the side of this line M is on, never on N: matrices multiplied together and one by one give the same bits.
+constexpr int SK_MAX_ROWS = 128;
+
+// Time of a workgroup relative to others, us at K = 4096 (fitted to the sizes above within 10 %): what a weight tile costs
+// (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.
+inline double sk_cost(int nt, int mt) { return 1.55 * nt + mt * (0.78 + 0.25 * nt); }
+
+template <int KS, bool ALIGNED>
+int32_t skinny_launch_tiles(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, int nt, int mt) {
+#define SK_MT(NT_)                                                                                    \
+    switch (mt) {                                                                                     \
+        case 1: return skinny_launch<NT_, 1, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
+        case 2: return skinny_launch<NT_, 2, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
+        case 3: return skinny_launch<NT_, 3, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
+        case 4: return skinny_launch<NT_, 4, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
+        default: return skinny_launch<NT_, SK_MAX_MT, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);   \
+    }
+    if (nt == 1) SK_MT(1)
+    if (nt == 2) SK_MT(2)
+    SK_MT(4)
+#undef SK_MT
+}
+
+// Tiles per wave by that cost and the rounds of workgroups over the CUs; the rows may be split over several workgroups.
+// KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.
+int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned) {
+    const int64_t cols = mats.swiglu_out ? 2 * (int64_t)mats.N[0] : mats.n_total, cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
+    const int t = (M + 15) / 16;
+    int nt = 0, mt = 0;
+    double best = 0.0;
+    for (int m = 1; m <= SK_MAX_MT && m <= t; m++)
+        for (int n = mats.swiglu_out ? 2 : 1; n <= 4; n *= 2) {
+            const int64_t wgs = (cols + 16 * n - 1) / (16 * n) * ((t + m - 1) / m);
+            const double cost = (double)((wgs + cus - 1) / cus) * sk_cost(n, m);
+            if (nt == 0 || cost < best) best = cost, nt = n, mt = m;
+        }
+    if (K >= 8192)
+        return aligned ? skinny_launch_tiles<8, true>(ctx, mats, Xh, K, kp_blocks, M, nt, mt)
+                       : skinny_launch_tiles<8, false>(ctx, mats, Xh, K, kp_blocks, M, nt, mt);
+    return aligned ? skinny_launch_tiles<4, true>(ctx, mats, Xh, K, kp_blocks, M, nt, mt)
+                   : skinny_launch_tiles<4, false>(ctx, mats, Xh, K, kp_blocks, M, nt, mt);
+}
+
+}  // namespace
