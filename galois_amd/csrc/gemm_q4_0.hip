@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256) void gemm_q4_0_mfma_v1(const uint8_t *__restri
 //     order the A operand of v_mfma_f32_16x16x32_f16 is held (per lane 8 consecutive k of one row),
 //     so a fragment is one contiguous KB: the consumer waves fetch their A fragments straight from
 //     global memory (the 4 MB panel stays in L2) two stages ahead, and X never touches LDS.
-//   - Workgroup tile 256 (M) x 96 (N), k-stage 64 (two Q4_0 blocks = one 36-byte slot per weight
+//   - Workgroup tile 256 (M; 192 or 128 where that leaves fewer rows of padding: RT = 3, 2) x 96 (N), k-stage 64 (two Q4_0 blocks = one 36-byte slot per weight
 //     row).  The 512 x 11008 prefill is 2 x 115 = 230 workgroups: one round on 256 CUs.
 //   - 8 waves: 4 consumers stacked in M, wave tile 64 x 96 -> 4 x 6 MFMA tiles with f32 accumulators
 //     in registers, and 4 producers that fetch the weights as whole 144-byte row pieces (4 stages at
@@ -148,7 +148,6 @@ __global__ __launch_bounds__(256) void gemm_q4_0_mfma_v1(const uint8_t *__restri
 //     contiguous range of weight tiles: X stays in that XCD's L2, W streams once per panel.
 // The N extent of the tile is a template parameter: 96 columns (6 MFMA tiles per consumer wave) for wide
 // matrices, 48 (3 per wave) when 96 would leave most CUs without a workgroup (N = 4096 at M = 512: 86 tiles).
-constexpr int GM = 256;
 constexpr int GBSTRIDE = 80;                  // halfs per B row in LDS: 160-byte rows
 constexpr int GNBUF = 3;
 constexpr int GRAW_STRIDE = 144;              // raw bytes per tile row per super-stage (4 slots)
@@ -491,8 +490,9 @@ __device__ __forceinline__ void gemm_producer(_Float16 *smem, const gemm_mats &m
 // order, so "at most n younger loads outstanding" is the exact condition for an older one to have
 // landed; left to the compiler, a load whose use is a loop iteration away is waited for with
 // vmcnt(0), which would also drain the prefetches just issued.
+template <int RT>
 struct gemm_a_regs {
-    u32x4_t c[8];  // [ks * 4 + i]: rows i*16 + lane%16 of the wave's 64, k = ks*32 + (lane/16)*8 ..
+    u32x4_t c[2 * RT];  // [ks * RT + i]: rows i*16 + lane%16 of the wave's 16 * RT, k = ks*32 + (lane/16)*8 ..
 };
 
 // One fragment.  Address = scalar base xs (the panel advanced to the stage: 2 KB per stage) + per-lane
@@ -506,14 +506,16 @@ __device__ __forceinline__ void gemm_load_a1(u32x4_t &dst, const _Float16 *xs, u
 }
 
 // Drains the load counter; naming the registers keeps all of them allocated until here.
-#define GEMM_DRAIN_A(r)                                                                                      \
-    asm volatile("s_waitcnt vmcnt(0)"                                                                        \
-                 : "+v"((r).c[0]), "+v"((r).c[1]), "+v"((r).c[2]), "+v"((r).c[3]), "+v"((r).c[4]), "+v"((r).c[5]), \
-                   "+v"((r).c[6]), "+v"((r).c[7])::"memory")
+template <int RT>
+__device__ __forceinline__ void gemm_drain_a(gemm_a_regs<RT> &r) {
+    GEMM_VMWAIT(0);
+#pragma unroll
+    for (int g = 0; g < 2 * RT; g++) asm volatile("" : "+v"(r.c[g])::"memory");
+}
 
 #define GEMM_LDB(dst, ptr) dst = *reinterpret_cast<const half8_t *>(ptr)
 #define GEMM_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0)
-template <int NF, int GN>
+template <int NF, int GN, int RT>
 __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float16 *__restrict__ Xh,
                                               const gemm_mats &mats, int K, int M, int m0, int n0, int wm, int ncol0,
                                               int nslots, size_t y_off) {
@@ -521,33 +523,33 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
     // relative to Y (a workgroup that holds one share of k of several writes a partial result)
     constexpr int GB_HALFS = gemm_cfg<GN>::B_HALFS;
     const int lane = threadIdx.x & 63;
-    float4_t acc[4][NF];
+    float4_t acc[RT][NF];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < RT; i++)
 #pragma unroll
         for (int j = 0; j < NF; j++) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-    uint32_t ro[4];  // byte offsets in the tiled panel (the host checks that the panel is below 4 GB)
+    uint32_t ro[RT];  // byte offsets in the tiled panel (the host checks that the panel is below 4 GB)
     const int m16_last = (M + 15) / 16 - 1;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        ro[i] = (uint32_t)min(m0 / 16 + wm * 4 + i, m16_last) * (uint32_t)(K / 32) * 1024u + lane * 16u;
+    for (int i = 0; i < RT; i++)
+        ro[i] = (uint32_t)min(m0 / 16 + wm * RT + i, m16_last) * (uint32_t)(K / 32) * 1024u + lane * 16u;
     const int b_off = (ncol0 + (lane & 15)) * GBSTRIDE + (lane >> 4) * 8;
 
-    // Stages of A fragments in flight: two for the wide tile (its accumulators leave room for no more), four for the
-    // narrow one, whose stages are short enough to run into the latency of the requests (measured: 512 x 11008 x 4096
+    // Stages of A fragments in flight: two for the wide tiles of more than 128 rows (their accumulators leave room for no
+    // more), four for the narrow and the low ones, whose stages are short enough to run into the latency of the requests (measured: 512 x 11008 x 4096
     // 70.7 -> 69.4 us, 512 x 4096 x 4096 31.4 -> 31.2 us).
-    constexpr int DEPTH = (NF <= 3) ? 4 : 2;
-    gemm_a_regs a0, a1, a2, a3;
+    constexpr int DEPTH = (NF <= 3 || RT <= 2) ? 4 : 2;
+    gemm_a_regs<RT> a0, a1, a2, a3;
     // requested in the order they are used: the waits below count younger requests
 #pragma unroll
-    for (int g = 0; g < 8; g++) gemm_load_a1(a0.c[g], Xh, ro[g & 3], g >> 2);
+    for (int g = 0; g < 2 * RT; g++) gemm_load_a1(a0.c[g], Xh, ro[g % RT], g / RT);
 #pragma unroll
-    for (int g = 0; g < 8; g++) gemm_load_a1(a1.c[g], Xh + 1024, ro[g & 3], g >> 2);
+    for (int g = 0; g < 2 * RT; g++) gemm_load_a1(a1.c[g], Xh + 1024, ro[g % RT], g / RT);
     if (DEPTH == 4) {
 #pragma unroll
-        for (int g = 0; g < 8; g++) gemm_load_a1(a2.c[g], Xh + 2048, ro[g & 3], g >> 2);
+        for (int g = 0; g < 2 * RT; g++) gemm_load_a1(a2.c[g], Xh + 2048, ro[g % RT], g / RT);
 #pragma unroll
-        for (int g = 0; g < 8; g++) gemm_load_a1(a3.c[g], Xh + 3072, ro[g & 3], g >> 2);
+        for (int g = 0; g < 2 * RT; g++) gemm_load_a1(a3.c[g], Xh + 3072, ro[g % RT], g / RT);
     }
     half8_t b0[NF], b1[NF];
     __syncthreads();  // R
@@ -555,26 +557,26 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
 #pragma unroll
     for (int j = 0; j < NF; j++) GEMM_LDB(b0[j], smem + b_off + j * 16 * GBSTRIDE);
 
-    // One stage = eight groups of NF matrix instructions; group g multiplies A fragment g (rows
-    // (g % 4) * 16 .., k-half g / 4) of AC with the B fragments of that k-half, then requests the same
+    // One stage = 2 * RT groups of NF matrix instructions; group g multiplies A fragment g (rows
+    // (g % RT) * 16 .., k-half g / RT) of AC with the B fragments of that k-half, then requests the same
     // fragment of the stage DEPTH stages on into the registers it has just consumed.  The requests are spread
     // over the stage so that the four waves never queue more than the memory pipe takes without blocking
-    // the issue of the matrix instructions; a fragment is needed 8 * DEPTH groups after its request, with
-    // 8 * DEPTH - 1 younger requests outstanding.
-    // The B reads are spread the same way: the second k-half of this stage during groups 0..2, the
-    // first k-half of the next stage (after the barrier that publishes it) during groups 4..6.
+    // the issue of the matrix instructions; a fragment is needed 2 * RT * DEPTH groups after its request, with
+    // 2 * RT * DEPTH - 1 younger requests outstanding.
+    // The B reads are spread the same way: the second k-half of this stage during its first groups, the
+    // first k-half of the next stage (after the barrier that publishes it) during groups RT ..
     // cur / nxt are the LDS offsets of this stage's and the next stage's B buffers.
     int cur = b_off, nxt = b_off + GB_HALFS;
-    constexpr int BPG = (NF + 2) / 3;  // B fragment reads per group
+    constexpr int BCH = RT < 3 ? RT : 3;          // groups the reads of a k-half are spread over
+    constexpr int BPG = (NF + BCH - 1) / BCH;     // B fragment reads per group
 #define GEMM_GROUP(G, AC, BV)                                                                              \
     {                                                                                                      \
-        if (DEPTH == 4) asm volatile("s_waitcnt vmcnt(31)" : "+v"((AC).c[G])::"memory");                   \
-        else asm volatile("s_waitcnt vmcnt(15)" : "+v"((AC).c[G])::"memory");                              \
+        asm volatile("s_waitcnt vmcnt(%1)" : "+v"((AC).c[G]) : "n"(2 * RT * DEPTH - 1) : "memory");        \
         __builtin_amdgcn_sched_barrier(0);                                                                 \
-        _Pragma("unroll") for (int j = 0; j < NF; j++) acc[(G) & 3][j] =                                   \
-            GEMM_MFMA(__builtin_bit_cast(half8_t, (AC).c[G]), BV[j], acc[(G) & 3][j]);                     \
+        _Pragma("unroll") for (int j = 0; j < NF; j++) acc[(G) % RT][j] =                                  \
+            GEMM_MFMA(__builtin_bit_cast(half8_t, (AC).c[G]), BV[j], acc[(G) % RT][j]);                    \
         __builtin_amdgcn_sched_barrier(0);                                                                 \
-        gemm_load_a1((AC).c[G], xs_next, ro[(G) & 3], (G) >> 2);                                           \
+        gemm_load_a1((AC).c[G], xs_next, ro[(G) % RT], (G) / RT);                                          \
     }
 #define GEMM_BREADS(G3, DST, OFF)                                                                          \
     _Pragma("unroll") for (int j = (G3) * BPG; j < NF && j < ((G3) + 1) * BPG; j++)                        \
@@ -582,20 +584,15 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
 #define GEMM_STAGE(S, AC, LAST)                                                                            \
     {                                                                                                      \
         const _Float16 *xs_next = Xh + min((S) + DEPTH, nslots - 1) * 1024;                                \
-        GEMM_BREADS(0, b1, cur + 32) GEMM_GROUP(0, AC, b0)                                                 \
-        GEMM_BREADS(1, b1, cur + 32) GEMM_GROUP(1, AC, b0)                                                 \
-        GEMM_BREADS(2, b1, cur + 32) GEMM_GROUP(2, AC, b0)                                                 \
-        GEMM_GROUP(3, AC, b0)                                                                              \
-        if (!(LAST)) {                                                                                     \
-            __syncthreads(); /* stage S+1 written */                                                           \
-            GEMM_BREADS(0, b0, nxt)                                                                        \
+        _Pragma("unroll") for (int g = 0; g < RT; g++) {                                                   \
+            if (g < BCH) { GEMM_BREADS(g, b1, cur + 32) }                                                  \
+            GEMM_GROUP(g, AC, b0)                                                                          \
         }                                                                                                  \
-        GEMM_GROUP(4, AC, b1)                                                                              \
-        if (!(LAST)) { GEMM_BREADS(1, b0, nxt) }                                                           \
-        GEMM_GROUP(5, AC, b1)                                                                              \
-        if (!(LAST)) { GEMM_BREADS(2, b0, nxt) }                                                           \
-        GEMM_GROUP(6, AC, b1)                                                                              \
-        GEMM_GROUP(7, AC, b1)                                                                              \
+        if (!(LAST)) __syncthreads(); /* stage S+1 written */                                              \
+        _Pragma("unroll") for (int g = 0; g < RT; g++) {                                                   \
+            if (!(LAST) && g < BCH) { GEMM_BREADS(g, b0, nxt) }                                            \
+            GEMM_GROUP(RT + g, AC, b1)                                                                     \
+        }                                                                                                  \
         cur = nxt;                                                                                         \
         nxt = (nxt == b_off + (GNBUF - 1) * GB_HALFS) ? b_off : nxt + GB_HALFS;                            \
     }
@@ -623,11 +620,11 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
 #undef GEMM_GROUP
 #undef GEMM_BREADS
     // the last two stages requested the last stage's fragments again (never used): drain before the registers die
-    GEMM_DRAIN_A(a0);
-    GEMM_DRAIN_A(a1);
+    gemm_drain_a(a0);
+    gemm_drain_a(a1);
     if (DEPTH == 4) {
-        GEMM_DRAIN_A(a2);
-        GEMM_DRAIN_A(a3);
+        gemm_drain_a(a2);
+        gemm_drain_a(a3);
     }
 
     // C layout of the 16x16 MFMA: column = lane % 16, row = 4 * (lane / 16) + e.
@@ -646,10 +643,10 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
             const int n = (n0 / 96) * 48 + j * 16 + (lane & 15);
             const size_t col_at = (size_t)(n >> 5) * 1024 + (size_t)((n & 31) >> 3) * 256 + (size_t)(n & 7) * 2;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < RT; i++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const int m = m0 + wm * 64 + i * 16 + 4 * (lane >> 4) + e;
+                    const int m = m0 + wm * (16 * RT) + i * 16 + 4 * (lane >> 4) + e;
                     const float g = acc[i][j][e], u = acc[i][j + 3 < NF ? j + 3 : j][e];
                     const float sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896340736f));
                     const uint32_t h = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)((g * sig) * u));
@@ -677,16 +674,16 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
         const int nl = n - first;
         Y += y_off;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < RT; i++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int m = m0 + wm * 64 + i * 16 + 4 * (lane >> 4) + e;
+                const int m = m0 + wm * (16 * RT) + i * 16 + 4 * (lane >> 4) + e;
                 if (m < M && n < mats.n_total) Y[(size_t)m * N + nl] = acc[i][j][e];
             }
     }
 }
 
-template <int GN>
+template <int GN, int RT>
 __global__ __launch_bounds__(512) void gemm_q4_0_mfma(const gemm_mats mats, const _Float16 *__restrict__ Xh, int K, int M,
                                                       int n_tiles, int m_tiles, int splits, size_t split_stride) {
     extern __shared__ __attribute__((aligned(16))) _Float16 smem[];  // [3] B stage | [2] raw | pad
@@ -697,7 +694,7 @@ __global__ __launch_bounds__(512) void gemm_q4_0_mfma(const gemm_mats mats, cons
     if (tile >= total) return;
     const int mts = tile / n_tiles, nt = tile - mts * n_tiles;
     const int sp = mts / m_tiles, mt = mts - sp * m_tiles;
-    const int m0 = mt * GM, n0 = nt * GN;
+    const int m0 = mt * (64 * RT), n0 = nt * GN;
     // share sp of k: whole pieces of 256 (four stages), as evenly as they divide; its results lie split_stride
     // floats after the previous share's
     const int nsuper_all = K / 256;
@@ -705,8 +702,8 @@ __global__ __launch_bounds__(512) void gemm_q4_0_mfma(const gemm_mats mats, cons
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (wave >= 4)
         gemm_producer<GN>(smem, mats, K, n0, sup0, sup1 - sup0);
-    else  // four consumer waves stacked in M, each 64 rows x GN columns; a piece of 256 is 8 KB of a row group's panel
-        gemm_consumer<GN / 16, GN>(smem, Xh + (size_t)sup0 * 4096, mats, K, M, m0, n0, wave, 0, (sup1 - sup0) * 4,
+    else  // four consumer waves stacked in M, each 16 * RT rows x GN columns; a piece of 256 is 8 KB of a row group's panel
+        gemm_consumer<GN / 16, GN, RT>(smem, Xh + (size_t)sup0 * 4096, mats, K, M, m0, n0, wave, 0, (sup1 - sup0) * 4,
                                    (size_t)sp * split_stride);
 }
 
@@ -737,19 +734,19 @@ __global__ __launch_bounds__(256) void gemm_sum_tail(const float *p, const float
 }
 
 // Launch of one tile width.
-template <int GN>
+template <int GN, int RT>
 int32_t gemm_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int M, int splits = 1,
                     size_t split_stride = 0) {
     const int n_tiles = (mats.n_total + GN - 1) / GN;
-    const int m_tiles = (M + GM - 1) / GM;
+    const int m_tiles = (M + 64 * RT - 1) / (64 * RT);
     const int total = n_tiles * m_tiles * splits;
     const int grid = ((total + 7) / 8) * 8;
     const size_t lds = gemm_cfg<GN>::LDS_BYTES;
     // the attribute lives with the function on the current device: set per launch (a table lookup), which is right
     // for every device and every thread without any flag of our own
-    hipError_t e = hipFuncSetAttribute((const void *)gemm_q4_0_mfma<GN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute((const void *)gemm_q4_0_mfma<GN, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return gh_hip(ctx, e, "hipFuncSetAttribute(LDS size)");
-    hipLaunchKernelGGL(gemm_q4_0_mfma<GN>, dim3(grid), dim3(512), lds, ctx->stream, mats, Xh, K, M, n_tiles, m_tiles, splits,
+    hipLaunchKernelGGL((gemm_q4_0_mfma<GN, RT>), dim3(grid), dim3(512), lds, ctx->stream, mats, Xh, K, M, n_tiles, m_tiles, splits,
                        split_stride);
     return GALOIS_HIP_OK;
 }
@@ -760,9 +757,42 @@ int32_t gemm_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *
 
 namespace {
 
-// Tile width by how many workgroups it gives the device.  Cost model: rounds of workgroups over the CUs
-// times the relative cost of a k-stage (a 48-column stage has half the matrix instructions and half
-// the dequantisation of a 96-column one but the same barriers and A requests: ~0.65).
+// The tile by how many workgroups it gives the device: rounds of workgroups over the CUs times the relative cost of a
+// k-stage.  A narrower tile has fewer matrix instructions and less dequantisation a stage but the same barriers and
+// activation requests; a lower one fewer matrix instructions and requests but the same dequantisation and barriers.
+// Costs of a stage on a full device, 96 columns x 256 rows = 1 (0.64 us), measured at K = 4096: gate | up + SwiGLU at 150 rows
+// (230 workgroups) 42.9 / 38.0 us with 256 / 192 rows, at 128 rows 44.6 / 38.4 / 32.5 with 256 / 192 / 128; q | k | v at 150
+// rows in 48 columns 28.1 / 24.7, at 128 rows 28.9 / 25.1 / 22.2; at 300 rows in 96 columns 48.7 / 41.5.  The order of a
+// result's sum is the same in all of them.
+struct gemm_tile {
+    int gn, rt;
+    double cost;  // rounds x relative cost of a stage
+};
+gemm_tile gemm_pick(const galois_hip_ctx *ctx, int64_t cols, int64_t M, int gn, int splits = 1) {
+    const double stage96[3] = {0.70, 0.86, 1.0}, stage64[3] = {0.50, 0.60, 0.75}, stage48[3] = {0.44, 0.53, 0.65};
+    const double *stage = gn == 96 ? stage96 : gn == 64 ? stage64 : stage48;
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
+    gemm_tile best = {gn, 4, 0.0};
+    for (int rt = 4; rt >= 2; rt--) {
+        const int64_t wgs = (cols + gn - 1) / gn * ((M + 64 * rt - 1) / (64 * rt)) * splits;
+        const double cost = (double)((wgs + cus - 1) / cus) * stage[rt - 2];
+        if (rt == 4 || cost < best.cost) best = {gn, rt, cost};
+    }
+    return best;
+}
+
+int32_t gemm_launch_tile(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int M, const gemm_tile &t, int splits = 1,
+                         size_t split_stride = 0) {
+#define GEMM_RT(GN_)                                                                                   \
+    return t.rt == 4   ? gemm_launch<GN_, 4>(ctx, mats, Xh, K, M, splits, split_stride)                \
+           : t.rt == 3 ? gemm_launch<GN_, 3>(ctx, mats, Xh, K, M, splits, split_stride)                \
+                       : gemm_launch<GN_, 2>(ctx, mats, Xh, K, M, splits, split_stride)
+    if (t.gn == 96) GEMM_RT(96);
+    if (t.gn == 64) GEMM_RT(64);
+    GEMM_RT(48);
+#undef GEMM_RT
+}
+
 // Numbers the columns of the first n_mats matrices through (col0, n_total).
 void gemm_concat(gemm_mats &mats, int n_mats) {
     int64_t cols = 0;
@@ -776,12 +806,8 @@ void gemm_concat(gemm_mats &mats, int n_mats) {
 int32_t gemm_launch_any(galois_hip_ctx *ctx, gemm_mats mats, int n_mats, const _Float16 *Xh, int K, int M) {
     gemm_concat(mats, n_mats);
     if (M <= SK_MAX_ROWS) return skinny_launch_any(ctx, mats, Xh, K, K / 32, M, true);
-    const int64_t cols = mats.n_total;
-    const int64_t m_tiles = (M + GM - 1) / GM;
-    const int64_t wg96 = (cols + 95) / 96 * m_tiles, wg48 = (cols + 47) / 48 * m_tiles;
-    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
-    const double cost96 = (double)((wg96 + cus - 1) / cus), cost48 = 0.65 * (double)((wg48 + cus - 1) / cus);
-    return cost48 < cost96 ? gemm_launch<48>(ctx, mats, Xh, K, M) : gemm_launch<96>(ctx, mats, Xh, K, M);
+    const gemm_tile t96 = gemm_pick(ctx, mats.n_total, M, 96), t48 = gemm_pick(ctx, mats.n_total, M, 48);
+    return gemm_launch_tile(ctx, mats, Xh, K, M, t48.cost < t96.cost ? t48 : t96);
 }
 
 // What the main kernel asks of its operands: whole 4-stage pieces of every weight row, 16-byte requests, and a panel
@@ -803,30 +829,36 @@ int32_t launch_to_panel(galois_hip_ctx *ctx, const float *x, const float *up, _F
 
 namespace {
 
-// Whether one matrix against the panel is better multiplied as two shares of k, each a workgroup of 64 columns, than
-// as whole-k tiles: the cost model of gemm_launch_any (rounds of workgroups x cost of a stage x stages; a 64-column
-// stage on a full device at 0.75 of a 96-column one) plus the pass that adds the two partial results, which costs
-// about fourteen stages per 2^21 results.  Measured at M = 512 on 256 CUs: 11008 -> 4096 70.3 -> 54.8 us,
-// 4096 -> 4096 32.5 -> 30.2 us (both with the residual); the shapes the model leaves whole are slower when forced
-// into shares.  margin > 1 asks for a clearer win (where the adding pass replaces nothing the caller would launch anyway),
-// min_cost for a product large enough that the model's neglect of fixed costs does not matter.
-bool gemm_two_shares_pay(const galois_hip_ctx *ctx, int K, int N, int M, double margin = 1.0, double min_cost = 0.0) {
-    const int64_t m_tiles = (M + GM - 1) / GM, cus = ctx->n_cu > 0 ? ctx->n_cu : 256, stages = K / 64;
-    const int64_t wg96 = ((int64_t)N + 95) / 96 * m_tiles, wg48 = ((int64_t)N + 47) / 48 * m_tiles, wg64x2 = ((int64_t)N + 63) / 64 * m_tiles * 2;
+// How one matrix is multiplied by the panel when its result may come in parts: whole-k tiles, two shares of k (each a
+// workgroup of 64 columns; the caller's next pass adds the two partial results), or the skinny kernel beyond the
+// rows that run on it anyway (a narrow matrix of long rows gives the tiles of either other form too few workgroups:
+// 11008 -> 4096 at 150 rows 27.3 us against 57 us whole and 39 us in shares).  The cost model of gemm_pick (rounds of
+// workgroups x cost of a stage x stages) plus the pass that adds the two partial results, which costs about fourteen stages
+// per 2^21 results.  Measured at M = 512 on 256 CUs: 11008 -> 4096 70.3 -> 54.8 us, 4096 -> 4096 32.5 -> 30.2 us (both
+// with the residual); the shapes the model leaves whole are slower when forced into shares.  margin > 1 asks for a clearer
+// win (where the adding pass replaces nothing the caller would launch anyway), min_cost for a product large enough that the
+// model's neglect of fixed costs does not matter.
+enum gemm_form { GEMM_WHOLE, GEMM_TWO_SHARES, GEMM_SKINNY };
+gemm_form gemm_pick_form(const galois_hip_ctx *ctx, int K, int N, int M, double margin = 1.0, double min_cost = 0.0) {
+    if (M <= SK_MAX_ROWS) return GEMM_WHOLE;  // on the skinny kernel
+    const double stages = K / 64;
     const int64_t mn = (int64_t)M * N;
-    if (M <= SK_MAX_ROWS) return false;
-    const double c96 = (double)((wg96 + cus - 1) / cus) * stages, c48 = 0.65 * (double)((wg48 + cus - 1) / cus) * stages;
-    const double c64x2 = 0.75 * (double)((wg64x2 + cus - 1) / cus) * (stages / 2 + 2) + 14.0 * (double)mn / (double)(1 << 21);
-    return K >= 512 && mn % 4 == 0 && margin * c64x2 < c96 && margin * c64x2 < c48 && c96 >= min_cost && c48 >= min_cost;
+    const double c96 = gemm_pick(ctx, N, M, 96).cost * stages, c48 = gemm_pick(ctx, N, M, 48).cost * stages;
+    const double whole = c96 < c48 ? c96 : c48;
+    const double c64x2 = gemm_pick(ctx, N, M, 64, 2).cost * (K / 128 + 2) + 14.0 * (double)mn / (double)(1 << 21);
+    const bool shares = K >= 512 && mn % 4 == 0 && margin * c64x2 < whole && whole >= min_cost;
+    if (margin == 1.0 && skinny_us(ctx, N, K, M) < 0.64 * (shares ? c64x2 : whole)) return GEMM_SKINNY;
+    return shares ? GEMM_TWO_SHARES : GEMM_WHOLE;
 }
 
-// W . panel into dst as one result (shares = 1) or as two partial results M * N floats apart (shares = 2).
-int32_t gemm_launch_shares(galois_hip_ctx *ctx, const void *W, const _Float16 *panel, float *dst, int K, int N, int M, int shares) {
+// W . panel into dst as one result or as two partial results M * N floats apart.
+int32_t gemm_launch_form(galois_hip_ctx *ctx, const void *W, const _Float16 *panel, float *dst, int K, int N, int M, gemm_form form) {
     gemm_mats mats = {};
     mats.W[0] = (const uint8_t *)W, mats.Y[0] = dst, mats.N[0] = N;
-    if (shares == 1) return gemm_launch_any(ctx, mats, 1, panel, K, M);
+    if (form == GEMM_WHOLE) return gemm_launch_any(ctx, mats, 1, panel, K, M);
     gemm_concat(mats, 1);
-    return gemm_launch<64>(ctx, mats, panel, K, M, 2, (size_t)M * N);
+    if (form == GEMM_SKINNY) return skinny_launch_any(ctx, mats, panel, K, K / 32, M, true);
+    return gemm_launch_tile(ctx, mats, panel, K, M, gemm_pick(ctx, N, M, 64, 2), 2, (size_t)M * N);
 }
 
 }  // namespace
@@ -847,7 +879,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
     const size_t panel_bytes = ((size_t)m_pad * k_pad * sizeof(_Float16) + 255) & ~(size_t)255;
     const bool wide = K == k_pad && gh_aligned(W, 16);  // what the 256-row kernel asks of the weights
     const bool skinny = !wide || M <= SK_MAX_ROWS;
-    const bool shares = !skinny && mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_two_shares_pay(ctx, K, N, M, 1.1, 64.0);
+    const bool shares = !skinny && mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_pick_form(ctx, K, N, M, 1.1, 64.0) == GEMM_TWO_SHARES;
     const size_t need = panel_bytes + (shares ? 2 * (size_t)mn * sizeof(float) : 0);
     bool panel = gemm_panel_shape_ok((int32_t)k_pad, M);
     if (panel && ctx->ws_bytes < need) {
@@ -885,13 +917,13 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
             if (st != GALOIS_HIP_OK) return st;
         } else if (shares) {
             float *parts = reinterpret_cast<float *>(static_cast<unsigned char *>(ctx->ws) + panel_bytes);
-            const int32_t st = gemm_launch_shares(ctx, W, Xh, parts, K, N, M, 2);
+            const int32_t st = gemm_launch_form(ctx, W, Xh, parts, K, N, M, GEMM_TWO_SHARES);
             if (st != GALOIS_HIP_OK) return st;
             hipLaunchKernelGGL(gemm_sum_pass, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, ctx->stream,
                                reinterpret_cast<const float4 *>(parts), static_cast<const float4 *>(nullptr),
                                reinterpret_cast<float4 *>(Y), mn / 4, mn / 4);
         } else {
-            const int32_t st = gemm_launch_shares(ctx, W, Xh, Y, K, N, M, 1);
+            const int32_t st = gemm_launch_form(ctx, W, Xh, Y, K, N, M, GEMM_WHOLE);
             if (st != GALOIS_HIP_OK) return st;
         }
     } else {
@@ -976,7 +1008,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f16_panel(galois_hip_ctx *ctx, const 
         mats.W[j] = (const uint8_t *)items[j].W, mats.Y[j] = items[j].Y, mats.N[j] = items[j].N;
         cols += items[j].N;
     }
-    GH_REQUIRE(ctx, cols < 0x7FFFFF00 && (cols + 47) / 48 * ((M + GM - 1) / GM) < 0x7FFFFF00, GALOIS_HIP_E_SHAPE,
+    GH_REQUIRE(ctx, cols < 0x7FFFFF00 && (cols + 47) / 48 * ((M + 127) / 128) < 0x7FFFFF00, GALOIS_HIP_E_SHAPE,
                "mul_mat_q4_0_f16_panel: too many columns");
     GH_BIND(ctx);
     const int32_t st = gemm_launch_any(ctx, mats, n_items, (const _Float16 *)panel, K, M);
@@ -999,8 +1031,10 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f16_panel_add(galois_hip_ctx *ctx, co
     GH_BIND(ctx);
     const int64_t mn = (int64_t)M * N;
     const dim3 sum_grid((unsigned)((mn / 4 + 255) / 256));
-    if (gemm_two_shares_pay(ctx, K, N, M) && workspace && workspace_bytes >= 2 * mn * (int64_t)sizeof(float)) {
-        const int32_t st = gemm_launch_shares(ctx, W, (const _Float16 *)panel, static_cast<float *>(workspace), K, N, M, 2);
+    // with room for two results the product may take any form; without it, it is the plain call's product bit for bit
+    const gemm_form form = workspace && workspace_bytes >= 2 * mn * (int64_t)sizeof(float) ? gemm_pick_form(ctx, K, N, M) : GEMM_WHOLE;
+    if (form == GEMM_TWO_SHARES) {
+        const int32_t st = gemm_launch_form(ctx, W, (const _Float16 *)panel, static_cast<float *>(workspace), K, N, M, form);
         if (st != GALOIS_HIP_OK) return st;
         hipLaunchKernelGGL(gemm_sum_pass, sum_grid, dim3(256), 0, ctx->stream, static_cast<const float4 *>(workspace),
                            reinterpret_cast<const float4 *>(residual), reinterpret_cast<float4 *>(Y), mn / 4, mn / 4);
@@ -1012,7 +1046,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f16_panel_add(galois_hip_ctx *ctx, co
                        "mul_mat_q4_0_f16_panel_add: Y may be the residual only with a workspace of M * N floats or more");
             prod = static_cast<float *>(workspace);
         }
-        const int32_t st = gemm_launch_shares(ctx, W, (const _Float16 *)panel, prod, K, N, M, 1);
+        const int32_t st = gemm_launch_form(ctx, W, (const _Float16 *)panel, prod, K, N, M, form);
         if (st != GALOIS_HIP_OK) return st;
         if (residual) {
             if (mn % 4 == 0)
@@ -1040,10 +1074,10 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f16_panel_shares(galois_hip_ctx *ctx,
     GH_REQUIRE(ctx, shares_bytes >= mn * (int64_t)sizeof(float), GALOIS_HIP_E_SHAPE,
                "mul_mat_q4_0_f16_panel_shares: room for at least one result of M * N floats");
     GH_BIND(ctx);
-    const int n = gemm_two_shares_pay(ctx, K, N, M) && shares_bytes >= 2 * mn * (int64_t)sizeof(float) ? 2 : 1;
-    const int32_t st = gemm_launch_shares(ctx, W, (const _Float16 *)panel, shares, K, N, M, n);
+    const gemm_form form = shares_bytes >= 2 * mn * (int64_t)sizeof(float) ? gemm_pick_form(ctx, K, N, M) : GEMM_WHOLE;
+    const int32_t st = gemm_launch_form(ctx, W, (const _Float16 *)panel, shares, K, N, M, form);
     if (st != GALOIS_HIP_OK) return st;
-    *n_shares = n;
+    *n_shares = form == GEMM_TWO_SHARES ? 2 : 1;
     GH_LAUNCH_CHECK(ctx, "mul_mat_q4_0_f16_panel_shares launch");
 }
 
@@ -1087,8 +1121,8 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_swiglu_f16_panel(galois_hip_ctx *ctx,
     for (int j = 0; j < GEMM_MAX_MATS; j++) mats.col0[j] = 0x7FFFFFFF;
     mats.n_total = 96 * ((N + 47) / 48);
     mats.swiglu_out = static_cast<_Float16 *>(panel_out);
-    const int32_t st = M <= SK_MAX_ROWS ? skinny_launch_any(ctx, mats, (const _Float16 *)panel, K, K / 32, M, true)
-                                        : gemm_launch<96>(ctx, mats, (const _Float16 *)panel, K, M);
+    const int32_t st = M <= SK_MAX_SWIGLU_ROWS ? skinny_launch_any(ctx, mats, (const _Float16 *)panel, K, K / 32, M, true)
+                                               : gemm_launch_tile(ctx, mats, (const _Float16 *)panel, K, M, gemm_pick(ctx, mats.n_total, M, 96));
     if (st != GALOIS_HIP_OK) return st;
     GH_LAUNCH_CHECK(ctx, "mul_mat_q4_0_swiglu_f16_panel launch");
 }

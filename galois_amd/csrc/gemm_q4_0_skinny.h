@@ -284,6 +284,8 @@ int32_t skinny_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16
 // 20.3 / 53.3, 24.1 / 54.4; 4096 x 4096 7.1 / 23.0, 10.2 / 23.2, 11.9 / 22.7.  A result's sum order depends on K and
 // on the side of this line M is on, never on N: matrices multiplied together and one by one give the same bits.
 constexpr int SK_MAX_ROWS = 128;
+// gate | up: always wide, so the 128-row tile catches up sooner (31.6 / 31.7 us at 77 rows, 40.4 / 31.8 at 100).
+constexpr int SK_MAX_SWIGLU_ROWS = 80;
 
 // Time of a workgroup relative to others, us at K = 4096 (fitted to the sizes above within 10 %): what a weight tile costs
 // (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.
@@ -306,23 +308,33 @@ int32_t skinny_launch_tiles(galois_hip_ctx *ctx, const gemm_mats &mats, const _F
 }
 
 // Tiles per wave by that cost and the rounds of workgroups over the CUs; the rows may be split over several workgroups.
-// KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.
-int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned) {
-    const int64_t cols = mats.swiglu_out ? 2 * (int64_t)mats.N[0] : mats.n_total, cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
+struct sk_tiles {
+    int nt, mt;
+    double cost;
+};
+inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int M, bool swiglu) {
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
     const int t = (M + 15) / 16;
-    int nt = 0, mt = 0;
-    double best = 0.0;
+    sk_tiles best = {0, 0, 0.0};
     for (int m = 1; m <= SK_MAX_MT && m <= t; m++)
-        for (int n = mats.swiglu_out ? 2 : 1; n <= 4; n *= 2) {
+        for (int n = swiglu ? 2 : 1; n <= 4; n *= 2) {
             const int64_t wgs = (cols + 16 * n - 1) / (16 * n) * ((t + m - 1) / m);
             const double cost = (double)((wgs + cus - 1) / cus) * sk_cost(n, m);
-            if (nt == 0 || cost < best) best = cost, nt = n, mt = m;
+            if (best.nt == 0 || cost < best.cost) best = {n, m, cost};
         }
+    return best;
+}
+inline double skinny_us(const galois_hip_ctx *ctx, int N, int K, int M) { return skinny_pick(ctx, N, M, false).cost * K / 4096.0; }
+
+// KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.
+int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned) {
+    const bool swiglu = mats.swiglu_out != nullptr;
+    const sk_tiles t = skinny_pick(ctx, swiglu ? 2 * (int64_t)mats.N[0] : mats.n_total, M, swiglu);
     if (K >= 8192)
-        return aligned ? skinny_launch_tiles<8, true>(ctx, mats, Xh, K, kp_blocks, M, nt, mt)
-                       : skinny_launch_tiles<8, false>(ctx, mats, Xh, K, kp_blocks, M, nt, mt);
-    return aligned ? skinny_launch_tiles<4, true>(ctx, mats, Xh, K, kp_blocks, M, nt, mt)
-                   : skinny_launch_tiles<4, false>(ctx, mats, Xh, K, kp_blocks, M, nt, mt);
+        return aligned ? skinny_launch_tiles<8, true>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
+                       : skinny_launch_tiles<8, false>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt);
+    return aligned ? skinny_launch_tiles<4, true>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
+                   : skinny_launch_tiles<4, false>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt);
 }
 
 }  // namespace

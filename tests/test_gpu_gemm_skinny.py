@@ -128,3 +128,52 @@ def test_swiglu_and_several_matrices(dev, m, k, n):
     assert emax < TOL and el2 < TOL, (emax, el2)
     for b in [xb, gb, ub, pb, po] + ys + parts:
         dev.free(b)
+
+
+@pytest.mark.parametrize("m,n", [(129, 5000), (150, 12288), (192, 700), (193, 11008), (300, 12288), (385, 9000), (640, 2000)])
+def test_row_tiles_of_the_wide_kernel(dev, m, n):
+    """129 rows and up: tiles of 128, 192 or 256 rows and 96 or 48 columns by the workgroups they give.  Against the oracle on a
+    sample, and the first 140 rows bit for bit as a batch of their own (another tile, the same order of sums)."""
+    k = 512
+    wq, x = _case(m + n, m, k, n)
+    got = _run(dev, wq, x)
+    cols = np.unique(np.concatenate([[0, n - 1], np.random.default_rng(n).choice(n, 96, replace=False)]))
+    emax, el2 = npref.rel_err(got[:, cols], oracle.mul_mat_q4_0_f32(wq[cols], x))
+    assert emax < TOL and el2 < TOL, (emax, el2)
+    if m > 140:
+        assert np.array_equal(got[:140].view(np.uint32), _run(dev, wq, x[:140]).view(np.uint32))
+
+
+@pytest.mark.parametrize("m,k,n", [(150, 4096, 768), (190, 1024, 512), (300, 4096, 4096), (390, 2048, 1024)])
+def test_forms_of_a_narrow_product(dev, m, k, n):
+    """With a workspace a narrow product comes whole, in two shares of k or from the few-rows kernel: each sums the same f32
+    products in its own order (1e-5 of the largest result)."""
+    wq, x = _case(m * 3 + n, m, k, n)
+    wb, xb = dev.upload(wq), dev.upload(x)
+    pb, ws, y = dev.alloc(dev.f16_panel_bytes(k, m)), dev.alloc(2 * m * n * 4), dev.alloc(m * n * 4)
+    dev.f32_to_f16_panel(xb, pb, k, m)
+    dev.mul_mat_q4_0_f16_panel([(wb, y, n)], pb, k, m)
+    plain = dev.download(y, np.float32, (m, n))
+    shares = dev.mul_mat_q4_0_f16_panel_shares(wb, pb, ws, 2 * m * n * 4, k, n, m)
+    got = dev.download(ws, np.float32, (2, m, n))[:shares].sum(axis=0)
+    assert np.max(np.abs(got - plain)) <= 1e-5 * np.max(np.abs(plain)), shares
+    dev.mul_mat_q4_0_f16_panel_add(wb, pb, None, y, k, n, m, ws, 2 * m * n * 4)
+    assert np.array_equal(dev.download(y, np.float32, (m, n)), got)
+    for b in (wb, xb, pb, ws, y):
+        dev.free(b)
+
+
+@pytest.mark.parametrize("m", [81, 128, 129, 192, 193, 260])
+def test_swiglu_row_tiles(dev, m):
+    k, n = 1024, 2816
+    (wg, x), (wu, _) = _case(m, m, k, n), _case(m + 1, m, k, n)
+    xb, gb, ub = dev.upload(x), dev.upload(wg), dev.upload(wu)
+    pb, po = dev.alloc(dev.f16_panel_bytes(k, m)), dev.alloc(dev.f16_panel_bytes(n, m))
+    dev.f32_to_f16_panel(xb, pb, k, m)
+    dev.mul_mat_q4_0_swiglu_f16_panel(gb, ub, pb, po, k, n, m)
+    t = dev.download(po, np.float16, ((m + 15) // 16, n // 32, 4, 16, 8)).transpose(0, 3, 1, 2, 4).reshape(-1, n)
+    want = oracle.mul(oracle.silu(oracle.mul_mat_q4_0_f32(wg, x)).reshape(-1), oracle.mul_mat_q4_0_f32(wu, x).reshape(-1)).reshape(m, n)
+    emax, el2 = npref.rel_err(t[:m].astype(np.float32), want)
+    assert emax < 2 * TOL and el2 < 2 * TOL and np.all(t[m:] == 0), (emax, el2)
+    for b in (xb, gb, ub, pb, po):
+        dev.free(b)
