@@ -913,7 +913,7 @@ int32_t launch_group(galois_hip_ctx *ctx, const galois_hip_gemv_item *items, int
 }
 
 // ---------------------------------------------------------------------------------------
-// The q | k | v products and the decode attention in one launch.
+// The q | k | v products and the decode attention in one launch (launch_qkv_attn: where that pays).
 //
 // Issued as two launches the attention starts when the last product row is out, pays a launch gap, and then spends
 // its first microseconds requesting the cache; its own end is a chain of dependent round trips (split records,
@@ -997,6 +997,23 @@ int32_t launch_qkv_attn(galois_hip_ctx *ctx, const galois_hip_gemv_item *items, 
                GALOIS_HIP_E_UNSUPPORTED, "qkv_attn_decode: n_head * ceil((n_past + 1) / 128) * (head_dim + 4) floats of partial "
                                          "results must fit the context's 4 MB scratch block");
     GH_REQUIRE(ctx, plan.blocks + (int64_t)n_head * S < 0x7FFFFFFF, GALOIS_HIP_E_SHAPE, "qkv_attn_decode: too many workgroups");
+    // One launch pays when there is much of both to overlap: three or more product workgroups per CU (the attention's
+    // registers leave room for two at a time instead of four, so few products gain nothing from being ahead) and a cache
+    // that takes longer to fetch than what the fused kernel adds.  Per layer of a decode step, us as two launches / one:
+    // 4096 wide, f32 cache, 200 keys 45.0 / 48.7, 800 47.8 / 57.6, 1600 (52 MB) 52.3 / 51.8, 2047 55.2 / 52.6, 4000 70.2 /
+    // 63.6; f16 cache 200 45.0 / 53.2, 1200 48.0 / 51.2, 2500 (41 MB) 52.9 / 52.4, 4000 62.0 / 58.7; 3072 wide, f32, 1200
+    // (29 MB) 40.9 / 43.7, 1600 (39 MB) 43.5 / 42.6; 2048 and 1024 wide two launches at every length (4000 keys 43.5 / 53.4 and
+    // 34.7 / 47.0).  A wait that is biased from outside (a test of the waits) keeps the launch that has them.
+    const int64_t cache_bytes = 2 * (int64_t)L * n_head * head_dim * (int64_t)sizeof(CT), cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
+    if ((cache_bytes < ((int64_t)38 << 20) || 4 * plan.blocks < 9 * cus) && n_head <= 65535 && ctx->wait_target_bias == 0) {
+        const int32_t sg = launch_group(ctx, items, 3, what);
+        if (sg != GALOIS_HIP_OK) return sg;
+        if (sizeof(CT) == 2)
+            return galois_hip_attn_decode_f16kv(ctx, items[0].dst, items[1].dst, items[2].dst, k_cache, v_cache, out, n_head, head_dim,
+                                                n_past, pos, freq_scale, theta_scale, scale, head_major_n_ctx);
+        return galois_hip_attn_decode_f32(ctx, items[0].dst, items[1].dst, items[2].dst, (float *)k_cache, (float *)v_cache, out, n_head,
+                                          head_dim, n_past, pos, freq_scale, theta_scale, scale, head_major_n_ctx);
+    }
     fa_args<CT> b;
     b.kc = k_cache, b.vc = v_cache, b.part = (float *)ctx->scratch, b.out = out;
     b.done = ctx->attn_done, b.ready = ctx->attn_done + GH_ATTN_HEADS, b.pos = pos;
