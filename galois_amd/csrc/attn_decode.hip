@@ -5,7 +5,7 @@
 // 698-782, 1597-1663).  Issued one by one these are nine launches that read the 64 MB of one layer's cache at
 // a third of the HBM rate, most of the time being launch gaps.  Here the same arithmetic runs in one launch:
 //
-//   attn_decode_partial: a workgroup owns 128 consecutive keys of one head.  It rotates its head's q (every
+//   attn_decode_partial: a workgroup owns 128 (64, 256) consecutive keys of one head.  It rotates its head's q (every
 //     workgroup of the head does, it is 128 floats), and the workgroup that owns position n_past also rotates
 //     the new k and writes k and v into row n_past of the caches.  Scores = scale * (k . q) go to LDS; the
 //     workgroup takes their maximum m, p = exp(score - m), the sum of p and the partial output sum p * v, and
@@ -20,9 +20,7 @@
 
 namespace {
 
-constexpr int AT_THREADS = 256;
-
-template <int LPR, typename CT>
+template <int LPR, typename CT, int KEYS, int AT_THREADS>
 __global__ __launch_bounds__(AT_THREADS) void attn_decode_partial(const float *__restrict__ q, const float *__restrict__ k,
                                                                   const float *__restrict__ v, CT *__restrict__ kc,
                                                                   CT *__restrict__ vc, float *__restrict__ part,
@@ -30,7 +28,7 @@ __global__ __launch_bounds__(AT_THREADS) void attn_decode_partial(const float *_
                                                                   const int32_t *__restrict__ pos, float freq_scale,
                                                                   float theta_scale, float scale, int64_t key_stride,
                                                                   int64_t head_stride) {
-    attn_decode_wg<LPR, CT, AT_THREADS, false>(q, k, v, kc, vc, part, done, out, H, L, pos, freq_scale, theta_scale, scale,
+    attn_decode_wg<LPR, CT, AT_THREADS, false, KEYS>(q, k, v, kc, vc, part, done, out, H, L, pos, freq_scale, theta_scale, scale,
                                                (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x, nullptr, 0u, key_stride,
                                                head_stride);
 }
@@ -82,13 +80,28 @@ int32_t attn_decode_launch(galois_hip_ctx *ctx, const float *q, const float *k, 
         done = ctx->attn_done;
     }
     GH_BIND(ctx);
-    const dim3 grid((unsigned)S, (unsigned)n_head), block(AT_THREADS);
-    if (head_dim == 128)
-        hipLaunchKernelGGL((attn_decode_partial<32, CT>), grid, block, 0, ctx->stream, q, k, v, k_cache, v_cache, part, done,
-                           out, n_head, L, pos, freq_scale, theta_scale, scale, key_stride, head_stride);
-    else
-        hipLaunchKernelGGL((attn_decode_partial<16, CT>), grid, block, 0, ctx->stream, q, k, v, k_cache, v_cache, part, done,
-                           out, n_head, L, pos, freq_scale, theta_scale, scale, key_stride, head_stride);
+    // Keys and threads of a workgroup.  The launch is a chain of dependent steps (requests, scores, softmax, merge), so
+    // while there are few workgroups more waves each do less: eight waves of 16 keys, or of 8 keys where even splits of 64
+    // keys leave CUs free.  A merge costs 2 us, so a head of 64 up to 256 keys long stays whole (its rows are half as
+    // long), and so do longer pieces of it once more than sixteen splits would have to be merged.  Beyond two workgroups
+    // per CU four waves a workgroup are better: more of them are resident.  Measured, us, 128 keys x 256 threads against the
+    // choice here: 32 heads of 128, 90 keys 6.8 -> 6.1, 203 9.0 -> 7.5, 512 10.1 -> 8.8, 1024 13.8 -> 12.1, 2048 19.7 ->
+    // 18.3 (f16 7.2 -> 6.2, 9.4 -> 7.6, 9.4 -> 8.4, 10.9 -> 10.2, 15.2 -> 14.4); 4000 keys with eight waves 42.9 against 33.7;
+    // 16 heads of 64, 203 keys 7.2 -> 6.1, 4000 15.8 -> 12.8.
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, s64 = (L + 63) / 64;
+#define AT_LAUNCH(LPR_, KEYS_, THREADS_)                                                                                          \
+    hipLaunchKernelGGL((attn_decode_partial<LPR_, CT, KEYS_, THREADS_>), dim3((unsigned)((L + KEYS_ - 1) / KEYS_), (unsigned)n_head), \
+                       dim3(THREADS_), 0, ctx->stream, q, k, v, k_cache, v_cache, part, done, out, n_head, L, pos, freq_scale,   \
+                       theta_scale, scale, key_stride, head_stride)
+    if (head_dim == 128) {
+        if (L > 128 && s64 <= 16 && n_head * s64 <= cus) AT_LAUNCH(32, 64, 512);
+        else if ((int64_t)n_head * S <= 2 * cus) AT_LAUNCH(32, 128, 512);
+        else AT_LAUNCH(32, 128, 256);
+    } else {
+        if ((L > 128 && L <= 256) || S > 16) AT_LAUNCH(16, 256, 512);
+        else AT_LAUNCH(16, 128, 256);
+    }
+#undef AT_LAUNCH
     GH_LAUNCH_CHECK(ctx, what);
 }
 

@@ -5,7 +5,8 @@
 
 namespace {
 
-constexpr int AT_KEYS = 128;  // keys per workgroup (measured: 64 and, for an f16 cache, 256 are slower)
+constexpr int AT_KEYS = 128;  // keys per workgroup of the launch that also carries the products (measured: 64 and, for an
+                              // f16 cache, 256 are slower); what the scratch limits of both launches count in
 
 template <int CTRL>
 __device__ __forceinline__ float at_dpp(float v) {
@@ -63,6 +64,31 @@ __device__ __forceinline__ float at_load(const float *p) {
     return __hip_atomic_load(const_cast<float *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Merge of up to N splits (up to 4096 keys at N = 32): every thread fetches all maxima, sums and its own element of every
+// partial output in one go -- one trip to memory instead of three dependent ones, and no barrier.  Same order of
+// additions as the general path of at_combine.
+template <int N>
+__device__ __forceinline__ void at_combine_few(const float *rec, float *__restrict__ out_h, int d, int D, int S) {
+    float ms[N], ss[N], os[N];
+#pragma unroll
+    for (int s = 0; s < N; s++) {
+        const float *r = rec + (size_t)min(s, S - 1) * (D + 4);
+        ms[s] = at_load(r), ss[s] = at_load(r + 1), os[s] = at_load(r + 4 + min(d, D - 1));
+    }
+    float M = ms[0];
+#pragma unroll
+    for (int s = 1; s < N; s++) M = fmaxf(M, s < S ? ms[s] : M);
+    float den = 0.0f, num = 0.0f;
+#pragma unroll
+    for (int s = 0; s < N; s++)
+        if (s < S) {
+            const float ws = expf(ms[s] - M);
+            den = __builtin_fmaf(ws, ss[s], den);
+            num = __builtin_fmaf(ws, os[s], num);
+        }
+    if (d < D) out_h[d] = num / den;
+}
+
 // Merge of a head's splits, run by the workgroup that finishes the head's last split: thread d < D owns output
 // element d.  The split maxima and sums are fetched by S threads at once and the weights exp(m_s - M) shared
 // through LDS; the partial outputs are then read eight splits at a time.
@@ -73,27 +99,11 @@ __device__ __forceinline__ void at_combine(const float *rec, float *__restrict__
     constexpr int WAVES = AT_THREADS / 64;
     const int d = threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (S <= 16) {
-        // Few splits (up to 2048 keys): every thread fetches all maxima, sums and its own element of every partial
-        // output in one go -- one trip to memory instead of three dependent ones, and no barrier.  Same order of
-        // additions as the general path below.
-        float ms[16], ss[16], os[16];
-#pragma unroll
-        for (int s = 0; s < 16; s++) {
-            const float *r = rec + (size_t)min(s, S - 1) * (D + 4);
-            ms[s] = at_load(r), ss[s] = at_load(r + 1), os[s] = at_load(r + 4 + min(d, D - 1));
-        }
-        float M = ms[0];
-#pragma unroll
-        for (int s = 1; s < 16; s++) M = fmaxf(M, s < S ? ms[s] : M);
-        float den = 0.0f, num = 0.0f;
-#pragma unroll
-        for (int s = 0; s < 16; s++)
-            if (s < S) {
-                const float ws = expf(ms[s] - M);
-                den = __builtin_fmaf(ws, ss[s], den);
-                num = __builtin_fmaf(ws, os[s], num);
-            }
-        if (d < D) out_h[d] = num / den;
+        at_combine_few<16>(rec, out_h, d, D, S);
+        return;
+    }
+    if (S <= 32) {
+        at_combine_few<32>(rec, out_h, d, D, S);
         return;
     }
     float mx = -__builtin_inff();
@@ -186,7 +196,7 @@ __device__ __forceinline__ float4 at_load4_coherent(const float *p) {
 // merges a head returns the three counters to zero.  A wait that runs out (spin_limit polls) is agreed on by the whole
 // workgroup: the head's record -- and with it the head's output, whichever workgroup merges it -- becomes NaN in
 // every element, and *status (pinned host memory the context reads after its next wait for the stream) is set.
-template <int LPR, typename CT, int AT_THREADS, bool FUSED>
+template <int LPR, typename CT, int AT_THREADS, bool FUSED, int KEYS = AT_KEYS>
 __device__ __forceinline__ void attn_decode_wg(const float *__restrict__ q, const float *__restrict__ k,
                                                const float *__restrict__ v, CT *__restrict__ kc, CT *__restrict__ vc,
                                                float *__restrict__ part, unsigned *__restrict__ done,
@@ -195,7 +205,6 @@ __device__ __forceinline__ void attn_decode_wg(const float *__restrict__ q, cons
                                                unsigned *ready, unsigned target, int64_t key_stride, int64_t head_stride,
                                                int spin_limit = 0, unsigned *status = nullptr) {
     constexpr int D = LPR * 4, RPL = 64 / LPR, WAVES = AT_THREADS / 64;
-    constexpr int KEYS = AT_KEYS;
     constexpr int KPW = KEYS / WAVES;     // keys per wave
     constexpr int U = KPW / RPL;          // wave-loads per wave, all in flight
     constexpr bool F16 = sizeof(CT) == 2;
