@@ -6,96 +6,153 @@
 //   dst[i2][m][n] = sum_k a[(i2 / r2) * a_s2 + n * a_s1 + k * a_s0] * b[(i2 * M + m) * K + k]
 //
 // v_mfma_f32_32x32x2_f32 multiplies and accumulates in f32, so nothing is rounded that the scalar kernels do not
-// round (an f16 a is widened exactly).  Workgroup tile 128 x 128, k step 16, four waves of 64 x 64; one grid layer
-// per batch slice.  a may be contiguous along K (a K^T-style view of a cache) or along N (a V-style view): the
-// staging loads follow the contiguous direction and the tile lands in LDS as [n][k] either way.  Any K, N, M: rows
-// and k past the end are staged as zeros.
+// round (an f16 a is widened exactly).  a may be contiguous along K (a K^T-style view of a cache) or along N (a V-style
+// view).  Any K, N, M: rows past the end are computed from the last row and not stored, k past the end is zero.
+//
+// What bounds it: at a head's 64 or 128 columns V p has few tiles and a long K, and scores have many tiles and a short K, so
+// neither fills the device with 128 x 128 tiles staged through LDS (what this kernel replaces); the operands come from
+// the caches either way.
+//   - A wave owns 32 rows of b and 64 columns of the result (two accumulators) and fetches its operands itself.  The
+//     matrix instruction adds over k in any order as long as both operands agree on it, so in a chunk of 16 k lane (r, h)
+//     takes k = 8h .. 8h+7: eight consecutive floats of a row that is contiguous along k, and one element per instruction
+//     of a row that is contiguous along n (32 lanes = one contiguous piece).  The next chunk is requested before the
+//     current one is multiplied; nothing meets at a barrier.
+//   - K_CONTIG (scores): the workgroup's four waves own neighbouring columns and all of K.  Otherwise (V p) they own
+//     the same 64 columns and every fourth chunk of K, and their sums meet in LDS at the end, in wave order.
+// Measured, us, 128 x 128 tiles against this: V p of 32 heads of 64, 300 rows over 600 keys 111.9 -> 22.4, 700 over 700 139.6 ->
+// 43.3, 17 over 517 81.1 -> 9.4; 32 heads of 128, 512 over 512 101.3 -> 33.1; scores of the same 29.1 -> 23.5, 61.5 -> 41.3, 13.6
+// -> 5.4, 51.8 -> 35.1.
 #include "common.h"
 
 namespace {
 
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
-constexpr int SM = 128, SN = 128, SK = 16;
-constexpr int S_STRIDE = SK + 1;  // floats per tile row: an odd stride spreads the 32 rows of a fragment over all banks
+constexpr int WM = 32, WN = 64, WK = 16;
+
+struct __attribute__((packed, aligned(4))) f32x8 {
+    float v[8];
+};
+struct __attribute__((packed, aligned(2))) f16x8 {
+    _Float16 v[8];
+};
+
+__device__ __forceinline__ void wt_load8(float (&d)[8], const float *p) {
+    const f32x8 t = *reinterpret_cast<const f32x8 *>(p);
+#pragma unroll
+    for (int e = 0; e < 8; e++) d[e] = t.v[e];
+}
+__device__ __forceinline__ void wt_load8(_Float16 (&d)[8], const _Float16 *p) {
+    const f16x8 t = *reinterpret_cast<const f16x8 *>(p);
+#pragma unroll
+    for (int e = 0; e < 8; e++) d[e] = t.v[e];
+}
 
 template <typename AT, bool K_CONTIG>
-__global__ __launch_bounds__(256) void gemm_f32_mfma(const AT *__restrict__ a, const float *__restrict__ b,
-                                                      float *__restrict__ dst, int K, int N, int M, int r2, int64_t a_s0,
-                                                      int64_t a_s1, int64_t a_s2) {
-    __shared__ float As[SM * S_STRIDE];  // rows of b (m)
-    __shared__ float Bs[SN * S_STRIDE];  // rows of a (n)
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * SM, n0 = blockIdx.x * SN, i2 = blockIdx.z;
+__global__ __launch_bounds__(256) void gemm_f32_wave_tiles(const AT *__restrict__ a, const float *__restrict__ b,
+                                                            float *__restrict__ dst, int K, int N, int M, int r2, int64_t a_s0,
+                                                            int64_t a_s1, int64_t a_s2, int n_tiles) {
+    __shared__ float part[K_CONTIG ? 1 : 3][2][16][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, h = lane >> 5;
+    const int mt = blockIdx.x / n_tiles, nt = blockIdx.x - mt * n_tiles;
+    const int m0 = mt * WM, i2 = blockIdx.y;
+    const int n0 = nt * (K_CONTIG ? 4 * WN : WN) + (K_CONTIG ? wave * WN : 0);
+    if (K_CONTIG && n0 >= N) return;
     const AT *ab = a + (int64_t)(i2 / r2) * a_s2;
-    const float *bb = b + (int64_t)i2 * M * K;
-    float *db = dst + (int64_t)i2 * M * N;
-
-    float16_t acc[2][2];
+    const float *brow = b + ((int64_t)i2 * M + min(m0 + r, M - 1)) * K;
+    const AT *acol[2];  // K_CONTIG: row n of the tile; otherwise its element of row k = 0
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+    for (int t = 0; t < 2; t++) acol[t] = ab + min(n0 + t * 32 + r, N - 1) * a_s1;
 
-    // staging along K: thread -> (tile row, half of the 16-wide k slice); along N: thread -> (k, 8 consecutive n)
-    const int srow = tid >> 1, sk = (tid & 1) * 8;
-    const int tk = tid >> 4, tn = (tid & 15) * 8;
-    const bool m_ok = m0 + srow < M, n_ok = n0 + srow < N;
-    const float *xp = bb + (size_t)min(m0 + srow, M - 1) * K;
-    const AT *wp = ab + (int64_t)min(n0 + srow, N - 1) * a_s1;
+    float16_t acc[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[t][e] = 0.0f;
 
-    for (int k0 = 0; k0 < K; k0 += SK) {
+    float bv[2][8];
+    AT av[2][2][8];
+    auto request = [&](int buf, int k0) {  // a whole chunk: k0 + 16 <= K
+        const int k = k0 + 8 * h;
+        wt_load8(bv[buf], brow + k);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            if (K_CONTIG) {
+                wt_load8(av[buf][t], acol[t] + k);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) av[buf][t][e] = acol[t][(int64_t)(k + e) * a_s0];
+            }
+        }
+    };
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[buf][e], (float)av[buf][t][e], acc[t], 0, 0, 0);
+    };
+    constexpr int STEP = K_CONTIG ? WK : 4 * WK;
+    int k0 = K_CONTIG ? 0 : wave * WK;
+    if (k0 + WK <= K) {
+        request(0, k0);
+        for (; k0 + STEP + WK <= K; k0 += 2 * STEP) {  // two chunks a turn: the buffers keep their registers
+            request(1, k0 + STEP);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(0);
+            if (k0 + 2 * STEP + WK > K) {
+                multiply(1);
+                k0 += 2 * STEP;
+                goto whole_chunks_done;
+            }
+            request(0, k0 + 2 * STEP);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(1);
+        }
+        multiply(0);
+        k0 += STEP;
+    }
+whole_chunks_done:
+    if (k0 < K) {  // the last, partial chunk: k past the end is zero in both operands and read in neither
+        const int k = k0 + 8 * h;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const int k = k0 + sk + e;
-            As[srow * S_STRIDE + sk + e] = (m_ok && k < K) ? xp[k] : 0.0f;
+            const bool in = k + e < K;
+            const int kk = in ? k + e : K - 1;
+            bv[0][e] = in ? brow[kk] : 0.0f;
+#pragma unroll
+            for (int t = 0; t < 2; t++) av[0][t][e] = in ? acol[t][K_CONTIG ? (int64_t)kk : (int64_t)kk * a_s0] : (AT)0.0f;
         }
-        if (K_CONTIG) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int k = k0 + sk + e;
-                Bs[srow * S_STRIDE + sk + e] = (n_ok && k < K) ? (float)wp[k] : 0.0f;
-            }
-        } else {
-            const int k = k0 + tk;
-            const AT *cp = ab + (int64_t)min(k, K - 1) * a_s0;
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int n = n0 + tn + e;
-                Bs[(tn + e) * S_STRIDE + tk] = (k < K && n < N) ? (float)cp[min(n, N - 1)] : 0.0f;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < SK / 2; ks++) {
-            float fa[2], fb[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) fa[i] = As[(wm * 64 + i * 32 + (lane & 31)) * S_STRIDE + ks * 2 + (lane >> 5)];
-#pragma unroll
-            for (int j = 0; j < 2; j++) fb[j] = Bs[(wn * 64 + j * 32 + (lane & 31)) * S_STRIDE + ks * 2 + (lane >> 5)];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
+        multiply(0);
     }
-
-    // C layout of the 32x32 MFMA (A rows = m, B rows = n): column n = lane % 32, row m = 8*(e/4) + 4*(lane/32) + e%4
+    if (!K_CONTIG) {
+        if (wave != 0) {
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int n = n0 + wn * 64 + j * 32 + (lane & 31);
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int m = m0 + wm * 64 + i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                if (m < M && n < N) db[(size_t)m * N + n] = acc[i][j][e];
-            }
+                for (int e = 0; e < 16; e++) part[wave - 1][t][e][lane] = acc[t][e];
         }
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int w = 0; w < 3; w++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[t][e] += part[w][t][e][lane];
+    }
+    // C layout of the 32x32 MFMA (A rows = m, B rows = n): column n = lane % 32, row m = 8*(e/4) + 4*(lane/32) + e%4
+    float *db = dst + (int64_t)i2 * M * N;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int n = n0 + t * 32 + r;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int m = m0 + 8 * (e >> 2) + 4 * h + (e & 3);
+            if (m < M && n < N) db[(size_t)m * N + n] = acc[t][e];
+        }
+    }
 }
 
 }  // namespace
@@ -105,14 +162,16 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma(const AT *__restrict__ a, c
 template <typename AT>
 bool gh_mul_mat_f32_mfma(galois_hip_ctx *ctx, const AT *a, const float *b, float *dst, int K, int N, int M, int ne02,
                          int ne12, int64_t a_s0, int64_t a_s1, int64_t a_s2) {
-    if (ne12 > 65535 || (M + SM - 1) / SM > 65535 || (a_s0 != 1 && a_s1 != 1)) return false;
-    const dim3 grid((N + SN - 1) / SN, (M + SM - 1) / SM, ne12);
+    const int64_t n_tiles = a_s0 == 1 ? ((int64_t)N + 4 * WN - 1) / (4 * WN) : ((int64_t)N + WN - 1) / WN;
+    const int64_t tiles = n_tiles * (((int64_t)M + WM - 1) / WM);
+    if (ne12 > 65535 || tiles > 0x7FFFFFFF || (a_s0 != 1 && a_s1 != 1)) return false;
+    const dim3 grid((unsigned)tiles, (unsigned)ne12);
     if (a_s0 == 1)
-        hipLaunchKernelGGL((gemm_f32_mfma<AT, true>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0,
-                           a_s1, a_s2);
+        hipLaunchKernelGGL((gemm_f32_wave_tiles<AT, true>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0,
+                           a_s1, a_s2, (int)n_tiles);
     else
-        hipLaunchKernelGGL((gemm_f32_mfma<AT, false>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0,
-                           a_s1, a_s2);
+        hipLaunchKernelGGL((gemm_f32_wave_tiles<AT, false>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0,
+                           a_s1, a_s2, (int)n_tiles);
     return true;
 }
 template bool gh_mul_mat_f32_mfma<float>(galois_hip_ctx *, const float *, const float *, float *, int, int, int, int, int,
