@@ -1121,7 +1121,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_swiglu_f16_panel(galois_hip_ctx *ctx,
     for (int j = 0; j < GEMM_MAX_MATS; j++) mats.col0[j] = 0x7FFFFFFF;
     mats.n_total = 96 * ((N + 47) / 48);
     mats.swiglu_out = static_cast<_Float16 *>(panel_out);
-    const int32_t st = M <= SK_MAX_SWIGLU_ROWS ? skinny_launch_any(ctx, mats, (const _Float16 *)panel, K, K / 32, M, true)
+    const int32_t st = M <= SK_MAX_ROWS ? skinny_launch_any(ctx, mats, (const _Float16 *)panel, K, K / 32, M, true)
                                                : gemm_launch_tile(ctx, mats, (const _Float16 *)panel, K, M, gemm_pick(ctx, mats.n_total, M, 96));
     if (st != GALOIS_HIP_OK) return st;
     GH_LAUNCH_CHECK(ctx, "mul_mat_q4_0_swiglu_f16_panel launch");

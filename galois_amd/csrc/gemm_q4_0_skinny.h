@@ -278,14 +278,13 @@ int32_t skinny_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16
     return GALOIS_HIP_OK;
 }
 
-// Rows up to which the panel calls run here rather than on the 256-row kernel.  Measured (us, this kernel / that one, weights
-// from HBM): q | k | v of 4096 (12288 x 4096) 14.1 / 25.3 at 23 rows, 19.8 / 28.0 at 77, 27.3 / 30.6 at 128, 30.0 / 28.2 at
-// 150; gate | up + SwiGLU (2 x 11008 x 4096) 20.3 / 41.1, 31.6 / 43.9, 40.0 / 43.9, 55 / 43.4; 4096 x 11008 14.7 / 52.8,
-// 20.3 / 53.3, 24.1 / 54.4; 4096 x 4096 7.1 / 23.0, 10.2 / 23.2, 11.9 / 22.7.  A result's sum order depends on K and
-// on the side of this line M is on, never on N: matrices multiplied together and one by one give the same bits.
-constexpr int SK_MAX_ROWS = 128;
-// gate | up: always wide, so the 128-row tile catches up sooner (31.6 / 31.7 us at 77 rows, 40.4 / 31.8 at 100).
-constexpr int SK_MAX_SWIGLU_ROWS = 80;
+// Rows up to which the panel calls run here rather than on the wide kernel.  Measured (us, this kernel / that one at its best
+// tile, weights from HBM): q | k | v of 4096 (12288 x 4096) 14.1 / 25.3 at 23 rows, 19.8 / 21.2 at 77, 27.1 / 20.9 at 100;
+// gate | up + SwiGLU (2 x 11008 x 4096) 20.3 / 41.1, 31.6 / 31.7, 40.4 / 31.8.  Narrow matrices stay ahead here for longer (11008 ->
+// 4096 24.9 / 44.5 at 100 rows, 4096 -> 4096 11.9 / 19.2), which gemm_pick_form uses where a caller lets the sums take any
+// order; in the plain calls the order of a result's sum depends on K and on the side of this line M is on, never on N, so
+// matrices multiplied together, one by one or with the SwiGLU behind them give the same bits.
+constexpr int SK_MAX_ROWS = 80;
 
 // Time of a workgroup relative to others, us at K = 4096 (fitted to the sizes above within 10 %): what a weight tile costs
 // (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.

@@ -194,8 +194,10 @@ int32_t galois_hip_dequantize_mul_mat_vec_q4_0_group(galois_hip_ctx *ctx, const 
  * matmul.cu:133-174,452-504) with one call: Y[m*N + n] = sum_k deq(W)[n,k] * X[m*K + k]
  * (output layout of matmul.cu:359).  W tiles are dequantised to fp16 in LDS, X is
  * rounded to fp16, products accumulate in f32 on MFMA.  K % 32 == 0.  No Q8_1
- * scratch and no K padding (src/cuda.rs:1040-1068) are needed.  The fp16 copy of X lives in a workspace the context
- * owns and grows on demand (the call allocates when a larger one is needed; refused during a graph capture).  A large
+ * scratch and no K padding (src/cuda.rs:1040-1068) are needed from the caller.  Few rows (up to 80), and a K that is
+ * no multiple of 256 or a W that is not 16-byte aligned, run on a kernel that dequantises in registers.  The fp16 copy of X lives in a workspace the context
+ * owns and grows on demand (the call allocates when a larger one is needed; refused during a graph capture, except
+ * for such K and W, which then run without a workspace).  A large
  * product whose N leaves compute units idle (512 x 11008 x 4096 on 256 CUs) is computed as two shares of k that a
  * second launch adds: the f32 sums over k are then two chains instead of one, for the same operands on the same
  * device always the same way. */
@@ -345,9 +347,11 @@ int32_t galois_hip_attn_decode_f16kv(galois_hip_ctx *ctx, const float *q, const 
 
 /* The q | k | v products of a decode step (three CudaMatMul launches, src/cuda.rs:1011-1034, with whatever
  * normalisation galois_hip_dequantize_mul_mat_vec_q4_0_group folds in) and the attention that consumes them
- * (galois_hip_attn_decode_f32 / _f16kv above) as ONE launch: qkv[0..2] are the three products, whose dst are the
+ * (galois_hip_attn_decode_f32 / _f16kv above) as one call: qkv[0..2] are the three products, whose dst are the
  * q, k and v vectors of n_head * head_dim floats (written as by the group call, and read by the attention part).
- * The attention's workgroups follow the products' in the grid, request their cache rows while the last products
+ * Where there is enough of both to overlap (a cache of 38 MB or more up to n_past, nine product workgroups or more
+ * per four compute units) the call is ONE launch, otherwise the two launches of those calls.  In one launch the
+ * attention's workgroups follow the products' in the grid, request their cache rows while the last products
  * still stream, and wait -- bounded -- only for their own head's rows of q (k and v where position n_past lives);
  * should a wait ever run out, that head's whole output is NaN, the context's status word is set and the next synchronize
  * or *_sync_copy returns GALOIS_HIP_E_DEVICE_WAIT (once) after returning the counters to zero.  q, k, v and the appended cache rows equal those of the two
@@ -367,9 +371,9 @@ int32_t galois_hip_qkv_attn_decode_f16kv(galois_hip_ctx *ctx, const galois_hip_g
  *   - with 2 * M * N floats of it, a matrix too narrow to give every compute unit a workgroup (N = 4096 at M = 512:
  *     86 tiles of 96 columns, or 172 of 48, for 256 CUs) is multiplied as two shares of k by 256 workgroups of 64
  *     columns, and the pass that adds the residual adds the two partial results as well (M = 512, 11008 -> 4096 with
- *     the residual: 70 -> 55 us);
+ *     the residual: 70 -> 55 us), or, with few rows, by the few-rows kernel (11008 -> 4096 at 150 rows 57 -> 27 us);
  *   - Y may be the residual itself (the stream updated in place) when the workspace holds M * N floats or more.
- * The two shapes differ in the order of the f32 sums over k (one chain, or two halves added), i.e. by rounding only;
+ * The shapes differ in the order of the f32 sums over k (one chain, or parts added), i.e. by rounding only;
  * which one runs depends on shape, workspace and device alone, so a call repeats bit for bit.  One or two launches
  * (the product, then the adding pass when there is a residual or a second share). */
 int32_t galois_hip_mul_mat_q4_0_f16_panel_add(galois_hip_ctx *ctx, const void *W, const void *panel, const float *residual,

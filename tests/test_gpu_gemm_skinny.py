@@ -51,17 +51,18 @@ def test_tiles_and_remainders(dev, m, k, n):
 @pytest.mark.parametrize("m", [5, 70, 150])
 def test_the_alignment_of_the_weights_does_not_change_a_bit(dev, m, k):
     """2-byte aligned rows take their blocks apart differently; weights, products and sums stay the same.  (At K = 256
-    and 150 rows the 16-byte aligned weights run on the 256-row kernel, whose sums go in another order.)"""
+    and 150 rows the 16-byte aligned weights run on the wide kernel, whose sums go in another order.)"""
     wq, x = _case(m * k, m, k, 90)
     ref = _run(dev, wq, x, 4)
-    for shift in (2, 6, 8) + (() if k == 256 and m > 128 else (0,)):
+    for shift in (2, 6, 8) + (() if k == 256 and m > 80 else (0,)):
         assert np.array_equal(_run(dev, wq, x, shift).view(np.uint32), ref.view(np.uint32)), shift
 
 
 def test_a_result_does_not_depend_on_its_neighbours(dev):
     """Columns of a wide matrix equal the same rows multiplied as a matrix of their own, rows of a batch the same rows
-    in a smaller batch: tiles, rounds and row blocks change, the order of a result's sum does not."""
-    wq, x = _case(11, 100, 2048, 6000)
+    in a smaller batch (up to 80 rows, where the wide kernel takes over): tiles, rounds and row blocks change, the order of a
+    result's sum does not."""
+    wq, x = _case(11, 80, 2048, 6000)
     whole = _run(dev, wq, x)
     assert np.array_equal(whole[:, 333:350], _run(dev, wq[333:350], x))
     assert np.array_equal(whole[:37], _run(dev, wq, x[:37]))
@@ -105,7 +106,7 @@ def test_a_fresh_context_captures_a_ragged_product(dev):
     d2.close()
 
 
-@pytest.mark.parametrize("m,k,n", [(16, 256, 256), (45, 2048, 768), (80, 4096, 2816), (112, 8192, 256)])
+@pytest.mark.parametrize("m,k,n", [(16, 256, 256), (45, 2048, 768), (80, 4096, 2816), (81, 1024, 512), (112, 8192, 256)])
 def test_swiglu_and_several_matrices(dev, m, k, n):
     """gate | up with the SwiGLU in the epilogue against the oracle's ops (twice the bar: the result is a product of two), and
     matrices whose boundaries fall inside a tile."""
@@ -130,9 +131,9 @@ def test_swiglu_and_several_matrices(dev, m, k, n):
         dev.free(b)
 
 
-@pytest.mark.parametrize("m,n", [(129, 5000), (150, 12288), (192, 700), (193, 11008), (300, 12288), (385, 9000), (640, 2000)])
+@pytest.mark.parametrize("m,n", [(81, 3000), (128, 11008), (129, 5000), (150, 12288), (192, 700), (193, 11008), (300, 12288), (385, 9000), (640, 2000)])
 def test_row_tiles_of_the_wide_kernel(dev, m, n):
-    """129 rows and up: tiles of 128, 192 or 256 rows and 96 or 48 columns by the workgroups they give.  Against the oracle on a
+    """81 rows and up: tiles of 128, 192 or 256 rows and 96 or 48 columns by the workgroups they give.  Against the oracle on a
     sample, and the first 140 rows bit for bit as a batch of their own (another tile, the same order of sums)."""
     k = 512
     wq, x = _case(m + n, m, k, n)
@@ -144,7 +145,7 @@ def test_row_tiles_of_the_wide_kernel(dev, m, n):
         assert np.array_equal(got[:140].view(np.uint32), _run(dev, wq, x[:140]).view(np.uint32))
 
 
-@pytest.mark.parametrize("m,k,n", [(150, 4096, 768), (190, 1024, 512), (300, 4096, 4096), (390, 2048, 1024)])
+@pytest.mark.parametrize("m,k,n", [(100, 8192, 1024), (150, 4096, 768), (190, 1024, 512), (300, 4096, 4096), (390, 2048, 1024)])
 def test_forms_of_a_narrow_product(dev, m, k, n):
     """With a workspace a narrow product comes whole, in two shares of k or from the few-rows kernel: each sums the same f32
     products in its own order (1e-5 of the largest result)."""
