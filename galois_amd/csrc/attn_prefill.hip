@@ -57,7 +57,14 @@ struct pa_args {
     _Float16 *panel;    // the prefill matmul's fp16 panel of a [n_head * 128, n] operand
     int n, n_past, n_head, tiles;
     float qscale;       // scale * log2(e): the softmax runs in base 2
+    float *part;        // PA_PARTS: the records of the splits
+    int splits;
 };
+
+// Where a workgroup's result goes: f32 rows, the fp16 panel, or (the keys split over several workgroups) a record of its
+// 64 queries: their unnormalised outputs [64][128], then their maxima and sums [64] each.
+enum { PA_ROWS, PA_PANEL, PA_PARTS };
+constexpr int PA_REC = 64 * (PA_D + 2);  // floats
 
 __device__ __forceinline__ uint32_t pa_pack(float a, float b) {
     half2_t h;
@@ -155,7 +162,7 @@ __device__ __forceinline__ void pa_store(const pa_stage_regs<KV16> &s, unsigned 
     }
 }
 
-template <int QT, bool KV16, bool PANEL>
+template <int QT, bool KV16, int OUT>
 __global__ __launch_bounds__(PA_THREADS) void attn_prefill_kernel(const pa_args a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // two stages of two blocks: [K 32 x 272 | V^T 128 x 80]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
@@ -164,11 +171,15 @@ __global__ __launch_bounds__(PA_THREADS) void attn_prefill_kernel(const pa_args 
     const int t = tid & 255;
     constexpr int BM = 64 * QT;
     const int head = blockIdx.x % a.n_head;
-    const int tile = a.tiles - 1 - blockIdx.x / a.n_head;  // long walks first
+    const int rest = blockIdx.x / a.n_head, sp = OUT == PA_PARTS ? rest / a.tiles : 0;
+    const int tile = a.tiles - 1 - (rest - sp * a.tiles);  // long walks first
     const int m0 = tile * BM;
     const int m_last = (m0 + BM < a.n ? m0 + BM : a.n) - 1;   // the workgroup's last live query
     const int kend = a.n_past + m_last + 1;                   // keys it may see
     const int nstage = (kend + 2 * PA_BK - 1) / (2 * PA_BK);
+    // the stages of this workgroup's split (none, if the tile's walk is shorter than the number of splits)
+    const int sg0 = OUT == PA_PARTS ? (int)((int64_t)sp * nstage / a.splits) : 0;
+    const int sg1 = OUT == PA_PARTS ? (int)((int64_t)(sp + 1) * nstage / a.splits) : nstage;
     const int64_t E = (int64_t)a.n_head * PA_D;
     const int mw0 = m0 + wq * 16 * QT;                        // the wave's first query
 
@@ -201,12 +212,14 @@ __global__ __launch_bounds__(PA_THREADS) void attn_prefill_kernel(const pa_args 
     }
 
     pa_stage_regs<KV16> st;
-    pa_fetch<KV16>(st, a, head, half, kend, t);
-    pa_store<KV16>(st, lds + half * PA_BLOCK, half, kend, t);
+    if (OUT != PA_PARTS || sg0 < sg1) {
+        pa_fetch<KV16>(st, a, head, sg0 * 2 + half, kend, t);
+        pa_store<KV16>(st, lds + (sg0 & 1) * PA_STAGE + half * PA_BLOCK, sg0 * 2 + half, kend, t);
+    }
     __syncthreads();
 
-    for (int sg = 0; sg < nstage; sg++) {
-        const bool more = sg + 1 < nstage;
+    for (int sg = sg0; sg < sg1; sg++) {
+        const bool more = sg + 1 < sg1;
         if (more) pa_fetch<KV16>(st, a, head, (sg + 1) * 2 + half, kend, t);
         const unsigned char *ks = lds + (sg & 1) * PA_STAGE + half * PA_BLOCK, *vt = ks + PA_KBYTES;
         const int key0 = (sg * 2 + half) * PA_BK;
@@ -290,20 +303,28 @@ __global__ __launch_bounds__(PA_THREADS) void attn_prefill_kernel(const pa_args 
 #pragma unroll
     for (int qt = 0; qt < QT; qt++) {
         const float *x = xch + qt * 34 * 64;
-        // the first wave has seen key 0, so the common maximum is finite
+        // the first wave has seen key 0, so the common maximum is finite -- unless the walk began further on, behind the
+        // mask of some query: its maximum stays -inf, its sum and output are zeros
         const float m2 = x[0], m_all = fmaxf(m_run[qt], m2);
-        const float a1 = __builtin_amdgcn_exp2f(m_run[qt] - m_all), a2 = __builtin_amdgcn_exp2f(m2 - m_all);
+        const float m_ref = OUT == PA_PARTS && m_all == -INFINITY ? 0.0f : m_all;
+        const float a1 = __builtin_amdgcn_exp2f(m_run[qt] - m_ref), a2 = __builtin_amdgcn_exp2f(m2 - m_ref);
         float l = l_run[qt] * a1 + x[64] * a2;
         l += __shfl_xor(l, 16);
         l += __shfl_xor(l, 32);
-        const float inv = 1.0f / l;
+        const float inv = OUT == PA_PARTS ? 1.0f : 1.0f / l;
         float4_t o[8];
 #pragma unroll
         for (int tt = 0; tt < 8; tt++)
 #pragma unroll
             for (int j = 0; j < 4; j++) o[tt][j] = (acc[qt][tt][j] * a1 + x[(2 + tt * 4 + j) * 64] * a2) * inv;
         const int m = mw0 + qt * 16 + r;
-        if (PANEL) {
+        if (OUT == PA_PARTS) {
+            float *rec = a.part + ((int64_t)(sp * a.tiles + tile) * a.n_head + head) * PA_REC;
+            const int q = wq * 16 + r;  // QT = 1
+#pragma unroll
+            for (int tt = 0; tt < 8; tt++) *reinterpret_cast<float4_t *>(rec + q * PA_D + tt * 16 + g * 4) = o[tt];
+            if (g == 0) rec[64 * PA_D + q] = m_all, rec[64 * PA_D + 64 + q] = l;
+        } else if (OUT == PA_PANEL) {
             // element (m, k) of the panel: tile (m / 16, k / 32) of 1 KB, 16-byte piece ((k % 32) / 8) * 16 + m % 16
             const int m_pad = (a.n + 15) & ~15;
             if (m < m_pad) {
@@ -324,20 +345,80 @@ __global__ __launch_bounds__(PA_THREADS) void attn_prefill_kernel(const pa_args 
     }
 }
 
-template <int QT, bool KV16, bool PANEL>
+// The splits of a row and head together: four dims a thread, every split's record fetched at once.
+constexpr int PA_MAX_SPLITS = 8;
+__global__ __launch_bounds__(256) void attn_prefill_merge(const pa_args a) {
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int d = (int)(id & 31) * 4;
+    const int head = (int)((id >> 5) % a.n_head), m = (int)((id >> 5) / a.n_head);
+    const int m_end = a.panel ? (a.n + 15) & ~15 : a.n;
+    if (m >= m_end) return;
+    const int tile = m >> 6, q = m & 63;
+    float4_t o = {0.f, 0.f, 0.f, 0.f};
+    if (m < a.n) {
+        float ms[PA_MAX_SPLITS], ls[PA_MAX_SPLITS];
+        float4_t os[PA_MAX_SPLITS];
+#pragma unroll
+        for (int sp = 0; sp < PA_MAX_SPLITS; sp++) {
+            const float *rec = a.part + ((int64_t)(min(sp, a.splits - 1) * a.tiles + tile) * a.n_head + head) * PA_REC;
+            ms[sp] = rec[64 * PA_D + q], ls[sp] = rec[64 * PA_D + 64 + q];
+            os[sp] = *reinterpret_cast<const float4_t *>(rec + q * PA_D + d);
+        }
+        float mx = ms[0];  // finite: the first split begins with key 0, which every query sees
+#pragma unroll
+        for (int sp = 1; sp < PA_MAX_SPLITS; sp++) mx = fmaxf(mx, ms[sp]);
+        float l = 0.0f;
+#pragma unroll
+        for (int sp = 0; sp < PA_MAX_SPLITS; sp++)
+            if (sp < a.splits) {
+                const float w = __builtin_amdgcn_exp2f(ms[sp] - mx);
+                l += ls[sp] * w;
+                o += os[sp] * w;
+            }
+        o *= 1.0f / l;
+    }
+    const int64_t E = (int64_t)a.n_head * PA_D;
+    if (a.panel) {  // rows past n are zeros in a panel
+        unsigned char *p = reinterpret_cast<unsigned char *>(a.panel) + ((int64_t)(m >> 4) * (E >> 5) + head * 4 + (d >> 5)) * 1024 +
+                           ((d & 31) >> 3) * 256 + (m & 15) * 16 + (d & 7) * 2;
+        *reinterpret_cast<uint2 *>(p) = make_uint2(pa_pack(o[0], o[1]), pa_pack(o[2], o[3]));
+    } else {
+        *reinterpret_cast<float4_t *>(a.out + m * E + (int64_t)head * PA_D + d) = o;
+    }
+}
+
+template <int QT, bool KV16, int OUT>
 hipError_t pa_launch_one(galois_hip_ctx *ctx, const pa_args &a) {
-    const hipError_t e = hipFuncSetAttribute((const void *)attn_prefill_kernel<QT, KV16, PANEL>,
+    const hipError_t e = hipFuncSetAttribute((const void *)attn_prefill_kernel<QT, KV16, OUT>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, PA_LDS);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((attn_prefill_kernel<QT, KV16, PANEL>), dim3((unsigned)(a.tiles * a.n_head)), dim3(PA_THREADS), PA_LDS,
-                       ctx->stream, a);
+    hipLaunchKernelGGL((attn_prefill_kernel<QT, KV16, OUT>), dim3((unsigned)(a.tiles * a.n_head * (OUT == PA_PARTS ? a.splits : 1))),
+                       dim3(PA_THREADS), PA_LDS, ctx->stream, a);
     return hipSuccess;
 }
 
-template <int QT>
-hipError_t pa_launch(galois_hip_ctx *ctx, const pa_args &a, bool kv16, bool panel) {
-    if (kv16) return panel ? pa_launch_one<QT, true, true>(ctx, a) : pa_launch_one<QT, true, false>(ctx, a);
-    return panel ? pa_launch_one<QT, false, true>(ctx, a) : pa_launch_one<QT, false, false>(ctx, a);
+template <int QT, int OUT>
+hipError_t pa_launch(galois_hip_ctx *ctx, const pa_args &a, bool kv16) {
+    return kv16 ? pa_launch_one<QT, true, OUT>(ctx, a) : pa_launch_one<QT, false, OUT>(ctx, a);
+}
+
+// Over how many workgroups the keys of a tile are split.  A stage of 64 keys costs a CU about 1.3 us from an f16 cache and 1.75
+// us from an f32 one whatever the workgroup does with it (measured with the arithmetic compiled out: the same), because
+// that is what one CU fetches, so a launch that leaves CUs without a workgroup gains by handing them keys; the merge is a second
+// launch and two passes over the records.  Measured, us,
+// whole / split, f32 cache: 32 heads, 9 rows behind 1900 positions 57.0 / 20.6, 40 behind 1000 34.6 / 16.8, 100 behind 1900 58.8 /
+// 26.7, 150 behind 1201 41.2 / 29.2 (f16 43.6 / 17.5, 25.0 / 14.9, 45.9 / 22.6, 32.0 / 25.8); 8 heads, 512 behind 1536 49.9 / 26.0.
+// Where the model keeps the keys whole every forced split is slower (32 heads, 300 behind 600 29.8 / 31.9; 512 behind 1536 59.5 /
+// 65.3; 150 rows alone 8.4 / 13.8).
+int pa_pick_splits(int64_t wgs, int64_t cus, int nstage, bool kv16) {
+    const double stage = kv16 ? 1.3 : 1.75;
+    int best = 1;
+    double best_us = (double)((wgs + cus - 1) / cus) * (nstage * stage + 4.0) - 2.0;  // a split has to gain 2 us
+    for (int s = 2; s <= PA_MAX_SPLITS && wgs * s <= 2 * cus; s++) {
+        const double us = (double)((wgs * s + cus - 1) / cus) * (((nstage + s - 1) / s) * stage + 4.0) + 6.0 + 0.022 * (double)(wgs * s);
+        if (us < best_us) best = s, best_us = us;
+    }
+    return best;
 }
 
 int32_t pa_entry(galois_hip_ctx *ctx, const float *q, const void *k_cache, const void *v_cache, bool kv16, float *out, void *out_panel,
@@ -365,7 +446,25 @@ int32_t pa_entry(galois_hip_ctx *ctx, const float *q, const void *k_cache, const
     const int qt = (wg64 >= 4 * cus || (wg64 >= 2 * cus && n_past >= n_tokens)) ? 2 : 1;
     a.tiles = (n_tokens + 64 * qt - 1) / (64 * qt);
     GH_REQUIRE(ctx, (int64_t)a.tiles * n_head < ((int64_t)1 << 31), GALOIS_HIP_E_SHAPE, "attn_prefill: too many workgroups");
-    const hipError_t e = qt == 2 ? pa_launch<2>(ctx, a, kv16, out_panel != nullptr) : pa_launch<1>(ctx, a, kv16, out_panel != nullptr);
+    a.part = nullptr, a.splits = 1;
+    if (qt == 1) {
+        const int splits = pa_pick_splits(wg64, cus, (n_past + n_tokens + 63) / 64, kv16);
+        // the records live in the context's workspace; without one (while a graph is captured, or out of memory) the keys stay whole
+        if (splits > 1 && gh_reserve_workspace(ctx, (size_t)(wg64 * splits) * PA_REC * sizeof(float)))
+            a.splits = splits, a.part = static_cast<float *>(ctx->ws);
+    }
+    hipError_t e;
+    if (a.splits > 1) {
+        e = pa_launch<1, PA_PARTS>(ctx, a, kv16);
+        if (e == hipSuccess) {
+            const int64_t threads = (int64_t)((n_tokens + 15) / 16 * 16) * n_head * 32;
+            hipLaunchKernelGGL(attn_prefill_merge, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, a);
+        }
+    } else if (out_panel) {
+        e = qt == 2 ? pa_launch<2, PA_PANEL>(ctx, a, kv16) : pa_launch<1, PA_PANEL>(ctx, a, kv16);
+    } else {
+        e = qt == 2 ? pa_launch<2, PA_ROWS>(ctx, a, kv16) : pa_launch<1, PA_ROWS>(ctx, a, kv16);
+    }
     if (e != hipSuccess) return gh_hip(ctx, e, "hipFuncSetAttribute(LDS size)");
     GH_LAUNCH_CHECK(ctx, "attn_prefill");
 }

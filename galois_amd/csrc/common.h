@@ -73,6 +73,10 @@ static inline int32_t gh_hip(galois_hip_ctx *ctx, hipError_t e, const char *what
     } while (0)
 
 // Calls that allocate, free or block are refused while the stream is being captured.
+// Grows the context's workspace to `need` bytes; false when that would take an allocation during a capture, or when it
+// fails (device.hip).  What is in the workspace does not outlive a call.
+bool gh_reserve_workspace(galois_hip_ctx *ctx, size_t need);
+
 #define GH_NOT_CAPTURING(ctx, what) GH_REQUIRE((ctx), !(ctx)->capturing, GALOIS_HIP_E_UNSUPPORTED, what " during a graph capture")
 
 // Binds the context's device to the calling thread, then checks the launch that follows.

@@ -18,6 +18,23 @@ int32_t gh_check_device_status(galois_hip_ctx *ctx) {
                    "have been cleared: the context can be used again)");
 }
 
+bool gh_reserve_workspace(galois_hip_ctx *ctx, size_t need) {
+    if (ctx->ws_bytes >= need) return true;
+    if (ctx->capturing) return false;
+    // The outgrown block is kept until the context dies: work already queued, or a graph captured earlier, has its address
+    // baked in.  Growing by at least half bounds what the retired blocks add up to.
+    const size_t bytes = need > ctx->ws_bytes + ctx->ws_bytes / 2 ? need : ctx->ws_bytes + ctx->ws_bytes / 2;
+    void *grown = nullptr;
+    if (hipMalloc(&grown, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (ctx->ws) ctx->ws_retired.push_back(ctx->ws);
+    ctx->ws = grown;
+    ctx->ws_bytes = bytes;
+    return true;
+}
+
 extern "C" {
 
 const char *galois_hip_status_string(int32_t s) {

@@ -882,29 +882,14 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
     const bool shares = !skinny && mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_pick_form(ctx, K, N, M, 1.1, 64.0) == GEMM_TWO_SHARES;
     const size_t need = panel_bytes + (shares ? 2 * (size_t)mn * sizeof(float) : 0);
     bool panel = gemm_panel_shape_ok((int32_t)k_pad, M);
-    if (panel && ctx->ws_bytes < need) {
-        // weights that are not laid out in pieces of 256 have a kernel that needs no workspace: while a graph is being
-        // captured they run on it rather than fail
-        if (!wide && ctx->capturing) {
-            panel = false;
-        } else {
+    if (panel && !gh_reserve_workspace(ctx, need)) {
+        // weights that are not laid out in pieces of 256 have a kernel that needs no workspace, and run on it rather than
+        // fail while a graph is being captured (or when memory is short)
+        if (wide) {
             GH_NOT_CAPTURING(ctx, "mul_mat_q4_0_f32: growing the workspace");
-            // The outgrown block is kept until the context dies: work already queued, or a graph captured earlier,
-            // has its address baked in.  Growing by at least half bounds what the retired blocks add up to.
-            const size_t bytes = need > ctx->ws_bytes + ctx->ws_bytes / 2 ? need : ctx->ws_bytes + ctx->ws_bytes / 2;
-            void *grown = nullptr;
-            const hipError_t e = hipMalloc(&grown, bytes);
-            if (e == hipSuccess) {
-                if (ctx->ws) ctx->ws_retired.push_back(ctx->ws);
-                ctx->ws = grown;
-                ctx->ws_bytes = bytes;
-            } else if (wide) {
-                return gh_hip(ctx, e, "hipMalloc(workspace)");
-            } else {
-                (void)hipGetLastError();
-                panel = false;
-            }
+            return gh_hip(ctx, hipErrorOutOfMemory, "hipMalloc(workspace)");
         }
+        panel = false;
     }
     if (panel) {
         _Float16 *Xh = (_Float16 *)ctx->ws;
