@@ -410,16 +410,19 @@ hipError_t pa_launch(galois_hip_ctx *ctx, const pa_args &a, bool kv16) {
 // 26.7, 150 behind 1201 41.2 / 29.2 (f16 43.6 / 17.5, 25.0 / 14.9, 45.9 / 22.6, 32.0 / 25.8); 8 heads, 512 behind 1536 49.9 / 26.0.
 // Where the model keeps the keys whole every forced split is slower (32 heads, 300 behind 600 29.8 / 31.9; 512 behind 1536 59.5 /
 // 65.3; 150 rows alone 8.4 / 13.8).
+constexpr int PA_SPLIT_ROUNDS = 2;  // workgroups per CU a split launch has at most: bounds its records (33 KB each)
 int pa_pick_splits(int64_t wgs, int64_t cus, int nstage, bool kv16) {
     const double stage = kv16 ? 1.3 : 1.75;
     int best = 1;
     double best_us = (double)((wgs + cus - 1) / cus) * (nstage * stage + 4.0) - 2.0;  // a split has to gain 2 us
-    for (int s = 2; s <= PA_MAX_SPLITS && wgs * s <= 2 * cus; s++) {
+    for (int s = 2; s <= PA_MAX_SPLITS && wgs * s <= PA_SPLIT_ROUNDS * cus; s++) {
         const double us = (double)((wgs * s + cus - 1) / cus) * (((nstage + s - 1) / s) * stage + 4.0) + 6.0 + 0.022 * (double)(wgs * s);
         if (us < best_us) best = s, best_us = us;
     }
     return best;
 }
+
+int64_t pa_cus(int32_t n_cu) { return n_cu > 0 ? n_cu : 256; }
 
 int32_t pa_entry(galois_hip_ctx *ctx, const float *q, const void *k_cache, const void *v_cache, bool kv16, float *out, void *out_panel,
                  int32_t n_head, int32_t head_dim, int32_t n_tokens, int32_t n_past, float scale) {
@@ -442,16 +445,16 @@ int32_t pa_entry(galois_hip_ctx *ctx, const float *q, const void *k_cache, const
     // that the causal walks differ by at most a factor of two).  Measured on 256 CUs, 32 heads, f32 cache, us for 64 /
     // 128 queries: 512 rows 15.7 / 22.4, 1024 rows 31.0 / 37.4, 2048 rows 112 / 82.6, 1024 rows behind 1024 positions
     // 83.7 / 72.0, 512 behind 1536 59.0 / 71.4; 8 heads x 4096 rows 100 / 124.
-    const int64_t wg64 = ((int64_t)n_tokens + 63) / 64 * n_head, cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
+    const int64_t wg64 = ((int64_t)n_tokens + 63) / 64 * n_head, cus = pa_cus(ctx->n_cu);
     const int qt = (wg64 >= 4 * cus || (wg64 >= 2 * cus && n_past >= n_tokens)) ? 2 : 1;
     a.tiles = (n_tokens + 64 * qt - 1) / (64 * qt);
     GH_REQUIRE(ctx, (int64_t)a.tiles * n_head < ((int64_t)1 << 31), GALOIS_HIP_E_SHAPE, "attn_prefill: too many workgroups");
     a.part = nullptr, a.splits = 1;
     if (qt == 1) {
-        const int splits = pa_pick_splits(wg64, cus, (n_past + n_tokens + 63) / 64, kv16);
-        // the records live in the context's workspace; without one (while a graph is captured, or out of memory) the keys stay whole
-        if (splits > 1 && gh_reserve_workspace(ctx, (size_t)(wg64 * splits) * PA_REC * sizeof(float)))
-            a.splits = splits, a.part = static_cast<float *>(ctx->ws);
+        // the records have a block of their own in the context, so the same call takes the same path in every context, in
+        // and out of a capture, and allocates nothing
+        a.splits = pa_pick_splits(wg64, cus, (n_past + n_tokens + 63) / 64, kv16);
+        a.part = static_cast<float *>(ctx->attn_records);
     }
     hipError_t e;
     if (a.splits > 1) {
@@ -470,6 +473,8 @@ int32_t pa_entry(galois_hip_ctx *ctx, const float *q, const void *k_cache, const
 }
 
 }  // namespace
+
+size_t gh_attn_records_bytes(int32_t n_cu) { return (size_t)(PA_SPLIT_ROUNDS * pa_cus(n_cu)) * PA_REC * sizeof(float); }
 
 extern "C" int32_t galois_hip_attn_prefill_f32(galois_hip_ctx *ctx, const float *q, const float *k_cache, const float *v_cache,
                                                float *out, void *out_panel, int32_t n_head, int32_t head_dim, int32_t n_tokens,

@@ -19,6 +19,7 @@ struct galois_hip_ctx {
     void *scratch;    // fixed block made at creation: partial sums of the split f32 matmul, partial results of the decode attention
     unsigned *attn_done;  // 4 x GH_ATTN_HEADS counters, zero between calls: splits finished per head (decode attention), then
                           // per head the workgroups that have stored its q, its k, its v (the launch that carries both)
+    void *attn_records;   // fixed block made at creation: the records of a prefill attention whose keys are split over workgroups
     void *attn_static;    // this device's copy of the decode attention's static scratch (attn_decode.hip), found at creation
                           // (null if the lookup failed: only the entry point that needs it then refuses)
     unsigned *dev_status;      // one word of pinned host memory that kernels set when a bounded wait inside a launch runs
@@ -73,10 +74,6 @@ static inline int32_t gh_hip(galois_hip_ctx *ctx, hipError_t e, const char *what
     } while (0)
 
 // Calls that allocate, free or block are refused while the stream is being captured.
-// Grows the context's workspace to `need` bytes; false when that would take an allocation during a capture, or when it
-// fails (device.hip).  What is in the workspace does not outlive a call.
-bool gh_reserve_workspace(galois_hip_ctx *ctx, size_t need);
-
 #define GH_NOT_CAPTURING(ctx, what) GH_REQUIRE((ctx), !(ctx)->capturing, GALOIS_HIP_E_UNSUPPORTED, what " during a graph capture")
 
 // Binds the context's device to the calling thread, then checks the launch that follows.
@@ -87,6 +84,13 @@ bool gh_reserve_workspace(galois_hip_ctx *ctx, size_t need);
     } while (0)
 
 #define GH_LAUNCH_CHECK(ctx, what) return gh_hip((ctx), hipGetLastError(), (what))
+
+// device.hip: grows the context's workspace to `need` bytes; false when that would take an allocation during a capture, or
+// when it fails.  What is in the workspace does not outlive a call.
+bool gh_reserve_workspace(galois_hip_ctx *ctx, size_t need);
+
+// attn_prefill.hip: the bytes galois_hip_ctx::attn_records holds.
+size_t gh_attn_records_bytes(int32_t n_cu);
 
 // device.hip: after a wait for the stream, reports (and clears) what kernels left in the context's status word.
 int32_t gh_check_device_status(galois_hip_ctx *ctx);

@@ -435,9 +435,10 @@ int32_t galois_hip_rope_qk_append(galois_hip_ctx *ctx, const float *q, const flo
  * few units (unit-variance q and k); rounding q and k moves a score by about 2^-11 of the size of its terms and the
  * exponential makes that a relative error of the probabilities, so scores of +-100 are held to 5e-3.
  * head_dim 128; all pointers 16-byte aligned.  Few rows behind a long context leave compute
- * units without work: their keys are then split over several workgroups, whose records live in the context's workspace
- * (grown on demand, at most 17 MB; without one, as while a graph is captured, the keys stay whole), and a second launch
- * merges them: the same result up to the rounding of the probabilities. */
+ * units without work: their keys are then split over several workgroups, whose records live in a block the context
+ * made at creation (17 MB on 256 compute units), and a second launch merges them: the same result up to the rounding of
+ * the probabilities.  Which of the two runs depends on sizes, cache type and device alone, so a call repeats bit for bit in
+ * every context, captured or not; it allocates nothing. */
 int32_t galois_hip_attn_prefill_f32(galois_hip_ctx *ctx, const float *q, const float *k_cache, const float *v_cache, float *out,
                                     void *out_panel, int32_t n_head, int32_t head_dim, int32_t n_tokens, int32_t n_past,
                                     float scale);
