@@ -451,10 +451,10 @@ int32_t pa_entry(galois_hip_ctx *ctx, const float *q, const void *k_cache, const
     GH_REQUIRE(ctx, (int64_t)a.tiles * n_head < ((int64_t)1 << 31), GALOIS_HIP_E_SHAPE, "attn_prefill: too many workgroups");
     a.part = nullptr, a.splits = 1;
     if (qt == 1) {
-        // the records have a block of their own in the context, so the same call takes the same path in every context, in
+        // the records live in a block that every context has, so the same call takes the same path in every context, in
         // and out of a capture, and allocates nothing
         a.splits = pa_pick_splits(wg64, cus, (n_past + n_tokens + 63) / 64, kv16);
-        a.part = static_cast<float *>(ctx->attn_records);
+        a.part = static_cast<float *>(ctx->block);
     }
     hipError_t e;
     if (a.splits > 1) {
@@ -474,7 +474,7 @@ int32_t pa_entry(galois_hip_ctx *ctx, const float *q, const void *k_cache, const
 
 }  // namespace
 
-size_t gh_attn_records_bytes(int32_t n_cu) { return (size_t)(PA_SPLIT_ROUNDS * pa_cus(n_cu)) * PA_REC * sizeof(float); }
+size_t gh_block_bytes(int32_t n_cu) { return (size_t)(PA_SPLIT_ROUNDS * pa_cus(n_cu)) * PA_REC * sizeof(float); }
 
 extern "C" int32_t galois_hip_attn_prefill_f32(galois_hip_ctx *ctx, const float *q, const float *k_cache, const float *v_cache,
                                                float *out, void *out_panel, int32_t n_head, int32_t head_dim, int32_t n_tokens,

@@ -19,7 +19,8 @@ struct galois_hip_ctx {
     void *scratch;    // fixed block made at creation: partial sums of the split f32 matmul, partial results of the decode attention
     unsigned *attn_done;  // 4 x GH_ATTN_HEADS counters, zero between calls: splits finished per head (decode attention), then
                           // per head the workgroups that have stored its q, its k, its v (the launch that carries both)
-    void *attn_records;   // fixed block made at creation: the records of a prefill attention whose keys are split over workgroups
+    void *block;          // fixed block made at creation, gh_block_bytes(n_cu): the records of a prefill attention whose keys are
+                          // split over workgroups; the panel of a ragged product that finds the workspace too small
     void *attn_static;    // this device's copy of the decode attention's static scratch (attn_decode.hip), found at creation
                           // (null if the lookup failed: only the entry point that needs it then refuses)
     unsigned *dev_status;      // one word of pinned host memory that kernels set when a bounded wait inside a launch runs
@@ -89,8 +90,8 @@ static inline int32_t gh_hip(galois_hip_ctx *ctx, hipError_t e, const char *what
 // when it fails.  What is in the workspace does not outlive a call.
 bool gh_reserve_workspace(galois_hip_ctx *ctx, size_t need);
 
-// attn_prefill.hip: the bytes galois_hip_ctx::attn_records holds.
-size_t gh_attn_records_bytes(int32_t n_cu);
+// attn_prefill.hip: the bytes of galois_hip_ctx::block (17 MB on 256 compute units).
+size_t gh_block_bytes(int32_t n_cu);
 
 // device.hip: after a wait for the stream, reports (and clears) what kernels left in the context's status word.
 int32_t gh_check_device_status(galois_hip_ctx *ctx);

@@ -72,7 +72,7 @@ int32_t galois_hip_create(int32_t ordinal, galois_hip_ctx **out) {
     ctx->ws_bytes = 0;
     ctx->scratch = nullptr;
     ctx->attn_done = nullptr;
-    ctx->attn_records = nullptr;
+    ctx->block = nullptr;
     ctx->attn_static = nullptr;
     ctx->capturing = false;
     ctx->dev_status = nullptr;
@@ -90,9 +90,9 @@ int32_t galois_hip_create(int32_t ordinal, galois_hip_ctx **out) {
     if (e == hipSuccess) e = hipMemsetAsync(ctx->scratch, 0, scratch_bytes, ctx->stream);
     if (e == hipSuccess) e = hipMalloc((void **)&ctx->attn_done, 4 * GH_ATTN_HEADS * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemsetAsync(ctx->attn_done, 0, 4 * GH_ATTN_HEADS * sizeof(unsigned), ctx->stream);
-    // made here, so that whether a prefill attention splits its keys depends on its sizes alone: not on what ran before in
-    // the context, on a capture, or on how much memory is free
-    if (e == hipSuccess) e = hipMalloc(&ctx->attn_records, gh_attn_records_bytes(ctx->n_cu));
+    // made here, so that what a call computes depends on its arguments alone: not on what ran before in the context, on a
+    // capture, or on how much memory is free
+    if (e == hipSuccess) e = hipMalloc(&ctx->block, gh_block_bytes(ctx->n_cu));
     // the status word lives in pinned host memory that the device writes directly: reading it costs the host nothing
     if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->dev_status, 64, hipHostMallocMapped);
     if (e == hipSuccess) {
@@ -105,7 +105,7 @@ int32_t galois_hip_create(int32_t ordinal, galois_hip_ctx **out) {
     if (e != hipSuccess) {
         if (ctx->scratch) (void)hipFree(ctx->scratch);
         if (ctx->attn_done) (void)hipFree(ctx->attn_done);
-        if (ctx->attn_records) (void)hipFree(ctx->attn_records);
+        if (ctx->block) (void)hipFree(ctx->block);
         if (ctx->dev_status) (void)hipHostFree(ctx->dev_status);
         (void)hipStreamDestroy(ctx->stream);
         delete ctx;
@@ -123,7 +123,7 @@ int32_t galois_hip_destroy(galois_hip_ctx *ctx) {
     for (void *p : ctx->ws_retired) (void)hipFree(p);
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->attn_done) (void)hipFree(ctx->attn_done);
-    if (ctx->attn_records) (void)hipFree(ctx->attn_records);
+    if (ctx->block) (void)hipFree(ctx->block);
     if (ctx->dev_status) (void)hipHostFree(ctx->dev_status);
     hipError_t e = hipStreamDestroy(ctx->stream);
     delete ctx;

@@ -31,9 +31,8 @@ __device__ __forceinline__ uint32_t deq_pair(uint32_t bits, half2_t d2) {
     return __builtin_bit_cast(uint32_t, (magic - off) * d2);
 }
 
-// Any K % 32 == 0, no workspace: what a product that fits neither panel kernel runs on -- a K that is no multiple of 256 (or
-// weights that are not 16-byte aligned) while a graph is captured and the workspace is still too small, or operands past
-// 32-bit panel offsets (77 x 3200 x 8640: 93 us against 19.8 us on the skinny kernel).
+// Any K % 32 == 0, no workspace: what a product whose panel would have offsets past 32 bits, or rows too long for the context's
+// fixed block, runs on.
 __global__ __launch_bounds__(256) void gemm_q4_0_mfma_v1(const uint8_t *__restrict__ W, const float *__restrict__ X,
                                                           float *__restrict__ Y, int K, int N, int M) {
     __shared__ __attribute__((aligned(16))) _Float16 As[TM * LDS_STRIDE];
@@ -881,36 +880,41 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
     const bool skinny = !wide || M <= SK_MAX_ROWS;
     const bool shares = !skinny && mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_pick_form(ctx, K, N, M, 1.1, 64.0) == GEMM_TWO_SHARES;
     const size_t need = panel_bytes + (shares ? 2 * (size_t)mn * sizeof(float) : 0);
-    bool panel = gemm_panel_shape_ok((int32_t)k_pad, M);
-    if (panel && !gh_reserve_workspace(ctx, need)) {
-        // weights that are not laid out in pieces of 256 have a kernel that needs no workspace, and run on it rather than
-        // fail while a graph is being captured (or when memory is short)
-        if (wide) {
+    // rows of a panel that fit the context's fixed block: what a product of other rows than pieces of 256 is multiplied in,
+    // chunk after chunk, when the workspace is too small and cannot grow (while a graph is captured, or out of memory).  A
+    // result does not depend on the rows around it, so the bits are the same.
+    const int64_t chunk = (int64_t)(gh_block_bytes(ctx->n_cu) / ((size_t)k_pad * sizeof(_Float16))) & ~(int64_t)15;
+    if (gemm_panel_shape_ok(k_pad, M) && (wide || chunk > 0)) {
+        int32_t st = GALOIS_HIP_OK;
+        const bool ws = gh_reserve_workspace(ctx, need);
+        if (!ws && wide) {
             GH_NOT_CAPTURING(ctx, "mul_mat_q4_0_f32: growing the workspace");
             return gh_hip(ctx, hipErrorOutOfMemory, "hipMalloc(workspace)");
         }
-        panel = false;
-    }
-    if (panel) {
-        _Float16 *Xh = (_Float16 *)ctx->ws;
-        launch_to_panel(ctx, X, nullptr, Xh, K, (int)(k_pad / 32), M, false);
+        _Float16 *Xh = (_Float16 *)(ws ? ctx->ws : ctx->block);
         if (skinny) {
-            gemm_mats mats = {};
-            mats.W[0] = (const uint8_t *)W, mats.Y[0] = Y, mats.N[0] = N;
-            gemm_concat(mats, 1);
-            const int32_t st = skinny_launch_any(ctx, mats, Xh, K, (int)(k_pad / 32), M, K % 64 == 0 && gh_aligned(W, 4));
-            if (st != GALOIS_HIP_OK) return st;
+            const int64_t step = ws ? M : chunk;
+            for (int64_t m = 0; m < M && st == GALOIS_HIP_OK; m += step) {
+                const int rows = (int)(M - m < step ? M - m : step);
+                launch_to_panel(ctx, X + m * K, nullptr, Xh, K, (int)(k_pad / 32), rows, false);
+                gemm_mats mats = {};
+                mats.W[0] = (const uint8_t *)W, mats.Y[0] = Y + m * N, mats.N[0] = N;
+                gemm_concat(mats, 1);
+                st = skinny_launch_any(ctx, mats, Xh, K, (int)(k_pad / 32), rows, K % 64 == 0 && gh_aligned(W, 4));
+            }
         } else if (shares) {
+            launch_to_panel(ctx, X, nullptr, Xh, K, K / 32, M, false);
             float *parts = reinterpret_cast<float *>(static_cast<unsigned char *>(ctx->ws) + panel_bytes);
-            const int32_t st = gemm_launch_form(ctx, W, Xh, parts, K, N, M, GEMM_TWO_SHARES);
+            st = gemm_launch_form(ctx, W, Xh, parts, K, N, M, GEMM_TWO_SHARES);
             if (st != GALOIS_HIP_OK) return st;
             hipLaunchKernelGGL(gemm_sum_pass, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, ctx->stream,
                                reinterpret_cast<const float4 *>(parts), static_cast<const float4 *>(nullptr),
                                reinterpret_cast<float4 *>(Y), mn / 4, mn / 4);
         } else {
-            const int32_t st = gemm_launch_form(ctx, W, Xh, Y, K, N, M, GEMM_WHOLE);
-            if (st != GALOIS_HIP_OK) return st;
+            launch_to_panel(ctx, X, nullptr, Xh, K, K / 32, M, false);
+            st = gemm_launch_form(ctx, W, Xh, Y, K, N, M, GEMM_WHOLE);
         }
+        if (st != GALOIS_HIP_OK) return st;
     } else {
         const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
         hipLaunchKernelGGL(gemm_q4_0_mfma_v1, grid, dim3(256), 0, ctx->stream, (const uint8_t *)W, X, Y, K, N, M);

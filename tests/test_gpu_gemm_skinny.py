@@ -85,24 +85,35 @@ def test_infinities_and_zero_scales_stay_in_their_place(dev):
         assert np.isnan(got[3, i]) if np.isnan(want) else got[3, i] == want, i
 
 
-def test_a_fresh_context_captures_a_ragged_product(dev):
-    """While a graph is captured nothing is allocated: a product whose K is no multiple of 256 then runs on the kernel
-    without a workspace."""
+@pytest.mark.parametrize("m,k,n,shift", [(40, 96, 77, 0), (1, 288, 17, 2), (3, 736, 33, 6), (16, 3200, 131, 0), (17, 8224, 96, 0), (33, 1056, 300, 2),
+                                         (150, 992, 257, 0), (130, 512, 200, 2), (65, 11008, 48, 8), (100, 262432, 33, 0), (1600, 11008, 50, 2)])
+def test_a_captured_ragged_product_has_the_eager_bits(dev, m, k, n, shift):
+    """While a graph is captured nothing is allocated: in a fresh context a product whose K is no multiple of 256, or whose weights
+    are not 16-byte aligned, is multiplied in chunks of rows through the context's fixed block (17 MB on 256 compute units: the
+    last two cases take several).  Its bits are those of the same call outside a capture, and of a capture that finds the
+    workspace large enough."""
     import galois_amd
     d2 = galois_amd.Device(0)
-    wq, x = _case(3, 40, 96, 77)
-    wb, xb, yb = d2.upload(wq), d2.upload(x), d2.alloc(40 * 77 * 4)
-    d2.graph_begin_capture()
-    d2.mul_mat_q4_0_f32(wb, xb, yb, 96, 77, 40)
-    g = d2.graph_end_capture()
-    for _ in range(3):
-        d2.upload(np.zeros(40 * 77, np.float32), yb)
-        d2.graph_launch(g)
-        emax, el2 = npref.rel_err(d2.download(yb, np.float32, (40, 77)), oracle.mul_mat_q4_0_f32(wq, x))
-        assert emax < TOL and el2 < TOL
-    d2.graph_destroy(g)
-    for b in (wb, xb, yb):
-        d2.free(b)
+    wq, x = _case(m + k + n, m, k, n)
+    want = _run(dev, wq, x, shift)
+    emax, el2 = npref.rel_err(want, oracle.mul_mat_q4_0_f32(wq, x))
+    assert emax < TOL and el2 < TOL
+    raw = np.zeros(wq.nbytes + 16, np.uint8)
+    raw[shift:shift + wq.nbytes] = wq.reshape(-1)
+    wb, xb, yb = d2.upload(raw), d2.upload(x), d2.alloc((m * n + 64) * 4)
+    for warm in (False, True):
+        if warm:
+            d2.mul_mat_q4_0_f32(wb.view(shift), xb, yb, k, n, m)
+        d2.graph_begin_capture()
+        d2.mul_mat_q4_0_f32(wb.view(shift), xb, yb, k, n, m)
+        g = d2.graph_end_capture()
+        for _ in range(3):
+            d2.upload(np.full(m * n + 64, 7.5, np.float32), yb)
+            d2.graph_launch(g)
+            got = d2.download(yb, np.float32, m * n + 64)
+            assert np.array_equal(got[:m * n].view(np.uint32), want.reshape(-1).view(np.uint32)), warm
+            assert np.all(got[m * n:] == 7.5)
+        d2.graph_destroy(g)
     d2.close()
 
 
