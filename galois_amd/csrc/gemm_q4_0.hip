@@ -31,8 +31,8 @@ __device__ __forceinline__ uint32_t deq_pair(uint32_t bits, half2_t d2) {
     return __builtin_bit_cast(uint32_t, (magic - off) * d2);
 }
 
-// Any K % 32 == 0, no workspace: what a product whose panel would have offsets past 32 bits, or rows too long for the context's
-// fixed block, runs on.
+// Any K % 32 == 0, no workspace: short rows and many tiles of ragged rows (gemm_v1_pays), and what has no panel: offsets past 32
+// bits, or rows too long for the context's fixed block.
 __global__ __launch_bounds__(256) void gemm_q4_0_mfma_v1(const uint8_t *__restrict__ W, const float *__restrict__ X,
                                                           float *__restrict__ Y, int K, int N, int M) {
     __shared__ __attribute__((aligned(16))) _Float16 As[TM * LDS_STRIDE];
@@ -850,6 +850,29 @@ gemm_form gemm_pick_form(const galois_hip_ctx *ctx, int K, int N, int M, double 
     return shares ? GEMM_TWO_SHARES : GEMM_WHOLE;
 }
 
+// Whether a product that the wide kernel does not take (K no multiple of 256, W not 16-byte aligned) is better off on
+// gemm_q4_0_mfma_v1 than on the skinny kernel.  That one converts X in a launch of its own, gives every fourth piece of 256 k to a
+// wave and re-reads the panel per 64 columns, so it loses where rows are short (one piece keeps one wave of four busy) and
+// where there are enough 128 x 128 tiles to fill the device more than twice; v1 pays 0.82 us per 32 k however few tiles
+// it has.  Both sides in us, fitted to 1953 sizes (K 32 .. 11008, N 100 .. 32000, 1 .. 4096 rows, within 12 %).  Measured, us,
+// v1 / skinny: 3 x 96 x 16000 4.7 / 6.2, 1024 x 96 x 16000 15.7 / 45.5, 1024 x 288 x 4000 13 / 21, 2048 x 1056 x 4000 40 / 60, 4096 x
+// 3200 x 8640 455 / 514; the other way 3 x 288 x 4000 8.5 / 7.2, 1024 x 1056 x 4000 37 / 32, 2048 x 3200 x 8640 247 / 241.
+// Few rows of 288 or more never gain on v1 and are not worth the arithmetic; t receives the skinny kernel's tiles if they were
+// looked for.
+bool gemm_v1_pays(const galois_hip_ctx *ctx, int K, int N, int M, sk_tiles &t) {
+    if (K <= 192) return true;
+    if (M <= SK_MAX_ROWS && K >= 288 && N < 1 << 24) return false;
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
+    const double tiles = (double)(((int64_t)N + TN - 1) / TN * (((int64_t)M + TM - 1) / TM)) / (double)cus, mn = (double)M * N * 1e-6;
+    t = skinny_pick(ctx, N, M, false);
+    const int64_t m_blocks = (((int64_t)M + 15) / 16 + t.mt - 1) / t.mt, n_tiles = ((int64_t)N + 16 * t.nt - 1) / (16 * t.nt);
+    if ((n_tiles + 8) * m_blocks >= (int64_t)1 << 23) return true;  // a launch holds fewer than 2^32 threads
+    const double far = m_blocks > 16 ? (m_blocks < 32 ? (m_blocks - 16) / 16.0 : 1.0) : 0.0;  // row blocks past what shares a panel in L2
+    const double v1 = 2.7 + (K / 32) * (0.52 * tiles > 0.82 ? 0.52 * tiles : 0.82) + 0.51 * mn;
+    const double skinny = 6.2 + 1.63e-6 * M * K + 0.92 * t.cost * (K + 318.0) / 4096.0 * (1.0 + 0.28 * far) + 0.97 * mn;
+    return v1 < skinny;
+}
+
 // W . panel into dst as one result or as two partial results M * N floats apart.
 int32_t gemm_launch_form(galois_hip_ctx *ctx, const void *W, const _Float16 *panel, float *dst, int K, int N, int M, gemm_form form) {
     gemm_mats mats = {};
@@ -884,7 +907,8 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
     // chunk after chunk, when the workspace is too small and cannot grow (while a graph is captured, or out of memory).  A
     // result does not depend on the rows around it, so the bits are the same.
     const int64_t chunk = (int64_t)(gh_block_bytes(ctx->n_cu) / ((size_t)k_pad * sizeof(_Float16))) & ~(int64_t)15;
-    if (gemm_panel_shape_ok(k_pad, M) && (wide || chunk > 0)) {
+    sk_tiles tiles = {0, 0, 0.0};
+    if (gemm_panel_shape_ok(k_pad, M) && (wide || (chunk > 0 && !gemm_v1_pays(ctx, K, N, M, tiles)))) {
         int32_t st = GALOIS_HIP_OK;
         const bool ws = gh_reserve_workspace(ctx, need);
         if (!ws && wide) {
@@ -900,7 +924,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
                 gemm_mats mats = {};
                 mats.W[0] = (const uint8_t *)W, mats.Y[0] = Y + m * N, mats.N[0] = N;
                 gemm_concat(mats, 1);
-                st = skinny_launch_any(ctx, mats, Xh, K, (int)(k_pad / 32), rows, K % 64 == 0 && gh_aligned(W, 4));
+                st = skinny_launch_any(ctx, mats, Xh, K, (int)(k_pad / 32), rows, K % 64 == 0 && gh_aligned(W, 4), tiles);
             }
         } else if (shares) {
             launch_to_panel(ctx, X, nullptr, Xh, K, K / 32, M, false);

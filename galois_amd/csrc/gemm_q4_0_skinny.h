@@ -325,10 +325,11 @@ inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int M, bool
 }
 inline double skinny_us(const galois_hip_ctx *ctx, int N, int K, int M) { return skinny_pick(ctx, N, M, false).cost * K / 4096.0; }
 
-// KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.
-int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned) {
+// KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.  t: tiles the caller has picked.
+int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned,
+                          sk_tiles t = {0, 0, 0.0}) {
     const bool swiglu = mats.swiglu_out != nullptr;
-    const sk_tiles t = skinny_pick(ctx, swiglu ? 2 * (int64_t)mats.N[0] : mats.n_total, M, swiglu);
+    if (t.nt == 0) t = skinny_pick(ctx, swiglu ? 2 * (int64_t)mats.N[0] : mats.n_total, M, swiglu);
     if (K >= 8192)
         return aligned ? skinny_launch_tiles<8, true>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
                        : skinny_launch_tiles<8, false>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt);

@@ -195,10 +195,11 @@ int32_t galois_hip_dequantize_mul_mat_vec_q4_0_group(galois_hip_ctx *ctx, const 
  * (output layout of matmul.cu:359).  W tiles are dequantised to fp16 in LDS, X is
  * rounded to fp16, products accumulate in f32 on MFMA.  K % 32 == 0.  No Q8_1
  * scratch and no K padding (src/cuda.rs:1040-1068) are needed from the caller.  Few rows (up to 80), and a K that is
- * no multiple of 256 or a W that is not 16-byte aligned, run on a kernel that dequantises in registers.  The fp16 copy of X lives in a workspace the context
- * owns and grows on demand (the call allocates when a larger one is needed; refused during a graph capture, except
- * for such K and W, which then go through a block the context made at creation, a few hundred rows at a time, with the
- * same bits).  A large
+ * no multiple of 256 or a W that is not 16-byte aligned, run on a kernel that dequantises in registers; short rows
+ * of such K (up to 192), and so many results that they fill the device anyway, on one that needs no workspace.  The fp16
+ * copy of X lives in a workspace the context owns and grows on demand (the call allocates when a larger one is needed;
+ * refused during a graph capture, except for such K and W, which then go, where they need one, through a block the
+ * context made at creation, a few hundred rows at a time, with the same bits).  A large
  * product whose N leaves compute units idle (512 x 11008 x 4096 on 256 CUs) is computed as two shares of k that a
  * second launch adds: the f32 sums over k are then two chains instead of one, for the same operands on the same
  * device always the same way. */

@@ -85,6 +85,18 @@ def test_infinities_and_zero_scales_stay_in_their_place(dev):
         assert np.isnan(got[3, i]) if np.isnan(want) else got[3, i] == want, i
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 32, 130), (129, 160, 257), (300, 96, 385), (257, 192, 129), (1100, 288, 4000), (4097, 544, 3001)])
+def test_short_rows_and_many_tiles(dev, m, k, n):
+    """The sizes that run without a panel (gemm_v1_pays): remainders of its 128 x 128 tiles, weight rows at every 2-byte offset."""
+    wq, x = _case(m + k + n, m, k, n)
+    got = _run(dev, wq, x)
+    cols = np.unique(np.concatenate([[0, n - 1], np.random.default_rng(n).choice(n, min(n, 96), replace=False)]))
+    emax, el2 = npref.rel_err(got[:, cols], oracle.mul_mat_q4_0_f32(wq[cols], x))
+    assert emax < TOL and el2 < TOL, (emax, el2)
+    for shift in (2, 6, 8):
+        assert np.array_equal(_run(dev, wq, x, shift).view(np.uint32), got.view(np.uint32)), shift
+
+
 @pytest.mark.parametrize("m,k,n,shift", [(40, 96, 77, 0), (1, 288, 17, 2), (3, 736, 33, 6), (16, 3200, 131, 0), (17, 8224, 96, 0), (33, 1056, 300, 2),
                                          (150, 992, 257, 0), (130, 512, 200, 2), (65, 11008, 48, 8), (100, 262432, 33, 0), (1600, 11008, 50, 2)])
 def test_a_captured_ragged_product_has_the_eager_bits(dev, m, k, n, shift):
