@@ -766,16 +766,17 @@ namespace {
 struct gemm_tile {
     int gn, rt;
     double cost;  // rounds x relative cost of a stage
+    int64_t wgs;
 };
 gemm_tile gemm_pick(const galois_hip_ctx *ctx, int64_t cols, int64_t M, int gn, int splits = 1) {
     const double stage96[3] = {0.70, 0.86, 1.0}, stage64[3] = {0.50, 0.60, 0.75}, stage48[3] = {0.44, 0.53, 0.65};
     const double *stage = gn == 96 ? stage96 : gn == 64 ? stage64 : stage48;
     const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
-    gemm_tile best = {gn, 4, 0.0};
+    gemm_tile best = {gn, 4, 0.0, 0};
     for (int rt = 4; rt >= 2; rt--) {
         const int64_t wgs = (cols + gn - 1) / gn * ((M + 64 * rt - 1) / (64 * rt)) * splits;
         const double cost = (double)((wgs + cus - 1) / cus) * stage[rt - 2];
-        if (rt == 4 || cost < best.cost) best = {gn, rt, cost};
+        if (rt == 4 || cost < best.cost) best = {gn, rt, cost, wgs};
     }
     return best;
 }
@@ -834,19 +835,33 @@ namespace {
 // 11008 -> 4096 at 150 rows 27.3 us against 57 us whole and 39 us in shares).  The cost model of gemm_pick (rounds of
 // workgroups x cost of a stage x stages) plus the pass that adds the two partial results, which costs about fourteen stages
 // per 2^21 results.  Measured at M = 512 on 256 CUs: 11008 -> 4096 70.3 -> 54.8 us, 4096 -> 4096 32.5 -> 30.2 us (both
-// with the residual); the shapes the model leaves whole are slower when forced into shares.  margin > 1 asks for a clearer
-// win (where the adding pass replaces nothing the caller would launch anyway), min_cost for a product large enough that the
-// model's neglect of fixed costs does not matter.
+// with the residual); the shapes the model leaves whole are slower when forced into shares.  plain: the adding pass
+// replaces nothing the caller would launch anyway, and the result is to be that of whole tiles unless the product is large:
+// no skinny kernel, and shares only from 64 stages of a 256 x 96 tile on (512 x 13824 x 2816 55 us against 64 whole, 100 x 8192 x
+// 1000 24 against 38).
 enum gemm_form { GEMM_WHOLE, GEMM_TWO_SHARES, GEMM_SKINNY };
-gemm_form gemm_pick_form(const galois_hip_ctx *ctx, int K, int N, int M, double margin = 1.0, double min_cost = 0.0) {
+gemm_form gemm_pick_form(const galois_hip_ctx *ctx, int K, int N, int M, bool plain = false) {
     if (M <= SK_MAX_ROWS) return GEMM_WHOLE;  // on the skinny kernel
     const double stages = K / 64;
     const int64_t mn = (int64_t)M * N;
     const double c96 = gemm_pick(ctx, N, M, 96).cost * stages, c48 = gemm_pick(ctx, N, M, 48).cost * stages;
     const double whole = c96 < c48 ? c96 : c48;
-    const double c64x2 = gemm_pick(ctx, N, M, 64, 2).cost * (K / 128 + 2) + 14.0 * (double)mn / (double)(1 << 21);
-    const bool shares = K >= 512 && mn % 4 == 0 && margin * c64x2 < whole && whole >= min_cost;
-    if (margin == 1.0 && skinny_us(ctx, N, K, M) < 0.64 * (shares ? c64x2 : whole)) return GEMM_SKINNY;
+    const gemm_tile t64 = gemm_pick(ctx, N, M, 64, 2);
+    const double c64x2 = t64.cost * (K / 128 + 2) + 14.0 * (double)mn / (double)(1 << 21);
+    bool large = true;
+    double clear = 1.0;
+    if (plain) {
+        // large: in terms of 256-row tiles, as a lower tile is no reason to leave the shares, which come in lower tiles too
+        const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, m256 = ((int64_t)M + 255) / 256;
+        const double r96 = (double)((((int64_t)N + 95) / 96 * m256 + cus - 1) / cus);
+        const double r48 = (double)((((int64_t)N + 47) / 48 * m256 + cus - 1) / cus);
+        large = (r96 < 0.65 * r48 ? r96 : 0.65 * r48) * stages >= 64.0;
+        // a launch that leaves CUs free runs its stages faster than the model has it (512 x 8192 x 2816: 176 workgroups, 40 us
+        // against 43 whole), several full rounds slower (1024 x 8192 x 4096: 90 against 82)
+        clear = 4 * t64.wgs <= 3 * cus ? 0.9 : 1.04;
+    }
+    const bool shares = K >= 512 && mn % 4 == 0 && clear * c64x2 < whole && large;
+    if (!plain && skinny_us(ctx, N, K, M) < 0.64 * (shares ? c64x2 : whole)) return GEMM_SKINNY;
     return shares ? GEMM_TWO_SHARES : GEMM_WHOLE;
 }
 
@@ -901,7 +916,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
     const size_t panel_bytes = ((size_t)m_pad * k_pad * sizeof(_Float16) + 255) & ~(size_t)255;
     const bool wide = K == k_pad && gh_aligned(W, 16);  // what the 256-row kernel asks of the weights
     const bool skinny = !wide || M <= SK_MAX_ROWS;
-    const bool shares = !skinny && mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_pick_form(ctx, K, N, M, 1.1, 64.0) == GEMM_TWO_SHARES;
+    const bool shares = !skinny && mn < ((int64_t)1 << 31) && gh_aligned(Y, 16) && gemm_pick_form(ctx, K, N, M, true) == GEMM_TWO_SHARES;
     const size_t need = panel_bytes + (shares ? 2 * (size_t)mn * sizeof(float) : 0);
     // rows of a panel that fit the context's fixed block: what a product of other rows than pieces of 256 is multiplied in,
     // chunk after chunk, when the workspace is too small and cannot grow (while a graph is captured, or out of memory).  A

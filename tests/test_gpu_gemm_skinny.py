@@ -187,6 +187,25 @@ def test_forms_of_a_narrow_product(dev, m, k, n):
         dev.free(b)
 
 
+@pytest.mark.parametrize("m,k,n", [(81, 8192, 1000), (129, 6400, 48), (200, 8192, 257 * 4), (512, 8192, 2816), (260, 11008, 1536)])
+def test_a_large_narrow_product_from_f32_rows(dev, m, k, n):
+    """The f32 entry point multiplies these as two shares of k in tiles of 128, 192 or 256 rows: against the oracle on a sample, and
+    against the plain panel call, whose sums are one chain (1e-5 of the largest result)."""
+    wq, x = _case(m + 2 * n, m, k, n)
+    got = _run(dev, wq, x)
+    cols = np.unique(np.concatenate([[0, n - 1], np.random.default_rng(n).choice(n, min(n, 96), replace=False)]))
+    emax, el2 = npref.rel_err(got[:, cols], oracle.mul_mat_q4_0_f32(wq[cols], x))
+    assert emax < TOL and el2 < TOL, (emax, el2)
+    wb, xb, pb, y = dev.upload(wq), dev.upload(x), dev.alloc(dev.f16_panel_bytes(k, m)), dev.alloc(m * n * 4)
+    dev.f32_to_f16_panel(xb, pb, k, m)
+    dev.mul_mat_q4_0_f16_panel([(wb, y, n)], pb, k, m)
+    whole = dev.download(y, np.float32, (m, n))
+    assert np.max(np.abs(got - whole)) <= 1e-5 * np.max(np.abs(whole))
+    assert not np.array_equal(got, whole), "one chain: the call did not come in shares"
+    for b in (wb, xb, pb, y):
+        dev.free(b)
+
+
 @pytest.mark.parametrize("m", [81, 128, 129, 192, 193, 260])
 def test_swiglu_row_tiles(dev, m):
     k, n = 1024, 2816
