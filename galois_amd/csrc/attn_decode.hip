@@ -84,7 +84,8 @@ int32_t attn_decode_launch(galois_hip_ctx *ctx, const float *q, const float *k, 
     // while there are few workgroups more waves each do less: eight waves of 16 keys, or of 8 keys where even splits of 64
     // keys leave CUs free.  A merge costs 2 us, so a head of 64 up to 256 keys long stays whole (its rows are half as
     // long), and so do longer pieces of it once more than sixteen splits would have to be merged.  Beyond two workgroups
-    // per CU four waves a workgroup are better: more of them are resident.  Measured, us, 128 keys x 256 threads against the
+    // per CU four waves a workgroup are better: more of them are resident; so they are beyond 32 splits, whose merge takes the
+    // general path (8 heads, 8000 f32 keys 27.2 with eight waves against 24.7).  Measured, us, 128 keys x 256 threads against the
     // choice here: 32 heads of 128, 90 keys 6.8 -> 6.1, 203 9.0 -> 7.5, 512 10.1 -> 8.8, 1024 13.8 -> 12.1, 2048 19.7 ->
     // 18.3 (f16 7.2 -> 6.2, 9.4 -> 7.6, 9.4 -> 8.4, 10.9 -> 10.2, 15.2 -> 14.4); 4000 keys with eight waves 42.9 against 33.7;
     // 16 heads of 64, 203 keys 7.2 -> 6.1, 4000 15.8 -> 12.8.
@@ -95,7 +96,7 @@ int32_t attn_decode_launch(galois_hip_ctx *ctx, const float *q, const float *k, 
                        theta_scale, scale, key_stride, head_stride)
     if (head_dim == 128) {
         if (L > 128 && s64 <= 16 && n_head * s64 <= cus) AT_LAUNCH(32, 64, 512);
-        else if ((int64_t)n_head * S <= 2 * cus) AT_LAUNCH(32, 128, 512);
+        else if ((int64_t)n_head * S <= 2 * cus && S <= 32) AT_LAUNCH(32, 128, 512);
         else AT_LAUNCH(32, 128, 256);
     } else {
         if ((L > 128 && L <= 256) || S > 16) AT_LAUNCH(16, 256, 512);
