@@ -82,7 +82,7 @@ class Device:
             self._lib.galois_hip_destroy(self._ctx)
             self._ctx = None
 
-    OPT_GEMV_F32_ARITHMETIC, OPT_WAIT_SPIN_LIMIT, OPT_WAIT_TARGET_BIAS = 1, 2, 3
+    OPT_GEMV_F32_ARITHMETIC, OPT_WAIT_SPIN_LIMIT, OPT_WAIT_TARGET_BIAS, OPT_QKV_ATTN_LAUNCHES = 1, 2, 3, 4
 
     def set_option(self, option, value):
         self._check(self._lib.galois_hip_set_option(self._ctx, option, value))
@@ -274,11 +274,17 @@ class Device:
 
     def qkv_attn_decode(self, items, k_cache, v_cache, out, n_head, head_dim, n_past, pos, freq_scale, theta_scale, scale,
                         kv_f16=False, head_major_n_ctx=0):
-        """The three q | k | v products (gemv_items of length 3) and the decode attention in one launch."""
+        """The three q | k | v products (gemv_items of length 3) and the decode attention in one call (one launch or two)."""
         arr = items if isinstance(items, C.Array) else self.gemv_items(items)
         fn = self._lib.galois_hip_qkv_attn_decode_f16kv if kv_f16 else self._lib.galois_hip_qkv_attn_decode_f32
         self._check(fn(self._ctx, arr, _ptr(k_cache), _ptr(v_cache), _ptr(out), n_head, head_dim, n_past, _ptr(pos),
                        freq_scale, theta_scale, scale, head_major_n_ctx))
+
+    def qkv_attn_decode_launches(self, n_head, n_past, kv_f16=False):
+        """How many launches qkv_attn_decode issues for these sizes: 1 or 2."""
+        n = C.c_int32(0)
+        self._check(self._lib.galois_hip_qkv_attn_decode_launches(self._ctx, n_head, n_past, int(kv_f16), C.byref(n)))
+        return n.value
 
     def mul_mat_q4_0_f16_panel_add(self, W, panel, residual, Y, K, N, M, workspace=None, workspace_bytes=0):
         """Y = residual + W . panel (residual may be None); with a workspace of 2 * M * N floats a matrix too narrow

@@ -27,6 +27,7 @@ struct galois_hip_ctx {
     unsigned *dev_status_dev;  // out (the device's address of the same word); read and cleared after every stream wait
     int32_t wait_spin_limit;   // polls a bounded in-launch wait makes before it gives up (GALOIS_HIP_OPT_WAIT_SPIN_LIMIT)
     int32_t wait_target_bias;  // added to the count such a wait waits for: test hook (GALOIS_HIP_OPT_WAIT_TARGET_BIAS)
+    int32_t qkv_attn_launches; // 1 or 2: the form of qkv_attn_decode whatever the sizes (GALOIS_HIP_OPT_QKV_ATTN_LAUNCHES)
     bool gemv_f32;             // GALOIS_HIP_OPT_GEMV_F32_ARITHMETIC: one-product GEMV in the reference's f32 arithmetic
     bool capturing;   // between graph_begin_capture and graph_end_capture: nothing may allocate or block
     char last_error[256];

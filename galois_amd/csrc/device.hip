@@ -79,6 +79,7 @@ int32_t galois_hip_create(int32_t ordinal, galois_hip_ctx **out) {
     ctx->dev_status_dev = nullptr;
     ctx->wait_spin_limit = GH_WAIT_SPIN_DEFAULT;
     ctx->wait_target_bias = 0;
+    ctx->qkv_attn_launches = 0;
     ctx->gemv_f32 = false;
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
@@ -145,6 +146,10 @@ int32_t galois_hip_set_option(galois_hip_ctx *ctx, int32_t option, int32_t value
         case GALOIS_HIP_OPT_WAIT_TARGET_BIAS:
             GH_REQUIRE(ctx, value >= 0 && value <= 1, GALOIS_HIP_E_SHAPE, "set_option: the target bias is 0 or 1");
             ctx->wait_target_bias = value;
+            return GALOIS_HIP_OK;
+        case GALOIS_HIP_OPT_QKV_ATTN_LAUNCHES:
+            GH_REQUIRE(ctx, value >= 0 && value <= 2, GALOIS_HIP_E_SHAPE, "set_option: one launch, two, or 0 for by size");
+            ctx->qkv_attn_launches = value;
             return GALOIS_HIP_OK;
         default:
             return gh_fail(ctx, GALOIS_HIP_E_UNSUPPORTED, "set_option: unknown option");

@@ -913,7 +913,7 @@ int32_t launch_group(galois_hip_ctx *ctx, const galois_hip_gemv_item *items, int
 }
 
 // ---------------------------------------------------------------------------------------
-// The q | k | v products and the decode attention in one launch (launch_qkv_attn: where that pays).
+// The q | k | v products and the decode attention in one launch (fa_one_launch: where).
 //
 // Issued as two launches the attention starts when the last product row is out, pays a launch gap, and then spends
 // its first microseconds requesting the cache; its own end is a chain of dependent round trips (split records,
@@ -963,6 +963,19 @@ __global__ __launch_bounds__(FA_WAVES * 64, 4) void qkv_attn_decode_fused(const 
     }
 }
 
+// One launch pays when there is much of both to overlap: nine product workgroups or more per four CUs (the attention's
+// registers leave room for two at a time instead of four, so few products gain nothing from being ahead) and a cache
+// that takes longer to fetch than what the fused kernel adds.  Per layer of a decode step, us as two launches / one:
+// 4096 wide, f32 cache, 200 keys 45.0 / 48.7, 800 47.8 / 57.6, 1600 (52 MB) 52.3 / 51.8, 2047 55.2 / 52.6, 4000 70.2 /
+// 63.6; f16 cache 200 45.0 / 53.2, 1200 48.0 / 51.2, 2500 (41 MB) 52.9 / 52.4, 4000 62.0 / 58.7.
+bool fa_one_launch(const galois_hip_ctx *ctx, int64_t n_head, int64_t n_past, bool f16) {
+    // what the attention by itself refuses, and a wait that is biased from outside (a test of the waits), keep the one launch
+    if (n_head > 65535 || ctx->wait_target_bias != 0) return true;
+    if (ctx->qkv_attn_launches) return ctx->qkv_attn_launches == 1;
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, L = n_past + 1;
+    return 4 * 3 * n_head * (FA_HEAD_DIM / (FA_WAVES * FA_R)) >= 9 * cus && 2 * L * n_head * FA_HEAD_DIM * (f16 ? 2 : 4) >= (int64_t)38 << 20;
+}
+
 template <typename CT>
 int32_t launch_qkv_attn(galois_hip_ctx *ctx, const galois_hip_gemv_item *items, CT *k_cache, CT *v_cache, float *out,
                         int32_t n_head, int32_t head_dim, int32_t n_past, const int32_t *pos, float freq_scale,
@@ -997,15 +1010,7 @@ int32_t launch_qkv_attn(galois_hip_ctx *ctx, const galois_hip_gemv_item *items, 
                GALOIS_HIP_E_UNSUPPORTED, "qkv_attn_decode: n_head * ceil((n_past + 1) / 128) * (head_dim + 4) floats of partial "
                                          "results must fit the context's 4 MB scratch block");
     GH_REQUIRE(ctx, plan.blocks + (int64_t)n_head * S < 0x7FFFFFFF, GALOIS_HIP_E_SHAPE, "qkv_attn_decode: too many workgroups");
-    // One launch pays when there is much of both to overlap: three or more product workgroups per CU (the attention's
-    // registers leave room for two at a time instead of four, so few products gain nothing from being ahead) and a cache
-    // that takes longer to fetch than what the fused kernel adds.  Per layer of a decode step, us as two launches / one:
-    // 4096 wide, f32 cache, 200 keys 45.0 / 48.7, 800 47.8 / 57.6, 1600 (52 MB) 52.3 / 51.8, 2047 55.2 / 52.6, 4000 70.2 /
-    // 63.6; f16 cache 200 45.0 / 53.2, 1200 48.0 / 51.2, 2500 (41 MB) 52.9 / 52.4, 4000 62.0 / 58.7; 3072 wide, f32, 1200
-    // (29 MB) 40.9 / 43.7, 1600 (39 MB) 43.5 / 42.6; 2048 and 1024 wide two launches at every length (4000 keys 43.5 / 53.4 and
-    // 34.7 / 47.0).  A wait that is biased from outside (a test of the waits) keeps the launch that has them.
-    const int64_t cache_bytes = 2 * (int64_t)L * n_head * head_dim * (int64_t)sizeof(CT), cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
-    if ((cache_bytes < ((int64_t)38 << 20) || 4 * plan.blocks < 9 * cus) && n_head <= 65535 && ctx->wait_target_bias == 0) {
+    if (!fa_one_launch(ctx, n_head, n_past, sizeof(CT) == 2)) {
         const int32_t sg = launch_group(ctx, items, 3, what);
         if (sg != GALOIS_HIP_OK) return sg;
         if (sizeof(CT) == 2)
@@ -1079,6 +1084,16 @@ extern "C" int32_t galois_hip_dequantize_mul_mat_vec_q4_0_group(galois_hip_ctx *
                                                                 int32_t n_items) {
     GH_REQUIRE_CTX(ctx);
     return launch_group(ctx, items, n_items, "dequantize_mul_mat_vec_q4_0_group");
+}
+
+extern "C" int32_t galois_hip_qkv_attn_decode_launches(galois_hip_ctx *ctx, int32_t n_head, int32_t n_past, int32_t kv_f16,
+                                                       int32_t *n_launches) {
+    GH_REQUIRE_CTX(ctx);
+    GH_REQUIRE(ctx, n_launches != nullptr, GALOIS_HIP_E_NULL, "qkv_attn_decode_launches");
+    GH_REQUIRE(ctx, n_head > 0 && n_head <= GH_ATTN_HEADS && n_past >= 0 && n_past < 0x7FFFFF00, GALOIS_HIP_E_SHAPE,
+               "qkv_attn_decode_launches: n_head in 1..65536, n_past >= 0");
+    *n_launches = fa_one_launch(ctx, n_head, n_past, kv_f16 != 0) ? 1 : 2;
+    return GALOIS_HIP_OK;
 }
 
 extern "C" int32_t galois_hip_qkv_attn_decode_f32(galois_hip_ctx *ctx, const galois_hip_gemv_item *qkv, float *k_cache,

@@ -74,10 +74,13 @@ int32_t galois_hip_init_functions(galois_hip_ctx *ctx, int32_t abi_version, int3
  *   WAIT_SPIN_LIMIT (polls; 0 restores the default of 2^20, about a second) and WAIT_TARGET_BIAS (0 / 1): the bound
  *     of the waits inside galois_hip_qkv_attn_decode_* and an offset added to the count they wait for.  For tests of
  *     the give-up path only: with bias 1 every wait runs out, every kernel still ends normally, the call's output is
- *     NaN and the next synchronize returns GALOIS_HIP_E_DEVICE_WAIT. */
+ *     NaN and the next synchronize returns GALOIS_HIP_E_DEVICE_WAIT.
+ *   QKV_ATTN_LAUNCHES (0, 1, 2; default 0): galois_hip_qkv_attn_decode_* as one launch or as two whatever the sizes; 0 leaves
+ *     it to them.  The results differ by rounding only.  (Heads or a bias that one form cannot serve keep the other.) */
 #define GALOIS_HIP_OPT_GEMV_F32_ARITHMETIC 1
 #define GALOIS_HIP_OPT_WAIT_SPIN_LIMIT 2
 #define GALOIS_HIP_OPT_WAIT_TARGET_BIAS 3
+#define GALOIS_HIP_OPT_QKV_ATTN_LAUNCHES 4
 int32_t galois_hip_set_option(galois_hip_ctx *ctx, int32_t option, int32_t value);
 /* Text of the last non-zero status on this context ("" if none); never NULL. */
 const char *galois_hip_last_error(const galois_hip_ctx *ctx);
@@ -351,8 +354,9 @@ int32_t galois_hip_attn_decode_f16kv(galois_hip_ctx *ctx, const float *q, const 
  * normalisation galois_hip_dequantize_mul_mat_vec_q4_0_group folds in) and the attention that consumes them
  * (galois_hip_attn_decode_f32 / _f16kv above) as one call: qkv[0..2] are the three products, whose dst are the
  * q, k and v vectors of n_head * head_dim floats (written as by the group call, and read by the attention part).
- * Where there is enough of both to overlap (a cache of 38 MB or more up to n_past, nine product workgroups or more
- * per four compute units) the call is ONE launch, otherwise the two launches of those calls.  In one launch the
+ * Where there is enough of both to overlap (a cache of 38 MiB or more up to n_past, nine product workgroups or more
+ * per four compute units) the call is ONE launch, otherwise the two launches of those calls;
+ * GALOIS_HIP_OPT_QKV_ATTN_LAUNCHES overrides it.  In one launch the
  * attention's workgroups follow the products' in the grid, request their cache rows while the last products
  * still stream, and wait -- bounded -- only for their own head's rows of q (k and v where position n_past lives);
  * should a wait ever run out, that head's whole output is NaN, the context's status word is set and the next synchronize
@@ -366,6 +370,8 @@ int32_t galois_hip_qkv_attn_decode_f32(galois_hip_ctx *ctx, const galois_hip_gem
 int32_t galois_hip_qkv_attn_decode_f16kv(galois_hip_ctx *ctx, const galois_hip_gemv_item *qkv, void *k_cache,
                                          void *v_cache, float *out, int32_t n_head, int32_t head_dim, int32_t n_past,
                                          const int32_t *pos, float freq_scale, float theta_scale, float scale, int32_t head_major_n_ctx);
+/* How many launches such a call issues on this context (1 or 2): for these sizes, or as the option says. */
+int32_t galois_hip_qkv_attn_decode_launches(galois_hip_ctx *ctx, int32_t n_head, int32_t n_past, int32_t kv_f16, int32_t *n_launches);
 
 /* One Q4_0 matrix against the panel with the residual stream added: Y = residual + W . panel (residual may be null),
  * Y and residual [M][N] f32 -- an output or down projection and the add that follows it (CudaMatMul then add_f32,

@@ -1,6 +1,7 @@
 """The launch that carries the q | k | v products and the decode attention together against the same two calls issued
-one after the other.  q, k, v and the appended cache rows are bit-equal whenever the products' own call runs the same
-workgroup shape (8 waves x 2 rows); with few rows it runs 16 waves x 1 row, which adds up a normalising product's
+one after the other, at every size by asking for it (OPT_QKV_ATTN_LAUNCHES = 1) and in whichever form the call takes by
+itself (0: at the small sizes here the two launches); and which form that is on either side of its lines.  q, k, v
+and the appended cache rows are bit-equal whenever the products' own call runs the same workgroup shape (8 waves x 2 rows); with few rows it runs 16 waves x 1 row, which adds up a normalising product's
 sum of squares in another order, so there the bar is 2e-6 of the largest element.  The attention's output agrees up to
 the order of its f32 sums (eight waves instead of four share a split's keys): 1e-5 of the largest output, the
 tolerance of the attention's own parity test."""
@@ -10,6 +11,13 @@ import pytest
 import oracle
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(params=[1, 0], ids=["one_launch", "by_size"])
+def form(request, dev):
+    dev.set_option(dev.OPT_QKV_ATTN_LAUNCHES, request.param)
+    yield request.param
+    dev.set_option(dev.OPT_QKV_ATTN_LAUNCHES, 0)
 
 
 def _case(dev, H, K, n_past, mode, kv_f16, seed, repeats=1, n_ctx=None):
@@ -69,13 +77,15 @@ def _case(dev, H, K, n_past, mode, kv_f16, seed, repeats=1, n_ctx=None):
 @pytest.mark.parametrize("H,K,n_past,mode,kv_f16", [
     (2, 256, 0, 0, False), (2, 256, 5, 1, False), (3, 320, 130, 2, False), (4, 256, 127, 1, True),
     (2, 5120, 300, 1, False), (2, 4160, 300, 2, True), (2, 4160, 40, 0, False), (2, 11776, 70, 1, False),
-    (32, 4096, 2047, 2, False), (32, 4096, 2047, 1, False), (32, 4096, 2047, 2, True), (32, 4096, 2300, 0, False)])
-def test_qkv_attn_equals_the_two_calls(dev, H, K, n_past, mode, kv_f16):
+    (32, 4096, 2047, 2, False), (32, 4096, 2047, 1, False), (32, 4096, 2047, 2, True), (32, 4096, 2300, 0, False),
+    (32, 4096, 2600, 1, True), (40, 5120, 1100, 2, False), (40, 5120, 1700, 1, True), (24, 11776, 2100, 0, True)])
+def test_qkv_attn_equals_the_two_calls(dev, form, H, K, n_past, mode, kv_f16):
     _case(dev, H, K, n_past, mode, kv_f16, seed=H * 1000 + n_past)
 
 
-@pytest.mark.parametrize("H,K,n_past,n_ctx,kv_f16", [(32, 4096, 2047, 2048, False), (3, 256, 130, 200, True)])
-def test_qkv_attn_with_head_major_caches(dev, H, K, n_past, n_ctx, kv_f16):
+@pytest.mark.parametrize("H,K,n_past,n_ctx,kv_f16", [(32, 4096, 2047, 2048, False), (3, 256, 130, 200, True),
+                                                      (32, 4096, 2500, 2600, True)])
+def test_qkv_attn_with_head_major_caches(dev, form, H, K, n_past, n_ctx, kv_f16):
     """The same launch over caches kept [n_head][n_ctx][head_dim]: outputs and cache contents bit-equal."""
     D = 128
     E = H * D
@@ -130,7 +140,7 @@ def test_qkv_attn_argument_errors(dev):
         dev.free(b)
 
 
-def test_qkv_attn_repeated_calls(dev):
+def test_qkv_attn_repeated_calls(dev, form):
     """Counters return to zero: the same launch again and again, and a different head count after it."""
     _case(dev, 32, 4096, 1500, 2, False, seed=5, repeats=6)
     _case(dev, 5, 256, 700, 1, False, seed=6, repeats=3)
@@ -138,10 +148,10 @@ def test_qkv_attn_repeated_calls(dev):
 
 
 @pytest.mark.parametrize("H,K,n_past", [(32, 4096, 2047), (3, 256, 40)])
-def test_a_wait_that_runs_out_is_reported_and_leaves_the_context_usable(dev, H, K, n_past):
+def test_a_wait_that_runs_out_is_reported_and_leaves_the_context_usable(dev, form, H, K, n_past):
     """The give-up path of the waits inside the launch, forced from the host: the attention workgroups wait for one
     count more than the products can reach, with a bound of a few polls, so every wait runs out and every kernel
-    still ends normally.  Every head's output is NaN in all its elements, the products themselves are right, the next
+    still ends normally (a biased wait keeps the launch that has it whatever form is asked for).  Every head's output is NaN in all its elements, the products themselves are right, the next
     synchronize reports GALOIS_HIP_E_DEVICE_WAIT exactly once, and the same call afterwards -- with the default
     settings -- gives what it gave before, bit for bit (the counters the late products left non-zero are cleared)."""
     from galois_amd import GaloisHipError
@@ -189,3 +199,20 @@ def test_a_wait_that_runs_out_is_reported_and_leaves_the_context_usable(dev, H, 
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     for b in ws + [x, pos, q, k, v, out, kc, vc]:
         dev.free(b)
+
+
+def test_which_form_a_call_takes(dev):
+    """The lines on 256 CUs (a cache of 38 MiB; 24 heads are 576 product workgroups), and what overrides them."""
+    assert dev.info()["n_cu"] == 256
+    for H, n_past, kv_f16, launches in (
+            (32, 1214, False, 2), (32, 1215, False, 1), (23, 7000, False, 2), (24, 1700, False, 1), (1, 0, False, 2),
+            (32, 2430, True, 2), (32, 2431, True, 1), (23, 7000, True, 2), (65536, 0, False, 1)):
+        assert dev.qkv_attn_decode_launches(H, n_past, kv_f16) == launches, (H, n_past, kv_f16)
+    for option in (1, 2):
+        dev.set_option(dev.OPT_QKV_ATTN_LAUNCHES, option)
+        assert [dev.qkv_attn_decode_launches(H, n, False) for H, n in ((1, 0), (32, 4000))] == [option, option]
+        assert dev.qkv_attn_decode_launches(65536, 0, False) == 1
+    dev.set_option(dev.OPT_WAIT_TARGET_BIAS, 1)
+    assert dev.qkv_attn_decode_launches(1, 0, False) == 1
+    dev.set_option(dev.OPT_WAIT_TARGET_BIAS, 0)
+    dev.set_option(dev.OPT_QKV_ATTN_LAUNCHES, 0)
