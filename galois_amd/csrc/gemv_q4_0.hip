@@ -963,17 +963,21 @@ __global__ __launch_bounds__(FA_WAVES * 64, 4) void qkv_attn_decode_fused(const 
     }
 }
 
-// One launch pays when there is much of both to overlap: nine product workgroups or more per four CUs (the attention's
-// registers leave room for two at a time instead of four, so few products gain nothing from being ahead) and a cache
-// that takes longer to fetch than what the fused kernel adds.  Per layer of a decode step, us as two launches / one:
-// 4096 wide, f32 cache, 200 keys 45.0 / 48.7, 800 47.8 / 57.6, 1600 (52 MB) 52.3 / 51.8, 2047 55.2 / 52.6, 4000 70.2 /
-// 63.6; f16 cache 200 45.0 / 53.2, 1200 48.0 / 51.2, 2500 (41 MB) 52.9 / 52.4, 4000 62.0 / 58.7.
+// One launch pays when there is much of both to overlap.  Of the products, more than two workgroups per CU: the attention's
+// registers leave room for two at a time, so fewer products are all resident at once and gain nothing from being ahead
+// (21 heads, 3000 f32 keys 43.9 us a layer of a decode step as two launches / 44.8 as one, 22 heads 48.3 / 46.2).  Of the
+// attention, more than what the fused kernel adds: an f32 cache of 38 MiB up to n_past (32 heads, 600 keys 45.2 / 51.3, 1200 50.4 /
+// 51.8, 1600 51.6 / 51.5, 2047 53.7 / 52.5, 4000 69.0 / 62.9; 40 heads, 900 68.3 / 73.4, 1200 69.2 / 68.9, 1600 73.0 / 70.3);
+// an f16 cache, half as long to fetch, once the attention by itself leaves its fast shapes: a merge of sixteen splits,
+// two workgroups of eight waves per CU (24 heads, 1900 keys 40.8 / 40.5, 2400 42.3 / 41.1; 32 heads, 1600 47.9 / 48.9, 2100 50.9 /
+// 51.0, 4000 61.4 / 56.5; 40 heads, 1300 66.0 / 66.3, 1600 68.2 / 66.9; 52 heads, 1023 73.6 / 75.4, 1300 75.9 / 76.4, 1800 80.5 / 78.3).
 bool fa_one_launch(const galois_hip_ctx *ctx, int64_t n_head, int64_t n_past, bool f16) {
     // what the attention by itself refuses, and a wait that is biased from outside (a test of the waits), keep the one launch
     if (n_head > 65535 || ctx->wait_target_bias != 0) return true;
     if (ctx->qkv_attn_launches) return ctx->qkv_attn_launches == 1;
-    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, L = n_past + 1;
-    return 4 * 3 * n_head * (FA_HEAD_DIM / (FA_WAVES * FA_R)) >= 9 * cus && 2 * L * n_head * FA_HEAD_DIM * (f16 ? 2 : 4) >= (int64_t)38 << 20;
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, L = n_past + 1, S = (L + AT_KEYS - 1) / AT_KEYS;
+    if (3 * n_head * (FA_HEAD_DIM / (FA_WAVES * FA_R)) <= 2 * cus) return false;
+    return f16 ? S > 16 || n_head * S > 2 * cus : 2 * L * n_head * FA_HEAD_DIM * 4 >= (int64_t)38 << 20;
 }
 
 template <typename CT>

@@ -354,9 +354,10 @@ int32_t galois_hip_attn_decode_f16kv(galois_hip_ctx *ctx, const float *q, const 
  * normalisation galois_hip_dequantize_mul_mat_vec_q4_0_group folds in) and the attention that consumes them
  * (galois_hip_attn_decode_f32 / _f16kv above) as one call: qkv[0..2] are the three products, whose dst are the
  * q, k and v vectors of n_head * head_dim floats (written as by the group call, and read by the attention part).
- * Where there is enough of both to overlap (a cache of 38 MiB or more up to n_past, nine product workgroups or more
- * per four compute units) the call is ONE launch, otherwise the two launches of those calls;
- * GALOIS_HIP_OPT_QKV_ATTN_LAUNCHES overrides it.  In one launch the
+ * Where there is enough of both to overlap the call is ONE launch, otherwise the two launches of those calls: one where
+ * the products come to more than two workgroups of 16 rows per compute unit (22 heads or more on 256) and the cache up to
+ * n_past holds 38 MiB or more in f32, or in f16 more than 16 splits of 128 keys a head or more than two splits per compute
+ * unit in all (32 heads: from 1216 f32 or 2049 f16 keys on); GALOIS_HIP_OPT_QKV_ATTN_LAUNCHES overrides it.  In one launch the
  * attention's workgroups follow the products' in the grid, request their cache rows while the last products
  * still stream, and wait -- bounded -- only for their own head's rows of q (k and v where position n_past lives);
  * should a wait ever run out, that head's whole output is NaN, the context's status word is set and the next synchronize

@@ -202,11 +202,13 @@ def test_a_wait_that_runs_out_is_reported_and_leaves_the_context_usable(dev, for
 
 
 def test_which_form_a_call_takes(dev):
-    """The lines on 256 CUs (a cache of 38 MiB; 24 heads are 576 product workgroups), and what overrides them."""
+    """The lines on 256 CUs (22 heads are 528 product workgroups; a cache of 38 MiB in f32; 16 splits a head or two per CU in
+    f16), and what overrides them."""
     assert dev.info()["n_cu"] == 256
     for H, n_past, kv_f16, launches in (
-            (32, 1214, False, 2), (32, 1215, False, 1), (23, 7000, False, 2), (24, 1700, False, 1), (1, 0, False, 2),
-            (32, 2430, True, 2), (32, 2431, True, 1), (23, 7000, True, 2), (65536, 0, False, 1)):
+            (32, 1214, False, 2), (32, 1215, False, 1), (21, 7000, False, 2), (22, 1767, False, 2), (22, 1768, False, 1), (1, 0, False, 2),
+            (32, 2047, True, 2), (32, 2048, True, 1), (40, 1535, True, 2), (40, 1536, True, 1), (21, 7000, True, 2), (22, 2048, True, 1),
+            (65535, 0, True, 1), (65536, 0, False, 1)):
         assert dev.qkv_attn_decode_launches(H, n_past, kv_f16) == launches, (H, n_past, kv_f16)
     for option in (1, 2):
         dev.set_option(dev.OPT_QKV_ATTN_LAUNCHES, option)
