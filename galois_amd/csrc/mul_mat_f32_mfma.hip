@@ -17,11 +17,14 @@
 //     takes k = 8h .. 8h+7: eight consecutive floats of a row that is contiguous along k, and one element per instruction
 //     of a row that is contiguous along n (32 lanes = one contiguous piece).  The next chunk is requested before the
 //     current one is multiplied; nothing meets at a barrier.
-//   - K_CONTIG (scores): the workgroup's four waves own neighbouring columns and all of K.  Otherwise (V p) they own
-//     the same 64 columns and every fourth chunk of K, and their sums meet in LDS at the end, in wave order.
+//   - Scores, and V p where that fills the device: the workgroup's four waves own neighbouring columns and all of K.  SPLIT
+//     (V p of few tiles): they own the same 64 columns and every fourth chunk of K, and their sums meet in LDS at the
+//     end, in wave order.  Merge and idle waves cost, so a short K or many tiles are better whole (wt_split_pays).
 // Measured, us, 128 x 128 tiles against this: V p of 32 heads of 64, 300 rows over 600 keys 111.9 -> 22.4, 700 over 700 139.6 ->
 // 43.3, 17 over 517 81.1 -> 9.4; 32 heads of 128, 512 over 512 101.3 -> 33.1; scores of the same 29.1 -> 23.5, 61.5 -> 41.3, 13.6
-// -> 5.4, 51.8 -> 35.1.
+// -> 5.4, 51.8 -> 35.1.  Products with neither side short gain as much: 512 x 4096 x 4096 743 -> 172 (a contiguous along k), 760 -> 227
+// (along n), 2048 x 2048 x 2048 386 -> 179, 400 -> 182 (f16 a 367 -> 174); 16 rows of 4096 x 4096, where this kernel begins, 676 -> 149, 731 ->
+// 45.
 #include "common.h"
 
 namespace {
@@ -48,17 +51,17 @@ __device__ __forceinline__ void wt_load8(_Float16 (&d)[8], const _Float16 *p) {
     for (int e = 0; e < 8; e++) d[e] = t.v[e];
 }
 
-template <typename AT, bool K_CONTIG>
+template <typename AT, bool K_CONTIG, bool SPLIT>
 __global__ __launch_bounds__(256) void gemm_f32_wave_tiles(const AT *__restrict__ a, const float *__restrict__ b,
                                                             float *__restrict__ dst, int K, int N, int M, int r2, int64_t a_s0,
                                                             int64_t a_s1, int64_t a_s2, int n_tiles) {
-    __shared__ float part[K_CONTIG ? 1 : 3][2][16][64];
+    __shared__ float part[SPLIT ? 3 : 1][2][16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, h = lane >> 5;
     const int mt = blockIdx.x / n_tiles, nt = blockIdx.x - mt * n_tiles;
     const int m0 = mt * WM, i2 = blockIdx.y;
-    const int n0 = nt * (K_CONTIG ? 4 * WN : WN) + (K_CONTIG ? wave * WN : 0);
-    if (K_CONTIG && n0 >= N) return;
+    const int n0 = nt * (SPLIT ? WN : 4 * WN) + (SPLIT ? 0 : wave * WN);
+    if (!SPLIT && n0 >= N) return;
     const AT *ab = a + (int64_t)(i2 / r2) * a_s2;
     const float *brow = b + ((int64_t)i2 * M + min(m0 + r, M - 1)) * K;
     const AT *acol[2];  // K_CONTIG: row n of the tile; otherwise its element of row k = 0
@@ -93,8 +96,8 @@ __global__ __launch_bounds__(256) void gemm_f32_wave_tiles(const AT *__restrict_
             for (int t = 0; t < 2; t++)
                 acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[buf][e], (float)av[buf][t][e], acc[t], 0, 0, 0);
     };
-    constexpr int STEP = K_CONTIG ? WK : 4 * WK;
-    int k0 = K_CONTIG ? 0 : wave * WK;
+    constexpr int STEP = SPLIT ? 4 * WK : WK;
+    int k0 = SPLIT ? wave * WK : 0;
     if (k0 + WK <= K) {
         request(0, k0);
         for (; k0 + STEP + WK <= K; k0 += 2 * STEP) {  // two chunks a turn: the buffers keep their registers
@@ -126,7 +129,7 @@ whole_chunks_done:
         }
         multiply(0);
     }
-    if (!K_CONTIG) {
+    if (SPLIT) {
         if (wave != 0) {
 #pragma unroll
             for (int t = 0; t < 2; t++)
@@ -155,6 +158,18 @@ whole_chunks_done:
     }
 }
 
+// Whether V p is better off with its K dealt to the four waves of a workgroup: rounds of workgroups times what one costs, a
+// quarter of the chunks and a merge worth 32 k against all of them.  rows: row tiles of all slices.  Measured over 4112 sizes (K
+// 16 .. 4096, N 33 .. 16000, 16 .. 4096 rows, 1 .. 32 slices), us, split / whole: one slice of 4096 x 4096 at 16 rows 45 / 150, 32 heads of 128,
+// 512 rows over 512 keys 33 / 52, 8 slices of 1000 columns, 300 rows over 4096 k 219 / 366; the other way 32 slices, 2048 rows of
+// 128 k and 2048 columns 601 / 430 (f16 638 / 450), 4096 rows of 16 k and 16000 columns 156 / 45.
+bool wt_split_pays(int64_t K, int64_t N, int64_t rows, int64_t cus) {
+    if (K <= WK) return false;
+    const int64_t split = (N + WN - 1) / WN * rows, whole = (N + 4 * WN - 1) / (4 * WN) * rows;
+    const double rounds = split > cus ? (double)split / (double)cus : 1.0;
+    return 0.8 * rounds * ((double)K / 4.0 + 32.0) < (double)((whole + cus - 1) / cus) * (double)(K + 16);
+}
+
 }  // namespace
 
 // M > 1 rows of b against a contiguous along K (a_s0 == 1) or along N (a_s1 == 1); false when the grid does not
@@ -162,16 +177,19 @@ whole_chunks_done:
 template <typename AT>
 bool gh_mul_mat_f32_mfma(galois_hip_ctx *ctx, const AT *a, const float *b, float *dst, int K, int N, int M, int ne02,
                          int ne12, int64_t a_s0, int64_t a_s1, int64_t a_s2) {
-    const int64_t n_tiles = a_s0 == 1 ? ((int64_t)N + 4 * WN - 1) / (4 * WN) : ((int64_t)N + WN - 1) / WN;
-    const int64_t tiles = n_tiles * (((int64_t)M + WM - 1) / WM);
-    if (ne12 > 65535 || tiles > 0x7FFFFFFF || (a_s0 != 1 && a_s1 != 1)) return false;
+    if (ne12 > 65535 || (a_s0 != 1 && a_s1 != 1)) return false;
+    const int64_t m_tiles = ((int64_t)M + WM - 1) / WM, cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
+    const bool split = a_s0 != 1 && wt_split_pays(K, N, m_tiles * ne12, cus);
+    const int64_t n_tiles = ((int64_t)N + (split ? WN : 4 * WN) - 1) / (split ? WN : 4 * WN), tiles = n_tiles * m_tiles;
+    if (tiles > 0x7FFFFFFF) return false;
     const dim3 grid((unsigned)tiles, (unsigned)ne12);
-    if (a_s0 == 1)
-        hipLaunchKernelGGL((gemm_f32_wave_tiles<AT, true>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0,
-                           a_s1, a_s2, (int)n_tiles);
-    else
-        hipLaunchKernelGGL((gemm_f32_wave_tiles<AT, false>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0,
-                           a_s1, a_s2, (int)n_tiles);
+#define WT_LAUNCH(K_, S_)                                                                                                     \
+    hipLaunchKernelGGL((gemm_f32_wave_tiles<AT, K_, S_>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0, \
+                       a_s1, a_s2, (int)n_tiles)
+    if (a_s0 == 1) WT_LAUNCH(true, false);
+    else if (split) WT_LAUNCH(false, true);
+    else WT_LAUNCH(false, false);
+#undef WT_LAUNCH
     return true;
 }
 template bool gh_mul_mat_f32_mfma<float>(galois_hip_ctx *, const float *, const float *, float *, int, int, int, int, int,

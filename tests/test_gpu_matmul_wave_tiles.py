@@ -1,5 +1,6 @@
 """The f32 matrix-core products at the edges of their tiles: 32 rows of b, 64 columns, chunks of 16 k dealt to four waves --
 against the oracle through the cases of test_gpu_matmul_prefill_attn (scores and V p of the same sizes)."""
+import numpy as np
 import pytest
 
 from tests import test_gpu_matmul_prefill_attn as cases
@@ -12,3 +13,24 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("f16", [False, True])
 def test_tile_edges(dev, L, H, D, M, f16):
     cases.test_prefill_attention_products(dev, L, H, D, M, f16)
+
+
+@pytest.mark.parametrize("K,N,M,B", [(16, 64, 16, 1), (17, 33, 31, 3), (40, 300, 500, 8), (33, 1000, 130, 16), (100, 4099, 257, 2), (64, 64, 2048, 32),
+                                     (128, 2048, 512, 8), (500, 130, 40, 2)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_a_contiguous_along_n_split_and_whole(dev, K, N, M, B, f16):
+    """Either side of the rule that deals K to a workgroup's waves.  Every result of K f32 products is within (K + 2) 2^-24 of the sum
+    of their magnitudes, whatever the order they are added in."""
+    rng = np.random.default_rng(K + N)
+    a = rng.standard_normal((B, K, N)).astype(np.float16 if f16 else np.float32)
+    b = rng.standard_normal((B, M, K)).astype(np.float32)
+    ab, bb, db = dev.upload(a), dev.upload(b), dev.upload(np.full(B * M * N + 64, 7.5, np.float32))
+    (dev.mul_mat_f16_f32 if f16 else dev.mul_mat_f32)(ab, bb, db, K, N, M, B, B, N, 1, K * N)
+    got = dev.download(db, np.float32, B * M * N + 64)
+    assert np.all(got[B * M * N:] == 7.5)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    for i in {0, B - 1}:
+        err = np.abs(got[i * M * N:(i + 1) * M * N].reshape(M, N) - b[i] @ a[i])
+        assert np.all(err <= (K + 2) * 2.0 ** -24 * (np.abs(b[i]) @ np.abs(a[i])))
+    for buf in (ab, bb, db):
+        dev.free(buf)
