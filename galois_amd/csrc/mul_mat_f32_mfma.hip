@@ -58,7 +58,9 @@ __global__ __launch_bounds__(256) void gemm_f32_wave_tiles(const AT *__restrict_
     __shared__ float part[SPLIT ? 3 : 1][2][16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, h = lane >> 5;
-    const int mt = blockIdx.x / n_tiles, nt = blockIdx.x - mt * n_tiles;
+    const uint32_t tile = blockIdx.z * gridDim.x + blockIdx.x;  // (a launch holds fewer than 2^32 threads along x)
+    const int mt = tile / (uint32_t)n_tiles, nt = tile - (uint32_t)mt * n_tiles;
+    if (mt > (M - 1) / WM) return;
     const int m0 = mt * WM, i2 = blockIdx.y;
     const int n0 = nt * (SPLIT ? WN : 4 * WN) + (SPLIT ? 0 : wave * WN);
     if (!SPLIT && n0 >= N) return;
@@ -181,8 +183,9 @@ bool gh_mul_mat_f32_mfma(galois_hip_ctx *ctx, const AT *a, const float *b, float
     const int64_t m_tiles = ((int64_t)M + WM - 1) / WM, cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
     const bool split = a_s0 != 1 && wt_split_pays(K, N, m_tiles * ne12, cus);
     const int64_t n_tiles = ((int64_t)N + (split ? WN : 4 * WN) - 1) / (split ? WN : 4 * WN), tiles = n_tiles * m_tiles;
-    if (tiles > 0x7FFFFFFF) return false;
-    const dim3 grid((unsigned)tiles, (unsigned)ne12);
+    const int64_t x = tiles < (1 << 23) ? tiles : 1 << 23;
+    if ((tiles + x - 1) / x > 65535) return false;
+    const dim3 grid((unsigned)x, (unsigned)ne12, (unsigned)((tiles + x - 1) / x));
 #define WT_LAUNCH(K_, S_)                                                                                                     \
     hipLaunchKernelGGL((gemm_f32_wave_tiles<AT, K_, S_>), grid, dim3(256), 0, ctx->stream, a, b, dst, K, N, M, ne12 / ne02, a_s0, \
                        a_s1, a_s2, (int)n_tiles)

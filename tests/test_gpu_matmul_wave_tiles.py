@@ -34,3 +34,27 @@ def test_a_contiguous_along_n_split_and_whole(dev, K, N, M, B, f16):
         assert np.all(err <= (K + 2) * 2.0 ** -24 * (np.abs(b[i]) @ np.abs(a[i])))
     for buf in (ab, bb, db):
         dev.free(buf)
+
+
+def test_more_workgroups_than_a_launch_holds_along_x(dev):
+    """16 rows of more than 2^30 columns: over 2^32 threads, so the workgroups go on along z.  K = 1: every result is one product."""
+    N, M = (1 << 30) + 4099, 16
+    row = np.random.default_rng(0).standard_normal(1 << 20).astype(np.float32)
+    a, d = dev.alloc(N * 4), dev.alloc((N * M + 64) * 4)
+    dev.upload(row, a)
+    have = row.size
+    while have < N:
+        n = min(have, N - have)
+        dev.copy_d2d(a.view(have * 4), a, n * 4)
+        have += n
+    b = np.arange(1, M + 1, dtype=np.float32)
+    bb = dev.upload(b)
+    dev.mul_mat_f32(a, bb, d, 1, N, M, 1, 1, N, 1, N)
+    for m in (0, 7, 15):
+        for at in (0, (1 << 29) - 1000, N - 70000):
+            n = 70000
+            got = dev.download(d.view((m * N + at) * 4), np.float32, n)
+            assert np.array_equal(got, b[m] * row[(at + np.arange(n)) % row.size])
+    assert np.all(dev.download(d.view(N * M * 4), np.float32, 64) == 0)
+    for buf in (a, d, bb):
+        dev.free(buf)
