@@ -58,6 +58,21 @@ constexpr int QB = 128;                // blocks per workgroup
 constexpr int QB_CHUNKS = QB * 18 / 16;  // 16-byte pieces of them
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
+// Exchanges between the eight lanes of a block, on the vector pipe: as shuffles through LDS, and with a division per lane and
+// block, they made the kernel slower than a thread per block on inputs that are in a cache (131072 blocks: thread per
+// block 4.1 us, shuffles 4.9, this 4.0; 300000 blocks 8.6, 9.8, 8.3; from HBM 10.9, 11.2, 9.7).
+enum { QZ_SWAP1 = 0xB1, QZ_SWAP2 = 0x4E, QZ_REVERSE = 0x1B, QZ_HALF_MIRROR = 0x141 };  // quad_perm 1032, 2301, 3210; lane 7 - g
+template <int CTRL>
+__device__ __forceinline__ float qz_dpp(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ void qz_first_max(float &amax, float &mx, bool upper) {
+    const float oa = qz_dpp<CTRL>(amax), om = qz_dpp<CTRL>(mx);
+    const bool take = upper ? oa >= amax : oa > amax;
+    amax = take ? oa : amax, mx = take ? om : mx;
+}
+
 __global__ __launch_bounds__(256) void quantize_q4_0_lanes(const float4_t *__restrict__ x, uint8_t *__restrict__ y, int64_t nblocks) {
 #pragma clang fp contract(off)  // as above
     __shared__ __attribute__((aligned(16))) uint8_t out[QB * 18];
@@ -67,34 +82,40 @@ __global__ __launch_bounds__(256) void quantize_q4_0_lanes(const float4_t *__res
     float4_t v[QB / 32];
 #pragma unroll
     for (int i = 0; i < QB / 32; i++) v[i] = x[(b0 + (bl + 32 * i < nb ? bl + 32 * i : nb - 1)) * 8 + g];
+    float mx[QB / 32];
 #pragma unroll
     for (int i = 0; i < QB / 32; i++) {
-        float amax = 0.0f, mx = 0.0f;
+        float amax = 0.0f;
+        mx[i] = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const float a = __builtin_fabsf(v[i][j]);
-            if (amax < a) amax = a, mx = v[i][j];
+            if (amax < a) amax = a, mx[i] = v[i][j];
         }
         // the block's first element of largest magnitude: at equal magnitude the lower lane's
+        qz_first_max<QZ_SWAP1>(amax, mx[i], g & 1);
+        qz_first_max<QZ_SWAP2>(amax, mx[i], g & 2);
+        qz_first_max<QZ_HALF_MIRROR>(amax, mx[i], g & 4);  // the four lanes of a quad agree by now
+    }
+    // lane g works out the scale of block g % 4 of the lane's four, and the quad passes it round: one division instead of four
+    static_assert(QB / 32 == 4, "four blocks a lane, four lanes a quad");
+    const float mxs = (g & 2) ? ((g & 1) ? mx[3] : mx[2]) : ((g & 1) ? mx[1] : mx[0]);
+    float d = mxs * -0.125f;
+    asm volatile("" : "+v"(d));
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    if (g >= 4) *reinterpret_cast<uint16_t *>(out + (bl + 32 * (g - 4)) * 18) = __builtin_bit_cast(uint16_t, (_Float16)d);
+    const float ids[4] = {qz_dpp<0x00>(id), qz_dpp<0x55>(id), qz_dpp<0xAA>(id), qz_dpp<0xFF>(id)};
 #pragma unroll
-        for (int m = 1; m < 8; m <<= 1) {
-            const float oa = __shfl_xor(amax, m, 64), om = __shfl_xor(mx, m, 64);
-            const bool take = (g & m) ? oa >= amax : oa > amax;
-            amax = take ? oa : amax, mx = take ? om : mx;
-        }
-        float d = mx * -0.125f;
-        asm volatile("" : "+v"(d));
-        const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    for (int i = 0; i < QB / 32; i++) {
         uint32_t nib = 0;  // one value per byte
 #pragma unroll
-        for (int j = 0; j < 4; j++) nib |= (uint32_t)(min((int)(v[i][j] * id + 8.5f), 15) & 15) << (8 * j);
-        const uint32_t high = __shfl_xor(nib, 4, 64);  // lane g + 4 holds elements 16 + 4g ..: the high nibbles of the same bytes
+        for (int j = 0; j < 4; j++) nib |= (uint32_t)(min((int)(v[i][j] * ids[i] + 8.5f), 15) & 15) << (8 * j);
+        // lane g + 4 holds elements 16 + 4g ..: the high nibbles of the same bytes (its quad reversed, then the eight lanes)
+        const uint32_t high = __builtin_bit_cast(uint32_t, qz_dpp<QZ_HALF_MIRROR>(qz_dpp<QZ_REVERSE>(__builtin_bit_cast(float, nib))));
         uint16_t *o = reinterpret_cast<uint16_t *>(out + (bl + 32 * i) * 18);
         if (g < 4) {
             const uint32_t q = nib | high << 4;
             o[1 + 2 * g] = (uint16_t)q, o[2 + 2 * g] = (uint16_t)(q >> 16);
-        } else if (g == 4) {
-            o[0] = __builtin_bit_cast(uint16_t, (_Float16)d);
         }
     }
     __syncthreads();
