@@ -317,7 +317,11 @@ inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int M, bool
     sk_tiles best = {0, 0, 0.0};
     for (int m = 1; m <= SK_MAX_MT && m <= t; m++)
         for (int n = swiglu ? 2 : 1; n <= 4; n *= 2) {
-            const int64_t wgs = (cols + 16 * n - 1) / (16 * n) * ((t + m - 1) / m);
+            const int64_t tiles = (cols + 16 * n - 1) / (16 * n), blocks = (t + m - 1) / m;
+            // The weight tiles are dealt to eight XCDs (blockIdx % 8), so a launch runs as long as its fullest XCD, which may hold
+            // more workgroups than CUs where the device as a whole does not (524 x 8192 x 1792: 28 tiles of nine row blocks,
+            // 36 workgroups on four of the XCDs, 52 us against 32 with other tiles).  With very many rows that evens out.
+            const int64_t wgs = (t < 64 ? (tiles + 7) / 8 * 8 : tiles) * blocks;
             const double cost = (double)((wgs + cus - 1) / cus) * sk_cost(n, m);
             if (best.nt == 0 || cost < best.cost) best = {n, m, cost};
         }
