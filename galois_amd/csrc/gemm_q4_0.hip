@@ -834,7 +834,7 @@ namespace {
 // rows that run on it anyway (a narrow matrix of long rows gives the tiles of either other form too few workgroups:
 // 11008 -> 4096 at 150 rows 27.3 us against 57 us whole and 39 us in shares).  The cost model of gemm_pick (rounds of
 // workgroups x cost of a stage x stages) plus the pass that adds the two partial results, which costs about fourteen stages
-// per 2^21 results.  Measured at M = 512 on 256 CUs: 11008 -> 4096 70.3 -> 54.8 us, 4096 -> 4096 32.5 -> 30.2 us (both
+// per 2^21 results, or eight where the caller runs such a pass anyway.  Measured at M = 512 on 256 CUs: 11008 -> 4096 70.3 -> 54.8 us, 4096 -> 4096 32.5 -> 30.2 us (both
 // with the residual); the shapes the model leaves whole are slower when forced into shares.  plain: the adding pass
 // replaces nothing the caller would launch anyway, and the result is to be that of whole tiles unless the product is large:
 // no skinny kernel, and shares only from 64 stages of a 256 x 96 tile on (512 x 13824 x 2816 55 us against 64 whole, 100 x 8192 x
@@ -847,12 +847,16 @@ gemm_form gemm_pick_form(const galois_hip_ctx *ctx, int K, int N, int M, bool pl
     const double c96 = gemm_pick(ctx, N, M, 96).cost * stages, c48 = gemm_pick(ctx, N, M, 48).cost * stages;
     const double whole = c96 < c48 ? c96 : c48;
     const gemm_tile t64 = gemm_pick(ctx, N, M, 64, 2);
-    const double c64x2 = t64.cost * (K / 128 + 2) + 14.0 * (double)mn / (double)(1 << 21);
+    double c64x2 = t64.cost * (K / 128 + 2);
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
     bool large = true;
     double clear = 1.0;
-    if (plain) {
+    if (!plain) {  // the caller's pass reads one result more; stages of a launch that leaves CUs free are up to a tenth faster
+        c64x2 = c64x2 * (t64.wgs < cus ? 0.9 + 0.1 * (double)t64.wgs / (double)cus : 1.0) + 8.0 * (double)mn / (double)(1 << 21);
+    } else {
+        c64x2 += 14.0 * (double)mn / (double)(1 << 21);
         // large: in terms of 256-row tiles, as a lower tile is no reason to leave the shares, which come in lower tiles too
-        const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, m256 = ((int64_t)M + 255) / 256;
+        const int64_t m256 = ((int64_t)M + 255) / 256;
         const double r96 = (double)((((int64_t)N + 95) / 96 * m256 + cus - 1) / cus);
         const double r48 = (double)((((int64_t)N + 47) / 48 * m256 + cus - 1) / cus);
         large = (r96 < 0.65 * r48 ? r96 : 0.65 * r48) * stages >= 64.0;

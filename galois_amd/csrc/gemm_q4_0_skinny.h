@@ -327,7 +327,15 @@ inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int M, bool
         }
     return best;
 }
-inline double skinny_us(const galois_hip_ctx *ctx, int N, int K, int M) { return skinny_pick(ctx, N, M, false).cost * K / 4096.0; }
+inline double sk_far(const sk_tiles &t, int M) {  // row blocks past what shares a weight tile's panel traffic, 0 .. 1
+    const double blocks = (double)(((int64_t)M + 15) / 16 / t.mt);
+    return blocks <= 12.0 ? 0.0 : blocks < 28.0 ? (blocks - 12.0) / 16.0 : 1.0;
+}
+// Over 2652 sizes (K 512 .. 11008, N 512 .. 5120, 81 .. 2000 rows) within 10 %.
+inline double skinny_us(const galois_hip_ctx *ctx, int N, int K, int M) {
+    const sk_tiles t = skinny_pick(ctx, N, M, false);
+    return 1.0 + 1.05 * t.cost * K / 4096.0 * (1.0 + 0.3 * sk_far(t, M));
+}
 
 // KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.  t: tiles the caller has picked.
 int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned,
