@@ -168,7 +168,8 @@ def test_row_tiles_of_the_wide_kernel(dev, m, n):
         assert np.array_equal(got[:140].view(np.uint32), _run(dev, wq, x[:140]).view(np.uint32))
 
 
-@pytest.mark.parametrize("m,k,n", [(100, 8192, 1024), (150, 4096, 768), (190, 1024, 512), (300, 4096, 4096), (390, 2048, 1024)])
+@pytest.mark.parametrize("m,k,n", [(100, 8192, 1024), (150, 4096, 768), (190, 1024, 512), (300, 4096, 4096), (390, 2048, 1024),
+                                   (447, 8192, 2304), (1400, 4096, 768)])
 def test_forms_of_a_narrow_product(dev, m, k, n):
     """With a workspace a narrow product comes whole, in two shares of k or from the few-rows kernel: each sums the same f32
     products in its own order (1e-5 of the largest result)."""
