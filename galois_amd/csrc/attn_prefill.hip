@@ -1,4 +1,5 @@
-// Causal attention of many query rows over a KV cache in one launch: the prefill counterpart of attn_decode.hip.
+// Causal attention of many query rows over a KV cache in one launch (two where the keys are split over workgroups): the
+// prefill counterpart of attn_decode.hip.
 //
 // Replaces, per layer of a prefill, the op sequence cpy(q -> [D, M, H]), matmul(K^T, q), scale, diag_mask_inf +
 // soft_max, matmul(V, p), cpy(-> [D, H, M]) (CudaMatMul src/cuda.rs:867-992, scale src/cuda.rs:1597-1663,
@@ -364,7 +365,9 @@ __global__ __launch_bounds__(256) void attn_prefill_merge(const pa_args a) {
             ms[sp] = rec[64 * PA_D + q], ls[sp] = rec[64 * PA_D + 64 + q];
             os[sp] = *reinterpret_cast<const float4_t *>(rec + q * PA_D + d);
         }
-        float mx = ms[0];  // finite: the first split begins with key 0, which every query sees
+        // finite: some split holds key 0, which every query sees -- not always the first one, as a tile whose walk has fewer
+        // stages than splits leaves some of them empty (maximum -inf, sum and output zeros)
+        float mx = ms[0];
 #pragma unroll
         for (int sp = 1; sp < PA_MAX_SPLITS; sp++) mx = fmaxf(mx, ms[sp]);
         float l = 0.0f;

@@ -129,8 +129,8 @@ __global__ __launch_bounds__(256) void gemm_q4_0_mfma_v1(const uint8_t *__restri
 //     order the A operand of v_mfma_f32_16x16x32_f16 is held (per lane 8 consecutive k of one row),
 //     so a fragment is one contiguous KB: the consumer waves fetch their A fragments straight from
 //     global memory (the 4 MB panel stays in L2) two stages ahead, and X never touches LDS.
-//   - Workgroup tile 256 (M; 192 or 128 where that leaves fewer rows of padding: RT = 3, 2) x 96 (N), k-stage 64 (two Q4_0 blocks = one 36-byte slot per weight
-//     row).  The 512 x 11008 prefill is 2 x 115 = 230 workgroups: one round on 256 CUs.
+//   - Workgroup tile 256 (M; 192 or 128 where that leaves fewer rows of padding: RT = 3, 2) x 96 (N), k-stage 64 (two Q4_0
+//     blocks = one 36-byte slot per weight row).  The 512 x 11008 prefill is 2 x 115 = 230 workgroups: one round on 256 CUs.
 //   - 8 waves: 4 consumers stacked in M, wave tile 64 x 96 -> 4 x 6 MFMA tiles with f32 accumulators
 //     in registers, and 4 producers that fetch the weights as whole 144-byte row pieces (4 stages at
 //     a time), park them raw in LDS, and each stage dequantise one slot per row into an fp16 B tile

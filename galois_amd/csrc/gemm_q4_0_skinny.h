@@ -105,7 +105,7 @@ __device__ __forceinline__ half8_t sk_operand(const uint32_t (&q)[4], half2_t d)
 // Instructions of a piece whose activation fragments are requested together: about eight fragments in flight a wave.
 constexpr int sk_steps(int mt) { return mt <= 1 ? 4 : mt <= 4 ? 2 : 1; }
 // Waves per SIMD the registers are kept to: four hide the requests' latency where the tiles allow it (2 x 2 tiles: 138 -> 110
-// registers, gate | up at 23 rows 21.4 -> 20.3 us).
+// registers, gate | up at 23 rows 21.4 -> 20.3 us with weights in the Infinity Cache, 25.2 from HBM).
 constexpr int sk_occ(int nt, int mt) {
     const int regs = 4 * nt * mt + 8 * sk_steps(mt) * mt + 19 * nt + 40;
     return regs <= 138 ? 4 : regs <= 175 ? 3 : 2;
@@ -279,14 +279,16 @@ int32_t skinny_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16
 }
 
 // Rows up to which the panel calls run here rather than on the wide kernel.  Measured (us, this kernel / that one at its best
-// tile, weights from HBM): q | k | v of 4096 (12288 x 4096) 14.1 / 25.3 at 23 rows, 19.8 / 21.2 at 77, 27.1 / 20.9 at 100;
-// gate | up + SwiGLU (2 x 11008 x 4096) 20.3 / 41.1, 31.6 / 31.7, 40.4 / 31.8.  Narrow matrices stay ahead here for longer (11008 ->
-// 4096 24.9 / 44.5 at 100 rows, 4096 -> 4096 11.9 / 19.2), which gemm_pick_form uses where a caller lets the sums take any
-// order; in the plain calls the order of a result's sum depends on K and on the side of this line M is on, never on N, so
-// matrices multiplied together, one by one or with the SwiGLU behind them give the same bits.
+// tile, weights from HBM): q | k | v of 4096 (12288 x 4096) 16.5 / 20.6 at 23 rows, 19.9 / 21.2 at 64, 22.4 / 21.7 at 80, 29.9 / 21.8 at
+// 100; gate | up + SwiGLU (2 x 11008 x 4096) 25.2 / 31.8, 33.5 / 33.2, 35.9 / 33.2, 43.5 / 32.8; of models 1024 wide 5.5 / 7.8 and 6.0 /
+// 11.6 at 80 rows, 5.6 / 7.9 and 8.0 / 11.6 at 100.  Narrow matrices stay ahead here for longer (11008 -> 4096 at 150 rows 27 / 39 in
+// shares), which gemm_pick_form uses where a caller lets the sums take any order.  In the panel calls without that freedom, and in
+// the f32 entry point up to this line, the order of a result's sum depends on K and on the side of this line M is on, never on N, so
+// matrices multiplied together, one by one or with the SwiGLU behind them give the same bits (above it the f32 entry point may take
+// two shares of k by N).
 constexpr int SK_MAX_ROWS = 80;
 
-// Time of a workgroup relative to others, us at K = 4096 (fitted to the sizes above within 10 %): what a weight tile costs
+// Time of a workgroup relative to others, us at K = 4096 (fitted within 10 %): what a weight tile costs
 // (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.
 inline double sk_cost(int nt, int mt) { return 1.55 * nt + mt * (0.78 + 0.25 * nt); }
 

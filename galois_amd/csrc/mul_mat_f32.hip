@@ -220,7 +220,9 @@ bool gh_mul_mat_f32_mfma(galois_hip_ctx *ctx, const AT *a, const float *b, float
 
 namespace {
 
-constexpr int kMfmaMinRows = 16;  // rows of b from which the 32-row tiles of the f32 matrix-core kernel pay
+// Rows of b from which the 32-row tiles of the f32 matrix-core kernel run.  us at 15 rows (scalar) / 16: a along k, 32 slices of
+// 600 x 128 20.7 / 7.4, one of 1024 x 1024 27.7 / 38.8 (one chain of long k, few tiles); along n 55.9 / 6.0 and 410 / 13.5.
+constexpr int kMfmaMinRows = 16;
 
 template <typename AT>
 int32_t mul_mat_any(galois_hip_ctx *ctx, const AT *a, const float *b, float *dst, int32_t K, int32_t N, int32_t M,

@@ -289,7 +289,7 @@ GResult LlamaDecoder::step(int32_t n_past, int fused) {
     for (Layer &l : layers_) {
         const size_t li = (size_t)(&l - &layers_[0]);
         const bool split = fused >= 4;       // norms split over producer and consumer launches
-        const bool qkv_attn = fused >= 5;    // the three projections and the attention in one launch
+        const bool qkv_attn = fused >= 5;    // the three projections and the attention in one call
         if (grouped) {  // rms_norm * weight + the three projections: one launch
             MatvecItem mq = item(l.wq, x_, q_), mk_ = item(l.wk, x_, k_), mv = item(l.wv, x_, v_);
             if (split && li > 0) {  // the previous layer's last launch left x * attn_norm in a_ and the sums of squares of x

@@ -43,8 +43,8 @@ class LlamaDecoder {
     // fused = 4 splits the norms that follow a residual add over the launch that produces the residual stream (it
     // also writes the stream times the next norm weight and its partial sums of squares) and the launch that consumes
     // it (it fetches one vector instead of two and waits for no reduction): the same 5 launches per layer.
-    // fused = 5 sends the q | k | v products and the attention out as one launch (galois_qkv_attn_decode; heads of
-    // 128): 4 launches per layer.
+    // fused = 5 sends the q | k | v products and the attention out as one call (galois_qkv_attn_decode; heads of
+    // 128): 4 calls per layer, and 4 or 5 launches, as that call takes one or two by the sizes.
     // fused >= 3 are the plans that run with an f16 KV cache.
     GResult decode(int32_t token, int32_t n_past, int fused);
     // Records the same step as a graph / replays the recorded step.
@@ -54,7 +54,7 @@ class LlamaDecoder {
     // decode steps, issued with the many-row ops: the Q4_0 products through the prefill matmul on fp16 panels that the
     // norms and the SwiGLU write directly (q | k | v and gate | up one launch each), rope_custom over all positions,
     // the n new rows of both caches appended at once, scores = K^T Q and out = V P per head on the matrix cores with
-    // a causal soft_max between them (heads of 128: galois_attn_prefill instead, one launch that writes the panel of
+    // a causal soft_max between them (heads of 128: galois_attn_prefill instead, one call that writes the panel of
     // the output projection; f32 caches receive the rotated keys and the values directly); the output and down
     // projections add the residual stream where they store (galois_matmul_panel_add).  Afterwards the caches hold positions 0 .. n_past + n - 1 and logits() the last
     // token's.  n_embd and n_ff must be multiples of 256; caches [n_embd, n_ctx] (not head-major), f32 or f16.
@@ -63,7 +63,7 @@ class LlamaDecoder {
     size_t ops_per_prefill() const { return n_prefill_ops_; }  // library calls of the last prefill (a call is one or two launches)
     const Tensor &logits() const { return logits_; }
     const LlamaHParams &hparams() const { return hp_; }
-    size_t ops_per_step() const { return n_ops_; }
+    size_t ops_per_step() const { return n_ops_; }  // library calls of the last decode step (a call is one or two launches)
 
    private:
     struct Layer {
@@ -152,13 +152,15 @@ GResult galois_rope_qk_append(const RopeCustomOption &op, const Tensor &q, const
                               Tensor &q_out, Tensor &k_rows, Tensor *v_rows);
 
 // Causal attention of all rows of q ([n_embd, n] f32, rotated) over caches ([n_embd, n_ctx], both f32 or both f16) that
-// already hold positions 0 .. n_past + n - 1, in one launch (galois_hip_attn_prefill_f32 / _f16kv; heads of 128).
+// already hold positions 0 .. n_past + n - 1, in one call (galois_hip_attn_prefill_f32 / _f16kv; heads of 128; one launch, or
+// two where few rows leave compute units free).
 // dst is either an F32 tensor [n_embd, n] or an F16 panel of galois_panel_elems(n_embd, n) elements.
 GResult galois_attn_prefill(const Tensor &q, const Tensor &k_cache, const Tensor &v_cache, Tensor &dst, size_t n_head,
                             int32_t n_past, float scale);
 
 // The three products q | k | v (as galois_matvec_group takes them; plain or normalising) and the attention that
-// consumes them (galois_attn_decode on their dst tensors) in one launch (galois_hip_qkv_attn_decode_f32 / _f16kv).
+// consumes them (galois_attn_decode on their dst tensors) in one call (galois_hip_qkv_attn_decode_f32 / _f16kv: one launch
+// or two).
 GResult galois_qkv_attn_decode(const RopeCustomOption &op, const std::vector<MatvecItem> &qkv, Tensor &k_cache, Tensor &v_cache,
                                const Tensor &pos, Tensor &out, size_t n_head, int32_t n_past, float scale);
 

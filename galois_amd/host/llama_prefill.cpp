@@ -302,7 +302,7 @@ GResult LlamaDecoder::prefill(const int32_t *tokens, size_t n, int32_t n_past) {
     RopeCustomOption rope;
     rope.n_dims = D, rope.mode = 0, rope.n_ctx = (int32_t)C, rope.freq_base = hp_.freq_base, rope.freq_scale = hp_.freq_scale;
     size_t ops = 0;
-    const bool one_launch = D == 128;  // the attention of a layer as one launch (galois_attn_prefill)
+    const bool one_launch = D == 128;  // the attention of a layer as one call (galois_attn_prefill)
     const float attn_scale = 1.0f / sqrtf((float)D);
     G_TRY(galois_get_rows(tok_embd_, tok, x)); ops++;
     // the first layer's attention norm; every later one rides on the pass that adds the down projection's shares
