@@ -28,7 +28,8 @@ __global__ __launch_bounds__(AT_THREADS) void attn_decode_partial(const float *_
                                                                   const int32_t *__restrict__ pos, float freq_scale,
                                                                   float theta_scale, float scale, int64_t key_stride,
                                                                   int64_t head_stride) {
-    attn_decode_wg<LPR, CT, AT_THREADS, false, KEYS>(q, k, v, kc, vc, part, done, out, H, L, pos, freq_scale, theta_scale, scale,
+    // heads of 64 in pieces of 128 keys: up to sixteen splits, or many rows in flight a CU, which the registers of larger merges cost
+    attn_decode_wg<LPR, CT, AT_THREADS, false, KEYS, LPR == 16 && KEYS == 128 ? 16 : 32>(q, k, v, kc, vc, part, done, out, H, L, pos, freq_scale, theta_scale, scale,
                                                (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x, nullptr, 0u, key_stride,
                                                head_stride);
 }
@@ -89,7 +90,11 @@ int32_t attn_decode_launch(galois_hip_ctx *ctx, const float *q, const float *k, 
     // choice here: 32 heads of 128, 90 keys 6.8 -> 6.1, 203 9.0 -> 7.5, 512 10.1 -> 8.8, 1024 13.8 -> 12.1, 2048 19.7 ->
     // 18.3 (f16 7.2 -> 6.2, 9.4 -> 7.6, 9.4 -> 8.4, 10.9 -> 10.2, 15.2 -> 14.4); 4000 keys with eight waves 42.9 against 33.7;
     // 16 heads of 64, 203 keys 7.2 -> 6.1, 4000 15.8 -> 12.8.
-    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, s64 = (L + 63) / 64;
+    // Rows of 4096 elements lie on the same memory channels, and long pieces ask for more of them at a time: 64 heads of 64 keep
+    // pieces of 128 keys while those of 256 are up to three workgroups per CU (f16: two and a half); 2060 f32 keys 20.4
+    // against 23.8, 3000 29.0 / 30.0, 3500 31.9 / 31.8; f16 2060 16.1 / 17.8, 2700 20.1 / 19.2; 56 and 80 heads gain at all of these.
+    const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256, s64 = (L + 63) / 64, s256 = (L + 255) / 256;
+    const bool same_channels = key_stride % 4096 == 0 && 2 * n_head * s256 <= (sizeof(CT) == 4 ? 6 : 5) * cus;
 #define AT_LAUNCH(LPR_, KEYS_, THREADS_)                                                                                          \
     hipLaunchKernelGGL((attn_decode_partial<LPR_, CT, KEYS_, THREADS_>), dim3((unsigned)((L + KEYS_ - 1) / KEYS_), (unsigned)n_head), \
                        dim3(THREADS_), 0, ctx->stream, q, k, v, k_cache, v_cache, part, done, out, n_head, L, pos, freq_scale,   \
@@ -99,7 +104,7 @@ int32_t attn_decode_launch(galois_hip_ctx *ctx, const float *q, const float *k, 
         else if ((int64_t)n_head * S <= 2 * cus && S <= 32) AT_LAUNCH(32, 128, 512);
         else AT_LAUNCH(32, 128, 256);
     } else {
-        if ((L > 128 && L <= 256) || S > 16) AT_LAUNCH(16, 256, 512);
+        if ((L > 128 && L <= 256) || (S > 16 && !same_channels)) AT_LAUNCH(16, 256, 512);
         else AT_LAUNCH(16, 128, 256);
     }
 #undef AT_LAUNCH

@@ -95,7 +95,8 @@ __device__ __forceinline__ void at_combine_few(const float *rec, float *__restri
 // element d.  The split maxima and sums are fetched by S threads at once and the weights exp(m_s - M) shared
 // through LDS; the partial outputs are then read eight splits at a time.
 constexpr int AT_MAX_SPLITS = 1024;
-template <int AT_THREADS, bool FUSED>
+// FEW: splits that are merged in one trip (at_combine_few), 16, 24 or 32 at most.
+template <int AT_THREADS, bool FUSED, int FEW>
 __device__ __forceinline__ void at_combine(const float *rec, float *__restrict__ out_h, int D, int S, float *w,
                                            float (*red)[AT_THREADS / 64]) {
     constexpr int WAVES = AT_THREADS / 64;
@@ -104,11 +105,11 @@ __device__ __forceinline__ void at_combine(const float *rec, float *__restrict__
         at_combine_few<16>(rec, out_h, d, D, S);
         return;
     }
-    if (!FUSED && S <= 24) {  // (the launch with the products has its waves hide the difference, and was 0.4 us slower for the code)
+    if (FEW >= 24 && !FUSED && S <= 24) {  // (the launch with the products has its waves hide the difference, and was 0.4 us slower for the code)
         at_combine_few<24>(rec, out_h, d, D, S);
         return;
     }
-    if (S <= 32) {
+    if (FEW >= 32 && S <= 32) {
         at_combine_few<32>(rec, out_h, d, D, S);
         return;
     }
@@ -202,7 +203,7 @@ __device__ __forceinline__ float4 at_load4_coherent(const float *p) {
 // merges a head returns the three counters to zero.  A wait that runs out (spin_limit polls) is agreed on by the whole
 // workgroup: the head's record -- and with it the head's output, whichever workgroup merges it -- becomes NaN in
 // every element, and *status (pinned host memory the context reads after its next wait for the stream) is set.
-template <int LPR, typename CT, int AT_THREADS, bool FUSED, int KEYS = AT_KEYS>
+template <int LPR, typename CT, int AT_THREADS, bool FUSED, int KEYS = AT_KEYS, int FEW = 32>
 __device__ __forceinline__ void attn_decode_wg(const float *__restrict__ q, const float *__restrict__ k,
                                                const float *__restrict__ v, CT *__restrict__ kc, CT *__restrict__ vc,
                                                float *__restrict__ part, unsigned *__restrict__ done,
@@ -398,7 +399,7 @@ __device__ __forceinline__ void attn_decode_wg(const float *__restrict__ q, cons
     }
     __syncthreads();
     if (!last_flag) return;
-    at_combine<AT_THREADS, FUSED>(part + (size_t)h * S * (D + 4), out + (size_t)h * D, D, S, cw, cred);
+    at_combine<AT_THREADS, FUSED, FEW>(part + (size_t)h * S * (D + 4), out + (size_t)h * D, D, S, cw, cred);
 }
 
 }  // namespace

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
     (32, 128, 64), (32, 128, 192), (32, 128, 193), (32, 128, 256), (32, 128, 257), (32, 128, 512), (32, 128, 513), (32, 128, 2049),
     (8, 128, 1024), (8, 128, 1025), (5, 128, 4096), (5, 128, 4097), (64, 128, 1100), (2, 64, 128), (2, 64, 129), (2, 64, 256),
     (2, 64, 257), (3, 64, 2048), (3, 64, 2049), (3, 64, 4200), (3, 64, 8300), (2, 128, 3072), (2, 128, 3073),
-    (2, 64, 6144), (2, 64, 6145)])
+    (2, 64, 6144), (2, 64, 6145), (64, 64, 2100), (64, 64, 2600)])
 @pytest.mark.parametrize("f16", [False, True])
 def test_workgroup_shapes(dev, H, D, keys, f16):
     check = test_gpu_attn.test_attn_decode_with_f16_caches if f16 else test_gpu_attn.test_attn_decode_matches_the_op_sequence
