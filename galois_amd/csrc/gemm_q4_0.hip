@@ -879,6 +879,7 @@ gemm_form gemm_pick_form(const galois_hip_ctx *ctx, int K, int N, int M, bool pl
 // Few rows of 288 or more never gain on v1 and are not worth the arithmetic; t receives the skinny kernel's tiles if they were
 // looked for.
 bool gemm_v1_pays(const galois_hip_ctx *ctx, int K, int N, int M, sk_tiles &t) {
+    if (M > 65535 * TM) return false;  // its row tiles are the grid's y
     if (K <= 192) return true;
     if (M <= SK_MAX_ROWS && K >= 288 && N < 1 << 24) return false;
     const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
