@@ -13,7 +13,7 @@ int32_t gh_check_device_status(galois_hip_ctx *ctx) {
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return gh_hip(ctx, e, "clearing the wait counters");
     return gh_fail(ctx, GALOIS_HIP_E_DEVICE_WAIT,
-                   "qkv_attn_decode: a workgroup gave up waiting for the products of its launch; the attention output of "
+                   "qkv_attn_decode or llama_step: a workgroup gave up waiting for others of its launch; the result of "
                    "that call is NaN and what was launched after it on this context is not to be trusted (the counters "
                    "have been cleared: the context can be used again)");
 }

@@ -211,6 +211,15 @@ GResult LlamaDecoder::create(const LlamaHParams &hp, const Device &dev, std::uni
     G_TRY(mk(&m->logits_, F32, dev, V, 1));
     G_TRY(mk(&m->ssq_, F32, dev, (E + 15) / 16));
     G_TRY(mk(&m->ssq1_, F32, dev, (E + 15) / 16));
+    {
+        galois_hip_llama_model model;
+        std::vector<galois_hip_llama_layer> layers;
+        int64_t bytes = 0;
+        m->step_model(&model, &layers);
+        G_TRY(dev.gpu->check(galois_hip_llama_step_workspace(dev.gpu->ctx(), &model, &bytes)));
+        if (bytes > 0) G_TRY(mk(&m->step_ws_, F32, dev, (size_t)(bytes + 3) / 4));
+        m->step_ws_bytes_ = bytes;
+    }
     *out = std::move(m);
     return GError{};
 }
@@ -236,9 +245,46 @@ Tensor *LlamaDecoder::tensor(const std::string &name, int layer) {
     return nullptr;
 }
 
-GResult LlamaDecoder::set_inputs(int32_t token, int32_t n_past) {
+void LlamaDecoder::step_model(galois_hip_llama_model *m, std::vector<galois_hip_llama_layer> *layers) {
+    const size_t D = hp_.n_embd / hp_.n_head;
+    layers->clear();
+    for (Layer &l : layers_)
+        layers->push_back({l.wq.data(), l.wk.data(), l.wv.data(), l.wo.data(), l.w_gate.data(), l.w_up.data(), l.w_down.data(),
+                           (const float *)l.attn_norm.data(), (const float *)l.ffn_norm.data(), l.k_cache.data(), l.v_cache.data()});
+    memset(m, 0, sizeof(*m));
+    m->n_embd = (int32_t)hp_.n_embd, m->n_head = (int32_t)hp_.n_head, m->n_ff = (int32_t)hp_.n_ff, m->n_vocab = (int32_t)hp_.n_vocab;
+    m->n_layer = (int32_t)layers_.size(), m->n_ctx = (int32_t)hp_.n_ctx, m->kv_f16 = hp_.kv_f16;
+    m->head_major_n_ctx = hp_.kv_head_major ? (int32_t)hp_.n_ctx : 0;
+    m->rms_eps = hp_.rms_eps, m->freq_scale = hp_.freq_scale, m->theta_scale = powf(hp_.freq_base, -2.0f / (float)D);
+    m->scale = *(const float *)scale_.data();
+    m->tok_embd = tok_embd_.data(), m->output = output_.data(), m->out_norm = (const float *)out_norm_.data();
+    m->logits = (float *)logits_.data(), m->token = (int32_t *)tok_id_.data(), m->pos = (int32_t *)pos_.data();
+    m->layers = layers->data(), m->workspace = step_ws_bytes_ ? step_ws_.data() : nullptr, m->workspace_bytes = step_ws_bytes_;
+}
+
+// The whole step in one call where the library takes it (token < 0: the token on the device); *taken says whether it did.
+GResult LlamaDecoder::whole_step(int32_t token, int32_t n_past, bool *taken) {
+    *taken = false;
+    if (step_ws_bytes_ == 0) return GError{};
+    galois_hip_llama_model model;
+    std::vector<galois_hip_llama_layer> layers;
+    step_model(&model, &layers);
+    const int32_t st = galois_hip_llama_step(dev_.gpu->ctx(), &model, token, n_past);
+    if (st == GALOIS_HIP_E_UNSUPPORTED) return GError{};
+    G_TRY(dev_.gpu->check(st));
+    *taken = true;
+    n_ops_ = 2 + 4 * layers_.size();  // what the step consists of, as it is counted where its calls go out one by one
+    return GError{};
+}
+
+GResult LlamaDecoder::check_inputs(int32_t token, int32_t n_past) const {
     if (token < 0 || (size_t)token >= hp_.n_vocab) return err(GError::ShapeError, "decode: token id out of range");
     if (n_past < 0 || (size_t)n_past >= hp_.n_ctx) return err(GError::ShapeError, "decode: n_past must be below n_ctx");
+    return GError{};
+}
+
+GResult LlamaDecoder::set_inputs(int32_t token, int32_t n_past) {
+    G_TRY(check_inputs(token, n_past));
     if (token != last_token_) G_TRY(tok_id_.write(&token, sizeof(token)));  // synchronous copies: only when they change
     if (n_past != last_pos_) G_TRY(pos_.write(&n_past, sizeof(n_past)));
     last_token_ = token, last_pos_ = n_past;
@@ -258,6 +304,11 @@ GResult LlamaDecoder::step(int32_t n_past, int fused) {
     if (fused >= 5 && (D != 128 || E > 11776))
         return err(GError::Unimplemented, "LlamaDecoder: the launch that carries q | k | v and the attention (fused = 5) needs heads of 128 "
                                           "and n_embd up to 11776");
+    if (fused >= 5) {
+        bool taken = false;
+        G_TRY(whole_step(-1, n_past, &taken));
+        if (taken) return GError{};
+    }
     RopeCustomOption rope;
     rope.n_dims = D, rope.mode = 0, rope.n_ctx = (int32_t)C, rope.freq_base = hp_.freq_base, rope.freq_scale = hp_.freq_scale;
     size_t ops = 0;
@@ -415,6 +466,15 @@ GResult LlamaDecoder::step(int32_t n_past, int fused) {
 }
 
 GResult LlamaDecoder::decode(int32_t token, int32_t n_past, int fused) {
+    if (fused >= 5) {  // the call stores token and position on the device itself
+        G_TRY(check_inputs(token, n_past));
+        bool taken = false;
+        G_TRY(whole_step(token, n_past, &taken));
+        if (taken) {
+            last_token_ = token, last_pos_ = n_past;
+            return GError{};
+        }
+    }
     G_TRY(set_inputs(token, n_past));
     return step(n_past, fused);
 }

@@ -44,7 +44,8 @@ class LlamaDecoder {
     // also writes the stream times the next norm weight and its partial sums of squares) and the launch that consumes
     // it (it fetches one vector instead of two and waits for no reduction): the same 5 launches per layer.
     // fused = 5 sends the q | k | v products and the attention out as one call (galois_qkv_attn_decode; heads of
-    // 128): 4 calls per layer, and 4 or 5 launches, as that call takes one or two by the sizes.
+    // 128): 4 calls per layer, and 4 or 5 launches, as that call takes one or two by the sizes -- or, where
+    // galois_hip_llama_step takes the model (n_embd up to 4096), the whole step as that one call.
     // fused >= 3 are the plans that run with an f16 KV cache.
     GResult decode(int32_t token, int32_t n_past, int fused);
     // Records the same step as a graph / replays the recorded step.
@@ -63,13 +64,17 @@ class LlamaDecoder {
     size_t ops_per_prefill() const { return n_prefill_ops_; }  // library calls of the last prefill (a call is one or two launches)
     const Tensor &logits() const { return logits_; }
     const LlamaHParams &hparams() const { return hp_; }
-    size_t ops_per_step() const { return n_ops_; }  // library calls of the last decode step (a call is one or two launches)
+    size_t ops_per_step() const { return n_ops_; }  // calls the last decode step's plan consists of (a call is one or two launches; plan 5 may send
+                                                  // all of them out as one)
 
    private:
     struct Layer {
         Tensor attn_norm, ffn_norm, wq, wk, wv, wo, w_gate, w_up, w_down, k_cache, v_cache;
     };
+    GResult check_inputs(int32_t token, int32_t n_past) const;
     GResult set_inputs(int32_t token, int32_t n_past);
+    void step_model(galois_hip_llama_model *m, std::vector<galois_hip_llama_layer> *layers);
+    GResult whole_step(int32_t token, int32_t n_past, bool *taken);
     GResult step(int32_t n_past, int fused);
 
     LlamaHParams hp_;
@@ -79,6 +84,8 @@ class LlamaDecoder {
     Tensor tok_id_, pos_, scale_;                                    // I32 [1], I32 [1], host f32 [1]
     Tensor x_, t_, a_, q_, k_, v_, qr_, kr_, s_, p_, o_, ao_, x1_, f_, g_, u_, h_, d_, logits_;
     Tensor ssq_, ssq1_;  // partial sums of squares of x and x1 (fused = 4)
+    Tensor step_ws_;     // what galois_hip_llama_step keeps between its stages (fused = 5, where it takes the model)
+    int64_t step_ws_bytes_ = 0;
     struct Prefill {  // intermediates of prefill(), for up to `rows` tokens attending over up to `keys` positions
         size_t rows = 0, keys = 0;
         Tensor tok, pos, x, x1, q, k, v, qr, kr, q3, s, p, o, ao, panel_e, panel_f, split_ws;

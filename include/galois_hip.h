@@ -46,8 +46,8 @@ extern "C" {
 #define GALOIS_HIP_E_UNSUPPORTED (-5) /* the reference leaves this combination todo!() and so do we */
 #define GALOIS_HIP_E_ARCH (-6)      /* the device is not gfx950 */
 #define GALOIS_HIP_E_DEVICE_WAIT (-7) /* reported by synchronize / *_sync_copy: a workgroup of galois_hip_qkv_attn_decode_*
-                                       * gave up a bounded wait for other workgroups of its launch.  The attention output of
-                                       * that call is NaN, later launches on the context may have read stale vectors; the
+                                       * or galois_hip_llama_step gave up a bounded wait for other workgroups of its launch.
+                                       * The attention output (the logits) of that call is NaN, later launches on the context may have read stale vectors; the
                                        * status is reported once, the context is usable again afterwards */
 
 typedef struct galois_hip_ctx galois_hip_ctx;
@@ -373,6 +373,39 @@ int32_t galois_hip_qkv_attn_decode_f16kv(galois_hip_ctx *ctx, const galois_hip_g
                                          const int32_t *pos, float freq_scale, float theta_scale, float scale, int32_t head_major_n_ctx);
 /* How many launches such a call issues on this context (1 or 2): for these sizes, or as the option says. */
 int32_t galois_hip_qkv_attn_decode_launches(galois_hip_ctx *ctx, int32_t n_head, int32_t n_past, int32_t kv_f16, int32_t *n_launches);
+
+/* A decode step of a LLaMA-architecture model -- embedding row, every layer's products, attention, norms and residual adds,
+ * final norm and lm head -- in two launches (a deeper model than 40 layers: one more per 40), for a caller that would
+ * otherwise issue galois_hip_get_rows_q4_0, galois_hip_qkv_attn_decode_* and galois_hip_dequantize_mul_mat_vec_q4_0_group
+ * layer by layer (no counterpart in the reference, which has no model graph).  Same arithmetic as those calls with the
+ * norms split over producer and consumer, up to the order of f32 sums; row n_past of every layer's caches is written as
+ * galois_hip_qkv_attn_decode_* writes it.  Heads of 128 (n_embd = 128 * n_head), n_embd up to 4096, n_ff a multiple of 64
+ * up to 12288, up to 250 layers, 64 splits of 128 f32 or 256 f16 keys.
+ *   galois_hip_llama_step_workspace: bytes of zero-initialised device memory (256-byte aligned) the model's steps keep
+ *     between their stages -- one such block per model in flight; 0 if the step is not one this call takes.
+ *   token >= 0: the token to decode and its position n_past, which are also stored to model->token and model->pos.
+ *   token < 0: the token and the rotation's position are read from there when the launch runs (a recorded step).
+ * The stages of the step wait for one another inside the launch, with bounded waits: should one run out, the logits are
+ * NaN and the next synchronize or *_sync_copy returns GALOIS_HIP_E_DEVICE_WAIT (once). */
+typedef struct galois_hip_llama_layer {
+    const void *wq, *wk, *wv, *wo, *w_gate, *w_up, *w_down; /* Q4_0 */
+    const float *attn_norm, *ffn_norm;
+    void *k_cache, *v_cache;
+} galois_hip_llama_layer;
+typedef struct galois_hip_llama_model {
+    int32_t n_embd, n_head, n_ff, n_vocab, n_layer, n_ctx;
+    int32_t kv_f16, head_major_n_ctx; /* as the attention calls take them */
+    float rms_eps, freq_scale, theta_scale, scale;
+    const void *tok_embd, *output;    /* Q4_0 [n_vocab][n_embd] */
+    const float *out_norm;
+    float *logits;
+    int32_t *token, *pos;             /* one int32 each, on the device */
+    const galois_hip_llama_layer *layers; /* n_layer of them, on the host */
+    void *workspace;
+    int64_t workspace_bytes;
+} galois_hip_llama_model;
+int32_t galois_hip_llama_step_workspace(galois_hip_ctx *ctx, const galois_hip_llama_model *model, int64_t *bytes);
+int32_t galois_hip_llama_step(galois_hip_ctx *ctx, const galois_hip_llama_model *model, int32_t token, int32_t n_past);
 
 /* One Q4_0 matrix against the panel with the residual stream added: Y = residual + W . panel (residual may be null),
  * Y and residual [M][N] f32 -- an output or down projection and the add that follows it (CudaMatMul then add_f32,
