@@ -884,7 +884,7 @@ bool gemm_v1_pays(const galois_hip_ctx *ctx, int K, int N, int M, sk_tiles &t) {
     if (M <= SK_MAX_ROWS && K >= 288 && N < 1 << 24) return false;
     const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
     const double tiles = (double)(((int64_t)N + TN - 1) / TN * (((int64_t)M + TM - 1) / TM)) / (double)cus, mn = (double)M * N * 1e-6;
-    t = skinny_pick(ctx, N, M, false);
+    t = skinny_pick(ctx, N, K, M, false, false);
     const int64_t m_blocks = (((int64_t)M + 15) / 16 + t.mt - 1) / t.mt, n_tiles = ((int64_t)N + 16 * t.nt - 1) / (16 * t.nt);
     if ((n_tiles + 8) * m_blocks >= (int64_t)1 << 23) return true;  // a launch holds fewer than 2^32 threads
     const double far = m_blocks > 16 ? (m_blocks < 32 ? (m_blocks - 16) / 16.0 : 1.0) : 0.0;  // row blocks past what shares a panel in L2
@@ -927,7 +927,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_f32(galois_hip_ctx *ctx, const void *
     // chunk after chunk, when the workspace is too small and cannot grow (while a graph is captured, or out of memory).  A
     // result does not depend on the rows around it, so the bits are the same.
     const int64_t chunk = (int64_t)(gh_block_bytes(ctx->n_cu) / ((size_t)k_pad * sizeof(_Float16))) & ~(int64_t)15;
-    sk_tiles tiles = {0, 0, 0.0};
+    sk_tiles tiles = {0, 0, 0.0, false};
     if (gemm_panel_shape_ok(k_pad, M) && (wide || (chunk > 0 && !gemm_v1_pays(ctx, K, N, M, tiles)))) {
         int32_t st = GALOIS_HIP_OK;
         const bool ws = gh_reserve_workspace(ctx, need);

@@ -20,30 +20,51 @@
 
 namespace {
 
+constexpr int SK_PIECE = 144;  // bytes of a piece of 256 k of one row
 constexpr int SK_MAX_MT = 5;  // row tiles per wave: more would take the registers of the second wave per SIMD
 
-// A lane's share of a piece: two blocks, as they lie in memory.
-template <bool ALIGNED>
+// How a wave's weights arrive.  SK_BLOCKS: any 2-byte aligned block, by the lane that multiplies it.  SK_SLOTS (K % 64 == 0, W
+// 4-byte aligned): a 36-byte slot, likewise.  SK_RUNS (K % 256 == 0 besides): the 144 bytes a piece has of a row by a quad of
+// lanes, 16 bytes each, 16 more 64 bytes on, the last 16 by the first; slots then change lanes through LDS.  A request for
+// slots touches 32 to 40 lines and every line comes up in nine requests; runs are asked for once (23 rows of gate | up 20.3 ->
+// 17.9 us, q | k | v of 4096 14.2 -> 11.8, each at its best tiles; which pays: skinny_pick.  Rows that are not whole pieces lose: 77 x
+// 3200 x 8640 19.8 -> 21.8 with the last piece's requests moved back to the row's end).  The bits are the same.
+enum sk_form { SK_BLOCKS, SK_SLOTS, SK_RUNS };
+template <sk_form FORM>
 struct sk_raw;
 
 template <>
-struct sk_raw<true> {  // K % 64 == 0 and W 4-byte aligned: one 36-byte slot
+struct sk_raw<SK_SLOTS> {
     uint32_t w[9];
 };
 template <>
-struct sk_raw<false> {  // any 2-byte aligned block: its four aligned dwords and the two bytes before or behind them
+struct sk_raw<SK_RUNS> {
+    uint32_t w[12];
+};
+template <>
+struct sk_raw<SK_BLOCKS> {  // four aligned dwords and the two bytes before or behind them
     uint32_t w[2][4];
     uint32_t h[2];
 };
 
+// A piece of a tile in runs.  row: the lane's row, lane / 4 of the tile, at the lane's 16 bytes.
+__device__ __forceinline__ void sk_load(sk_raw<SK_RUNS> &q, const uint8_t *row, int piece) {
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(row + (size_t)piece * SK_PIECE);
+#pragma unroll
+    for (int i = 0; i < 4; i++) q.w[i] = p[i], q.w[4 + i] = p[16 + i];
+    if ((threadIdx.x & 3) == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) q.w[8 + i] = p[32 + i];
+    }
+}
 // block: index of the lane's first block in its row (even); nblocks: blocks of the row.  Blocks past the end are
-// loaded from the row's last ones and given a zero scale by sk_blocks.
-__device__ __forceinline__ void sk_load(sk_raw<true> &q, const uint8_t *row, int block, int nblocks) {
+// loaded from the row's last ones and given a zero scale by sk_unpack.
+__device__ __forceinline__ void sk_load(sk_raw<SK_SLOTS> &q, const uint8_t *row, int block, int nblocks) {
     const uint32_t *p = reinterpret_cast<const uint32_t *>(row + (size_t)min(block, nblocks - 2) * 18);
 #pragma unroll
     for (int i = 0; i < 9; i++) q.w[i] = p[i];
 }
-__device__ __forceinline__ void sk_load(sk_raw<false> &q, const uint8_t *row, int block, int nblocks) {
+__device__ __forceinline__ void sk_load(sk_raw<SK_BLOCKS> &q, const uint8_t *row, int block, int nblocks) {
 #pragma unroll
     for (int b = 0; b < 2; b++) {
         const uint8_t *p = row + (size_t)min(block + b, nblocks - 1) * 18;
@@ -59,18 +80,39 @@ struct sk_blocks {
     uint32_t q[2][4];  // the nibble dwords of both blocks
     half2_t d[2];
 };
-__device__ __forceinline__ void sk_unpack(sk_blocks &o, const sk_raw<true> &r, const uint8_t *, int block, int nblocks) {
+__device__ __forceinline__ void sk_unpack_slot(sk_blocks &o, const uint32_t (&w)[9], bool in) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        o.q[0][i] = __builtin_amdgcn_alignbit(r.w[i + 1], r.w[i], 16);
-        o.q[1][i] = r.w[5 + i];
+        o.q[0][i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], 16);
+        o.q[1][i] = w[5 + i];
     }
-    const bool in = block < nblocks;
-    const _Float16 a = __builtin_bit_cast(_Float16, (uint16_t)(in ? r.w[0] & 0xFFFFu : 0u));
-    const _Float16 b = __builtin_bit_cast(_Float16, (uint16_t)(in ? r.w[4] >> 16 : 0u));
+    const _Float16 a = __builtin_bit_cast(_Float16, (uint16_t)(in ? w[0] & 0xFFFFu : 0u));
+    const _Float16 b = __builtin_bit_cast(_Float16, (uint16_t)(in ? w[4] >> 16 : 0u));
     o.d[0] = half2_t{a, a}, o.d[1] = half2_t{b, b};
 }
-__device__ __forceinline__ void sk_unpack(sk_blocks &o, const sk_raw<false> &r, const uint8_t *row, int block, int nblocks) {
+__device__ __forceinline__ void sk_unpack(sk_blocks &o, const sk_raw<SK_SLOTS> &r, int block, int nblocks) {
+    sk_unpack_slot(o, r.w, block < nblocks);
+}
+// lds: the wave's own 2304 bytes, the tile's rows one behind the other.
+__device__ __forceinline__ void sk_unpack(sk_blocks &o, const sk_raw<SK_RUNS> &r, uint8_t *lds) {
+    const int lane = threadIdx.x & 63;
+    uint8_t *put = lds + (lane >> 2) * SK_PIECE + (lane & 3) * 16;
+    *reinterpret_cast<uint4 *>(put) = make_uint4(r.w[0], r.w[1], r.w[2], r.w[3]);
+    *reinterpret_cast<uint4 *>(put + 64) = make_uint4(r.w[4], r.w[5], r.w[6], r.w[7]);
+    if ((lane & 3) == 0) *reinterpret_cast<uint4 *>(put + 128) = make_uint4(r.w[8], r.w[9], r.w[10], r.w[11]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // (a wave's LDS instructions execute in order)
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t *get = reinterpret_cast<const uint32_t *>(lds) + (lane & 15) * (SK_PIECE / 4) + (lane >> 4) * 9;
+    uint32_t w[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) w[i] = get[i];  // 36 bytes from lane to lane: no two lanes in one bank
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    sk_unpack_slot(o, w, true);
+}
+__device__ __forceinline__ void sk_unpack(sk_blocks &o, const sk_raw<SK_BLOCKS> &r, const uint8_t *row, int block, int nblocks) {
 #pragma unroll
     for (int b = 0; b < 2; b++) {
         const bool odd = ((uintptr_t)(row + (size_t)min(block + b, nblocks - 1) * 18) & 2) != 0;
@@ -106,8 +148,8 @@ __device__ __forceinline__ half8_t sk_operand(const uint32_t (&q)[4], half2_t d)
 constexpr int sk_steps(int mt) { return mt <= 1 ? 4 : mt <= 4 ? 2 : 1; }
 // Waves per SIMD the registers are kept to: four hide the requests' latency where the tiles allow it (2 x 2 tiles: 138 -> 110
 // registers, gate | up at 23 rows 21.4 -> 20.3 us with weights in the Infinity Cache, 25.2 from HBM).
-constexpr int sk_occ(int nt, int mt) {
-    const int regs = 4 * nt * mt + 8 * sk_steps(mt) * mt + 19 * nt + 40;
+constexpr int sk_occ(int nt, int mt, sk_form form) {
+    const int regs = 4 * nt * mt + 8 * sk_steps(mt) * mt + (form == SK_RUNS ? 22 : 19) * nt + 40;
     return regs <= 138 ? 4 : regs <= 175 ? 3 : 2;
 }
 
@@ -138,18 +180,20 @@ __device__ __forceinline__ void sk_store4(const gemm_mats &mats, int n, int m, f
 
 // K: the rows' true length (a multiple of 32); kp_blocks: 32-k blocks of a panel row, a multiple of 8, zeros past K.
 // With mats.swiglu_out the first NT / 2 tiles are gate rows and the others the same rows of the up matrix.
-template <int NT, int MT, int KS, bool ALIGNED>
-__global__ __launch_bounds__(KS * 64, sk_occ(NT, MT)) void gemm_q4_0_skinny(const gemm_mats mats, const _Float16 *__restrict__ Xh, int K,
+template <int NT, int MT, int KS, sk_form FORM>
+__global__ __launch_bounds__(KS * 64, sk_occ(NT, MT, FORM)) void gemm_q4_0_skinny(const gemm_mats mats, const _Float16 *__restrict__ Xh, int K,
                                                             int kp_blocks, int M, int n_tiles, int m_blocks) {
     constexpr int SG = sk_steps(MT), GROUPS = 8 / SG;  // an even number of groups a piece
     __shared__ __attribute__((aligned(16))) float4_t part[KS][KS][64];
+    static_assert(sizeof(part[0]) >= 16 * SK_PIECE, "a wave's tile of weights lies in its share of the sums' LDS");
     // blockIdx % 8 is the XCD: the row blocks of one weight tile follow one another on it, so the second reads its
     // weights from that XCD's L2
     const int idx = blockIdx.x >> 3;
     const int nt0 = (idx / m_blocks) * 8 + (blockIdx.x & 7), mb = idx % m_blocks;
     if (nt0 >= n_tiles) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = lane & 15, kg = lane >> 4;
+    const int r = lane & 15, kg = lane >> 4, wr = FORM == SK_RUNS ? lane >> 2 : r;  // wr: the row whose weights the lane requests
+    uint8_t *const wlds = reinterpret_cast<uint8_t *>(part[wave]);
     const bool swiglu = mats.swiglu_out != nullptr;
     const int nblocks = K / 32, npieces = kp_blocks / 8;
     const size_t wrow_bytes = (size_t)nblocks * 18;
@@ -158,9 +202,9 @@ __global__ __launch_bounds__(KS * 64, sk_occ(NT, MT)) void gemm_q4_0_skinny(cons
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         if (NT > 1 && swiglu)
-            row[t] = mats.W[t >= NT / 2] + (size_t)min(nt0 * (NT / 2 * 16) + (t % (NT / 2 > 0 ? NT / 2 : 1)) * 16 + r, mats.N[0] - 1) * wrow_bytes;
+            row[t] = mats.W[t >= NT / 2] + (size_t)min(nt0 * (NT / 2 * 16) + (t % (NT / 2 > 0 ? NT / 2 : 1)) * 16 + wr, mats.N[0] - 1) * wrow_bytes;
         else
-            row[t] = gemm_w_row(mats, nt0 * (NT * 16) + t * 16 + r, wrow_bytes);
+            row[t] = gemm_w_row(mats, nt0 * (NT * 16) + t * 16 + wr, wrow_bytes);
     }
     // fragment (b, c) of row tile i, piece p: byte fo[i] + p * 8 KB + b * 1 KB + c * 256 of the panel
     const int m16_last = (M + 15) / 16 - 1;
@@ -183,21 +227,34 @@ __global__ __launch_bounds__(KS * 64, sk_occ(NT, MT)) void gemm_q4_0_skinny(cons
             for (int i = 0; i < MT; i++)
                 dst[j][i] = *reinterpret_cast<const half8_t *>(xb + (size_t)piece * 8192 + fo[i] + (g * SG + j) / 4 * 1024 + (g * SG + j) % 4 * 256);
     };
-    sk_raw<ALIGNED> raw[NT];
+    sk_raw<FORM> raw[NT];
+    auto weights = [&](sk_raw<FORM> &q, const uint8_t *w, int p) {
+        if constexpr (FORM == SK_RUNS)
+            sk_load(q, w + (lane & 3) * 16, p);
+        else
+            sk_load(q, w, p * 8 + kg * 2, nblocks);
+    };
     int piece = wave;
     if (piece < npieces) {
 #pragma unroll
-        for (int t = 0; t < NT; t++) sk_load(raw[t], row[t], piece * 8 + kg * 2, nblocks);
+        for (int t = 0; t < NT; t++) weights(raw[t], row[t], piece);
         frags(f[0], piece, 0);
     }
     for (; piece < npieces; piece += KS) {
         const int next = min(piece + KS, npieces - 1);  // the last round requests a piece again, unused
         sk_blocks blk[NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) sk_unpack(blk[t], raw[t], row[t], piece * 8 + kg * 2, nblocks);
+        for (int t = 0; t < NT; t++) {
+            if constexpr (FORM == SK_RUNS)
+                sk_unpack(blk[t], raw[t], wlds);
+            else if constexpr (FORM == SK_SLOTS)
+                sk_unpack(blk[t], raw[t], piece * 8 + kg * 2, nblocks);
+            else
+                sk_unpack(blk[t], raw[t], row[t], piece * 8 + kg * 2, nblocks);
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < NT; t++) sk_load(raw[t], row[t], next * 8 + kg * 2, nblocks);
+        for (int t = 0; t < NT; t++) weights(raw[t], row[t], next);
 #pragma unroll
         for (int g = 0; g < GROUPS; g++) {
             frags(f[(g + 1) & 1], g + 1 < GROUPS ? piece : next, (g + 1) % GROUPS);
@@ -224,7 +281,7 @@ __global__ __launch_bounds__(KS * 64, sk_occ(NT, MT)) void gemm_q4_0_skinny(cons
     constexpr int TILES = NT * MT;
 #pragma unroll
     for (int c0 = 0; c0 < TILES; c0 += KS) {
-        if (c0) __syncthreads();
+        if (c0 || FORM == SK_RUNS) __syncthreads();  // (the waves' weights lie where the first sums go)
 #pragma unroll
         for (int j = 0; j < KS; j++) {
             constexpr int H = NT / 2 > 0 ? NT / 2 : 1;
@@ -267,13 +324,13 @@ __global__ __launch_bounds__(KS * 64, sk_occ(NT, MT)) void gemm_q4_0_skinny(cons
     }
 }
 
-template <int NT, int MT, int KS, bool ALIGNED>
+template <int NT, int MT, int KS, sk_form FORM>
 int32_t skinny_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M) {
     const int cols_per_tile = mats.swiglu_out ? NT / 2 * 16 : NT * 16;
     const int cols = mats.swiglu_out ? mats.N[0] : mats.n_total;
     const int n_tiles = (cols + cols_per_tile - 1) / cols_per_tile, m_blocks = ((M + 15) / 16 + MT - 1) / MT;
     const dim3 grid((unsigned)((n_tiles + 7) / 8 * 8 * m_blocks));
-    hipLaunchKernelGGL((gemm_q4_0_skinny<NT, MT, KS, ALIGNED>), grid, dim3(KS * 64), 0, ctx->stream, mats, Xh, K, kp_blocks, M,
+    hipLaunchKernelGGL((gemm_q4_0_skinny<NT, MT, KS, FORM>), grid, dim3(KS * 64), 0, ctx->stream, mats, Xh, K, kp_blocks, M,
                        n_tiles, m_blocks);
     return GALOIS_HIP_OK;
 }
@@ -289,18 +346,21 @@ int32_t skinny_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16
 constexpr int SK_MAX_ROWS = 80;
 
 // Time of a workgroup relative to others, us at K = 4096 (fitted within 10 %): what a weight tile costs
-// (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.
-inline double sk_cost(int nt, int mt) { return 1.55 * nt + mt * (0.78 + 0.25 * nt); }
+// (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.  runs: by the form of the weights.
+inline double sk_cost(int nt, int mt, bool runs) {
+    if (runs) return nt == 1 ? 2.0 + 1.12 * mt : nt == 2 ? 3.6 + 1.05 * mt : 6.5 + 1.72 * mt;
+    return 1.55 * nt + mt * (0.78 + 0.25 * nt);
+}
 
-template <int KS, bool ALIGNED>
+template <int KS, sk_form FORM>
 int32_t skinny_launch_tiles(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, int nt, int mt) {
 #define SK_MT(NT_)                                                                                    \
     switch (mt) {                                                                                     \
-        case 1: return skinny_launch<NT_, 1, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
-        case 2: return skinny_launch<NT_, 2, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
-        case 3: return skinny_launch<NT_, 3, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
-        case 4: return skinny_launch<NT_, 4, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);            \
-        default: return skinny_launch<NT_, SK_MAX_MT, KS, ALIGNED>(ctx, mats, Xh, K, kp_blocks, M);   \
+        case 1: return skinny_launch<NT_, 1, KS, FORM>(ctx, mats, Xh, K, kp_blocks, M);            \
+        case 2: return skinny_launch<NT_, 2, KS, FORM>(ctx, mats, Xh, K, kp_blocks, M);            \
+        case 3: return skinny_launch<NT_, 3, KS, FORM>(ctx, mats, Xh, K, kp_blocks, M);            \
+        case 4: return skinny_launch<NT_, 4, KS, FORM>(ctx, mats, Xh, K, kp_blocks, M);            \
+        default: return skinny_launch<NT_, SK_MAX_MT, KS, FORM>(ctx, mats, Xh, K, kp_blocks, M);   \
     }
     if (nt == 1) SK_MT(1)
     if (nt == 2) SK_MT(2)
@@ -312,11 +372,13 @@ int32_t skinny_launch_tiles(galois_hip_ctx *ctx, const gemm_mats &mats, const _F
 struct sk_tiles {
     int nt, mt;
     double cost;
+    bool runs;
 };
-inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int M, bool swiglu) {
+// whole: the weights' rows are whole pieces and 4-byte aligned, so that runs are possible.
+inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int K, int M, bool swiglu, bool whole) {
     const int64_t cus = ctx->n_cu > 0 ? ctx->n_cu : 256;
     const int t = (M + 15) / 16;
-    sk_tiles best = {0, 0, 0.0};
+    sk_tiles best = {0, 0, 0.0, false};
     for (int m = 1; m <= SK_MAX_MT && m <= t; m++)
         for (int n = swiglu ? 2 : 1; n <= 4; n *= 2) {
             const int64_t tiles = (cols + 16 * n - 1) / (16 * n), blocks = (t + m - 1) / m;
@@ -324,8 +386,13 @@ inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int M, bool
             // more workgroups than CUs where the device as a whole does not (524 x 8192 x 1792: 28 tiles of nine row blocks,
             // 36 workgroups on four of the XCDs, 52 us against 32 with other tiles).  With very many rows that evens out.
             const int64_t wgs = (t < 64 ? (tiles + 7) / 8 * 8 : tiles) * blocks;
-            const double cost = (double)((wgs + cus - 1) / cus) * sk_cost(n, m);
-            if (best.nt == 0 || cost < best.cost) best = {n, m, cost};
+            // Runs pay where a CU has more to do than one workgroup's chain of requests, whose LDS trip they lengthen: long rows
+            // (eight waves), a second workgroup, four weight tiles a wave (over 500 sizes 3 to 6 % each; elsewhere -3 to 0 %).
+            // Workgroups that share a CU then overlap a little.
+            double rounds = (double)((wgs + cus - 1) / cus);
+            const bool runs = whole && (K >= 8192 || wgs > cus || n == 4);
+            const double cost = rounds * (runs && K < 8192 && rounds > 1 ? rounds > 2 ? 0.85 : 0.9 : 1.0) * sk_cost(n, m, runs);
+            if (best.nt == 0 || cost < best.cost) best = {n, m, cost, runs};
         }
     return best;
 }
@@ -335,20 +402,23 @@ inline double sk_far(const sk_tiles &t, int M) {  // row blocks past what shares
 }
 // Over 2652 sizes (K 512 .. 11008, N 512 .. 5120, 81 .. 2000 rows) within 10 %.
 inline double skinny_us(const galois_hip_ctx *ctx, int N, int K, int M) {
-    const sk_tiles t = skinny_pick(ctx, N, M, false);
+    const sk_tiles t = skinny_pick(ctx, N, K, M, false, true);
     return 1.0 + 1.05 * t.cost * K / 4096.0 * (1.0 + 0.3 * sk_far(t, M));
 }
 
 // KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.  t: tiles the caller has picked.
 int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned,
-                          sk_tiles t = {0, 0, 0.0}) {
+                          sk_tiles t = {0, 0, 0.0, false}) {
     const bool swiglu = mats.swiglu_out != nullptr;
-    if (t.nt == 0) t = skinny_pick(ctx, swiglu ? 2 * (int64_t)mats.N[0] : mats.n_total, M, swiglu);
-    if (K >= 8192)
-        return aligned ? skinny_launch_tiles<8, true>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
-                       : skinny_launch_tiles<8, false>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt);
-    return aligned ? skinny_launch_tiles<4, true>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
-                   : skinny_launch_tiles<4, false>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt);
+    if (t.nt == 0) t = skinny_pick(ctx, swiglu ? 2 * (int64_t)mats.N[0] : mats.n_total, K, M, swiglu, aligned && K % 256 == 0);
+    const sk_form form = !aligned ? SK_BLOCKS : t.runs ? SK_RUNS : SK_SLOTS;
+#define SK_FORM(KS_)                                                                                                     \
+    return form == SK_RUNS    ? skinny_launch_tiles<KS_, SK_RUNS>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)            \
+           : form == SK_SLOTS ? skinny_launch_tiles<KS_, SK_SLOTS>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)           \
+                              : skinny_launch_tiles<KS_, SK_BLOCKS>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
+    if (K >= 8192) SK_FORM(8);
+    SK_FORM(4);
+#undef SK_FORM
 }
 
 }  // namespace
