@@ -348,7 +348,7 @@ constexpr int SK_MAX_ROWS = 80;
 // Time of a workgroup relative to others, us at K = 4096 (fitted within 10 %): what a weight tile costs
 // (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.  runs: by the form of the weights.
 inline double sk_cost(int nt, int mt, bool runs) {
-    if (runs) return nt == 1 ? 2.0 + 1.12 * mt : nt == 2 ? 3.6 + 1.05 * mt : 6.5 + 1.72 * mt;
+    if (runs) return nt == 1 ? 2.0 + 1.12 * mt : nt == 2 ? 3.6 + 1.05 * mt : nt == 3 ? 5.0 + 1.3 * mt : 6.5 + 1.72 * mt;
     return 1.55 * nt + mt * (0.78 + 0.25 * nt);
 }
 
@@ -364,6 +364,7 @@ int32_t skinny_launch_tiles(galois_hip_ctx *ctx, const gemm_mats &mats, const _F
     }
     if (nt == 1) SK_MT(1)
     if (nt == 2) SK_MT(2)
+    if (nt == 3) SK_MT(3)
     SK_MT(4)
 #undef SK_MT
 }
@@ -380,17 +381,20 @@ inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int K, int 
     const int t = (M + 15) / 16;
     sk_tiles best = {0, 0, 0.0, false};
     for (int m = 1; m <= SK_MAX_MT && m <= t; m++)
-        for (int n = swiglu ? 2 : 1; n <= 4; n *= 2) {
+        for (int n = swiglu ? 2 : 1; n <= 4; n += swiglu ? 2 : 1) {
+            // three tiles a wave fill the device where two leave a second round nearly empty (77 x 3200 x 8640: 180 workgroups
+            // instead of 270 or 135; 12288 columns: 256); short rows are better off in more rounds
+            if (n == 3 && K <= (m == 1 ? 2560 : 512)) continue;
             const int64_t tiles = (cols + 16 * n - 1) / (16 * n), blocks = (t + m - 1) / m;
             // The weight tiles are dealt to eight XCDs (blockIdx % 8), so a launch runs as long as its fullest XCD, which may hold
             // more workgroups than CUs where the device as a whole does not (524 x 8192 x 1792: 28 tiles of nine row blocks,
             // 36 workgroups on four of the XCDs, 52 us against 32 with other tiles).  With very many rows that evens out.
             const int64_t wgs = (t < 64 ? (tiles + 7) / 8 * 8 : tiles) * blocks;
             // Runs pay where a CU has more to do than one workgroup's chain of requests, whose LDS trip they lengthen: long rows
-            // (eight waves), a second workgroup, four weight tiles a wave (over 500 sizes 3 to 6 % each; elsewhere -3 to 0 %).
+            // (eight waves), a second workgroup, three or four weight tiles a wave (over 500 sizes 3 to 6 % each; elsewhere -3 to 0 %).
             // Workgroups that share a CU then overlap a little.
             double rounds = (double)((wgs + cus - 1) / cus);
-            const bool runs = whole && (K >= 8192 || wgs > cus || n == 4);
+            const bool runs = whole && (K >= 8192 || wgs > cus || n >= 3);
             const double cost = rounds * (runs && K < 8192 && rounds > 1 ? rounds > 2 ? 0.85 : 0.9 : 1.0) * sk_cost(n, m, runs);
             if (best.nt == 0 || cost < best.cost) best = {n, m, cost, runs};
         }
