@@ -309,6 +309,13 @@ class Device:
         self._check(self._lib.galois_hip_add_rms_norm_mul_f16_panel(self._ctx, _ptr(a), _ptr(b), _ptr(c), _ptr(sum_out), _ptr(weight),
                                                                     _ptr(panel), ncols, nrows, eps))
 
+    def rope_pairs(self, pairs, n_tokens, first_pos, freq_scale, theta_scale):
+        self._check(self._lib.galois_hip_rope_pairs(self._ctx, _ptr(pairs), n_tokens, first_pos, freq_scale, theta_scale))
+
+    def mul_mat_q4_0_qkv_rope_f16_panel(self, wq, wk, wv, panel, pairs, q, k_rows, v_rows, kv_f16, head_dim, n_head, k, m):
+        self._check(self._lib.galois_hip_mul_mat_q4_0_qkv_rope_f16_panel(self._ctx, _ptr(wq), _ptr(wk), _ptr(wv), _ptr(panel), _ptr(pairs), _ptr(q),
+                                                                         _ptr(k_rows), _ptr(v_rows), int(kv_f16), head_dim, n_head, k, m))
+
     def rope_qk_append(self, q, k, v, q_out, k_rows, v_rows, kv_f16, head_dim, n_head, n_tokens, pos, freq_scale, theta_scale):
         """rope of q (to q_out) and of k (to the cache rows k_rows) and, when v is given, v to v_rows, one launch."""
         self._check(self._lib.galois_hip_rope_qk_append(self._ctx, _ptr(q), _ptr(k), _ptr(v), _ptr(q_out), _ptr(k_rows), _ptr(v_rows),

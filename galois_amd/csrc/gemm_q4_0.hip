@@ -327,7 +327,18 @@ struct gemm_mats {
     // has both products of an element in its registers and stores silu(gate) * up, as fp16, into the panel of the
     // [N[0], M] operand at swiglu_out.  n_total = 96 * ceil(N[0] / 48) then.
     _Float16 *swiglu_out;
+    // q | k | v of heads of 128, each N[0] columns: what leaves the epilogue of the first two is rotated (rope_custom, mode 0,
+    // n_dims 128).  rope: (cos, sin) of row m and pair i of a head at m * 64 + i; kv_f16: the second and third result are
+    // cache rows in f16, rounded to nearest even from the f32 result.  Null: no rotation.
+    const float2 *rope;
+    int32_t kv_f16;
 };
+
+// The rotation of one element x whose neighbour in its pair is p; odd: x is the pair's second.  The same sequence of
+// roundings as rope_f32: one product, then a fused multiply-add.
+__device__ __forceinline__ float gemm_rotate(float x, float p, float2 cs, bool odd) {
+    return odd ? __builtin_fmaf(p, cs.y, x * cs.x) : __builtin_fmaf(x, cs.x, -(p * cs.y));
+}
 
 // Row `c` of the concatenated weights (clamped to the last one): its bytes.
 __device__ __forceinline__ const uint8_t *gemm_w_row(const gemm_mats &mats, int c, size_t wrow_bytes) {
@@ -656,6 +667,50 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
                         *reinterpret_cast<uint2 *>(out + (size_t)(m >> 4) * (size_t)(N >> 5) * 1024 + col_at + (size_t)(m & 15) * 16) =
                             make_uint2(pair, pair2);
                 }
+        }
+        return;
+    }
+    // q | k | v: a pair of columns is a pair of neighbouring lanes, sixteen columns lie in one matrix.  The angles of four rows
+    // of every column tile are requested together (the operands' registers are free now).
+    if (mats.rope != nullptr) {
+        const bool odd = lane & 1;
+        const int N = mats.N[0];
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            const int mb = m0 + wm * (16 * RT) + i * 16 + 4 * (lane >> 4);
+            float2 cs[NF][4];
+#pragma unroll
+            for (int j = 0; j < NF; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    cs[j][e] = mats.rope[(uint32_t)min(mb + e, M - 1) * 64u + (uint32_t)(((n0 + ncol0 + j * 16 + (lane & 15)) & 127) >> 1)];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NF; j++) {
+                const int n = n0 + ncol0 + j * 16, t = n / N;  // uniform
+                const int nl = n - t * N + (lane & 15);
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float x = acc[i][j][e];
+                    const float p = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));
+                    v[e] = t < 2 ? gemm_rotate(x, p, cs[j][e], odd) : x;
+                }
+                if (t > 2) break;
+                if (t > 0 && mats.kv_f16) {
+                    _Float16 *Y = reinterpret_cast<_Float16 *>(mats.Y[t]);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        asm volatile("" : "+v"(v[e]));  // rounded to f32 first, as the ops one by one would
+                        if (mb + e < M) Y[(size_t)(mb + e) * N + nl] = (_Float16)v[e];
+                    }
+                } else {
+                    float *Y = mats.Y[t];
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (mb + e < M) Y[(size_t)(mb + e) * N + nl] = v[e];
+                }
+            }
         }
         return;
     }
@@ -1136,6 +1191,53 @@ extern "C" int32_t galois_hip_add_rms_norm_mul_f16_panel(galois_hip_ctx *ctx, co
     else
         hipLaunchKernelGGL((rms_norm_to_f16_tiles<4, true>), grid, block, 0, ctx->stream, a, weight, y, nrows, ncols, eps, groups, per_xcd, b, c, sum_out);
     GH_LAUNCH_CHECK(ctx, "add_rms_norm_mul_f16_panel launch");
+}
+
+namespace {
+// One thread per pair: the angles of rope_f32 at position first + row.
+__global__ __launch_bounds__(256) void rope_pairs(float2 *__restrict__ out, int n, int first, float freq_scale, float theta_scale) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n * 64) return;
+    const float p0 = (float)(first + (i >> 6)) * freq_scale;
+    float sn, cs;
+    sincosf(p0 * powf(theta_scale, (float)(i & 63)), &sn, &cs);
+    out[i] = make_float2(cs, sn);
+}
+}  // namespace
+
+extern "C" int32_t galois_hip_rope_pairs(galois_hip_ctx *ctx, float *pairs, int32_t n_tokens, int32_t first_pos, float freq_scale, float theta_scale) {
+    GH_REQUIRE_CTX(ctx);
+    GH_REQUIRE(ctx, pairs, GALOIS_HIP_E_NULL, "rope_pairs");
+    GH_REQUIRE(ctx, n_tokens > 0 && n_tokens <= 1 << 24 && first_pos >= 0 && (int64_t)first_pos + n_tokens <= 0x7FFFFFFF, GALOIS_HIP_E_SHAPE,
+               "rope_pairs: n_tokens positive, at most 2^24");
+    GH_REQUIRE(ctx, gh_aligned(pairs, 16), GALOIS_HIP_E_ALIGN, "rope_pairs: 16-byte aligned pairs");
+    GH_BIND(ctx);
+    hipLaunchKernelGGL(rope_pairs, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, ctx->stream, (float2 *)pairs, n_tokens, first_pos,
+                       freq_scale, theta_scale);
+    GH_LAUNCH_CHECK(ctx, "rope_pairs launch");
+}
+
+// q | k | v, the rotation of q and k and the append of k and v: one launch.
+extern "C" int32_t galois_hip_mul_mat_q4_0_qkv_rope_f16_panel(galois_hip_ctx *ctx, const void *W_q, const void *W_k, const void *W_v,
+                                                              const void *panel, const float *pairs, float *q, void *k_rows, void *v_rows,
+                                                              int32_t kv_f16, int32_t head_dim, int32_t n_head, int32_t K, int32_t M) {
+    GH_REQUIRE_CTX(ctx);
+    GH_REQUIRE(ctx, W_q && W_k && W_v && panel && pairs && q && k_rows && v_rows, GALOIS_HIP_E_NULL, "mul_mat_q4_0_qkv_rope_f16_panel");
+    GH_REQUIRE(ctx, head_dim == 128, GALOIS_HIP_E_UNSUPPORTED, "mul_mat_q4_0_qkv_rope_f16_panel: head_dim 128");
+    GH_REQUIRE(ctx, gemm_panel_shape_ok(K, M) && n_head > 0 && n_head <= 1 << 20, GALOIS_HIP_E_SHAPE,
+               "mul_mat_q4_0_qkv_rope_f16_panel: K a positive multiple of 256, (M + 16) * K below 2^31, n_head positive");
+    GH_REQUIRE(ctx, gh_aligned(W_q, 16) && gh_aligned(W_k, 16) && gh_aligned(W_v, 16) && gh_aligned(panel, 16) && gh_aligned(pairs, 16) &&
+                        gh_aligned(q, 16) && gh_aligned(k_rows, 16) && gh_aligned(v_rows, 16),
+               GALOIS_HIP_E_ALIGN, "mul_mat_q4_0_qkv_rope_f16_panel: 16-byte aligned operands");
+    GH_BIND(ctx);
+    gemm_mats mats = {};
+    mats.W[0] = (const uint8_t *)W_q, mats.W[1] = (const uint8_t *)W_k, mats.W[2] = (const uint8_t *)W_v;
+    mats.Y[0] = q, mats.Y[1] = (float *)k_rows, mats.Y[2] = (float *)v_rows;
+    mats.N[0] = mats.N[1] = mats.N[2] = n_head * head_dim;
+    mats.rope = (const float2 *)pairs, mats.kv_f16 = kv_f16 != 0;
+    const int32_t st = gemm_launch_any(ctx, mats, 3, (const _Float16 *)panel, K, M);
+    if (st != GALOIS_HIP_OK) return st;
+    GH_LAUNCH_CHECK(ctx, "mul_mat_q4_0_qkv_rope_f16_panel launch");
 }
 
 // gate | up and the SwiGLU between them and the down projection in one launch: the panel of silu(Wg . x) * (Wu . x).

@@ -163,6 +163,21 @@ __device__ __forceinline__ void sk_store4(const gemm_mats &mats, int n, int m, f
         const bool ge = n >= mats.col0[t];
         Y = ge ? mats.Y[t] : Y, N = ge ? mats.N[t] : N, first = ge ? mats.col0[t] : first;
     }
+    if (mats.rope != nullptr) {  // q | k | v: every matrix has whole sixteens of columns, its rows are 16-byte aligned
+        if (n < mats.col0[2]) {
+            const float4 cs = *reinterpret_cast<const float4 *>(mats.rope + (size_t)m * 64 + (((n - first) & 127) >> 1));
+            const float2 c0 = make_float2(cs.x, cs.y), c1 = make_float2(cs.z, cs.w);
+            v = float4_t{gemm_rotate(v[0], v[1], c0, false), gemm_rotate(v[1], v[0], c0, true), gemm_rotate(v[2], v[3], c1, false),
+                         gemm_rotate(v[3], v[2], c1, true)};
+        }
+        if (mats.kv_f16 && n >= mats.col0[1]) {
+            asm volatile("" : "+v"(v));  // rounded to f32 first, as the ops one by one would
+            typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+            *reinterpret_cast<h4 *>(reinterpret_cast<_Float16 *>(Y) + (size_t)m * N + (n - first)) =
+                h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+            return;
+        }
+    }
     float *dst = Y + (size_t)m * N + (n - first);
     if (n - first + 4 <= N && ((uintptr_t)dst & 15) == 0) {
         *reinterpret_cast<float4_t *>(dst) = v;

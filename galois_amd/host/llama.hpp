@@ -88,7 +88,7 @@ class LlamaDecoder {
     int64_t step_ws_bytes_ = 0;
     struct Prefill {  // intermediates of prefill(), for up to `rows` tokens attending over up to `keys` positions
         size_t rows = 0, keys = 0;
-        Tensor tok, pos, x, x1, q, k, v, qr, kr, q3, s, p, o, ao, panel_e, panel_f, split_ws;
+        Tensor tok, pos, pairs, x, x1, q, k, v, qr, kr, q3, s, p, o, ao, panel_e, panel_f, split_ws;
     };
     GResult prefill_buffers(size_t n, size_t keys);
     Prefill pf_;

@@ -242,8 +242,13 @@ GResult LlamaDecoder::prefill_buffers(size_t n, size_t keys) {
     const GGmlType F32 = GGmlType::F32;
     G_TRY(mk(&b.tok, GGmlType::I32, dev_, rows));
     G_TRY(mk(&b.pos, GGmlType::I32, dev_, rows));
-    for (Tensor *t : {&b.x, &b.x1, &b.q, &b.k}) G_TRY(mk(t, F32, dev_, E, rows));
-    if (hp_.kv_f16) G_TRY(mk(&b.v, F32, dev_, E, rows));  // an f32 cache takes the values straight from the product
+    for (Tensor *t : {&b.x, &b.x1}) G_TRY(mk(t, F32, dev_, E, rows));
+    if (op_sequence) {
+        for (Tensor *t : {&b.q, &b.k}) G_TRY(mk(t, F32, dev_, E, rows));
+        if (hp_.kv_f16) G_TRY(mk(&b.v, F32, dev_, E, rows));  // an f32 cache takes the values straight from the product
+    } else {  // heads of 128: q | k | v leave their products rotated, k and v go to the caches
+        G_TRY(mk(&b.pairs, F32, dev_, D, rows));
+    }
     G_TRY(mk(&b.qr, F32, dev_, D, H, rows));
     if (single_ropes && hp_.kv_f16) G_TRY(mk(&b.kr, F32, dev_, D, H, rows));
     if (op_sequence) {
@@ -279,10 +284,12 @@ GResult LlamaDecoder::prefill(const int32_t *tokens, size_t n, int32_t n_past) {
     {
         const size_t one[1] = {n}, en[2] = {E, n}, dhn[3] = {D, H, n}, dnh[3] = {D, n, H}, lnh[3] = {L, n, H};
         G_TRY(b.tok.view(0, 1, one, &tok));
-        G_TRY(b.pos.view(0, 1, one, &pos));
-        for (auto pr : {std::make_pair(&b.x, &x), std::make_pair(&b.x1, &x1), std::make_pair(&b.q, &q), std::make_pair(&b.k, &k)})
-            G_TRY(pr.first->view(0, 2, en, pr.second));
-        if (hp_.kv_f16) G_TRY(b.v.view(0, 2, en, &v));
+        for (auto pr : {std::make_pair(&b.x, &x), std::make_pair(&b.x1, &x1)}) G_TRY(pr.first->view(0, 2, en, pr.second));
+        if (D != 128) {
+            G_TRY(b.pos.view(0, 1, one, &pos));
+            for (auto pr : {std::make_pair(&b.q, &q), std::make_pair(&b.k, &k)}) G_TRY(pr.first->view(0, 2, en, pr.second));
+            if (hp_.kv_f16) G_TRY(b.v.view(0, 2, en, &v));
+        }
         G_TRY(b.qr.view(0, 3, dhn, &qr));
         if (hp_.kv_f16 && (D % 4 != 0 || D > 256)) G_TRY(b.kr.view(0, 3, dhn, &kr));
         if (D != 128) {
@@ -293,10 +300,12 @@ GResult LlamaDecoder::prefill(const int32_t *tokens, size_t n, int32_t n_past) {
             G_TRY(b.p.view(0, 3, lnh, &p));
         }
     }
-    std::vector<int32_t> positions(n);
-    for (size_t i = 0; i < n; i++) positions[i] = n_past + (int32_t)i;
     G_TRY(tok.write(tokens, n * sizeof(int32_t)));
-    G_TRY(pos.write(positions.data(), n * sizeof(int32_t)));
+    if (D != 128) {
+        std::vector<int32_t> positions(n);
+        for (size_t i = 0; i < n; i++) positions[i] = n_past + (int32_t)i;
+        G_TRY(pos.write(positions.data(), n * sizeof(int32_t)));
+    }
     last_token_ = last_pos_ = -1;  // the pass ends in buffers of the decode step (x_, a_, logits_): the next decode sets its inputs anew
 
     RopeCustomOption rope;
@@ -304,6 +313,9 @@ GResult LlamaDecoder::prefill(const int32_t *tokens, size_t n, int32_t n_past) {
     size_t ops = 0;
     const bool one_launch = D == 128;  // the attention of a layer as one call (galois_attn_prefill)
     const float attn_scale = 1.0f / sqrtf((float)D);
+    const float theta_scale = powf(rope.freq_base, -2.0f / (float)D);  // as galois_rope_custom derives it (src/cuda.rs:1327)
+    if (one_launch)  // every layer's rotations, once
+        G_TRY(dev_.gpu->check(galois_hip_rope_pairs(ctx, (float *)b.pairs.data(), (int32_t)n, n_past, rope.freq_scale, theta_scale)));
     G_TRY(galois_get_rows(tok_embd_, tok, x)); ops++;
     // the first layer's attention norm; every later one rides on the pass that adds the down projection's shares
     G_TRY(galois_rms_norm_mul_panel(x, layers_[0].attn_norm, b.panel_e, hp_.rms_eps)); ops++;
@@ -311,7 +323,7 @@ GResult LlamaDecoder::prefill(const int32_t *tokens, size_t n, int32_t n_past) {
         Layer &l = layers_[li];
         // attention block: (norm -> panel, above or at the end of the layer before) q | k | v in one launch
         Tensor q_heads, k_heads;
-        {
+        if (!one_launch) {
             const size_t dhn[3] = {D, H, n};
             G_TRY(q.view(0, 3, dhn, &q_heads));
             G_TRY(k.view(0, 3, dhn, &k_heads));
@@ -320,7 +332,12 @@ GResult LlamaDecoder::prefill(const int32_t *tokens, size_t n, int32_t n_past) {
         Tensor k_rows, v_rows;  // rows n_past .. n_past + n - 1 of both caches: one contiguous piece each
         G_TRY(l.k_cache.view(P * E, 2, en, &k_rows));
         G_TRY(l.v_cache.view(P * E, 2, en, &v_rows));
-        if (D % 4 == 0 && D <= 256) {
+        if (one_launch) {  // the products, both rotations and the append (counted as the two calls below)
+            G_TRY(dev_.gpu->check(galois_hip_mul_mat_q4_0_qkv_rope_f16_panel(
+                ctx, l.wq.data(), l.wk.data(), l.wv.data(), b.panel_e.data(), (const float *)b.pairs.data(), (float *)qr.data(), k_rows.data(),
+                v_rows.data(), hp_.kv_f16, (int32_t)D, (int32_t)H, (int32_t)E, (int32_t)n)));
+            ops += 2;
+        } else if (D % 4 == 0 && D <= 256) {
             // both rotations and the append in one launch; an f32 cache takes the values straight from the product
             if (!hp_.kv_f16) {
                 G_TRY(galois_matmul_panel({{&l.wq, &q}, {&l.wk, &k}, {&l.wv, &v_rows}}, b.panel_e, E, n));

@@ -460,6 +460,17 @@ int32_t galois_hip_rope_qk_append(galois_hip_ctx *ctx, const float *q, const flo
                                   void *v_rows, int32_t kv_f16, int32_t head_dim, int32_t n_head, int32_t n_tokens,
                                   const int32_t *pos, float freq_scale, float theta_scale);
 
+/* The three products q | k | v of a prefill on one panel (galois_hip_mul_mat_q4_0_f16_panel) and what
+ * galois_hip_rope_qk_append does behind them, in one launch: q receives the rotated queries [M][n_head * head_dim] f32,
+ * k_rows and v_rows the caches' rows of these tokens ([M][n_head * head_dim], f32 or, kv_f16, f16 rounded to nearest even
+ * from the f32 result).  The same bits as the two calls.  pairs: (cos, sin) of every token and pair of a head, as
+ * galois_hip_rope_pairs makes them for n_tokens consecutive positions from first_pos on ([n_tokens][64][2] floats, one launch
+ * for all layers of a pass).  head_dim 128, K % 256 == 0, 16-byte aligned operands. */
+int32_t galois_hip_rope_pairs(galois_hip_ctx *ctx, float *pairs, int32_t n_tokens, int32_t first_pos, float freq_scale, float theta_scale);
+int32_t galois_hip_mul_mat_q4_0_qkv_rope_f16_panel(galois_hip_ctx *ctx, const void *W_q, const void *W_k, const void *W_v,
+                                                   const void *panel, const float *pairs, float *q, void *k_rows, void *v_rows,
+                                                   int32_t kv_f16, int32_t head_dim, int32_t n_head, int32_t K, int32_t M);
+
 /* Causal attention of n_tokens query rows over a KV cache in ONE launch: what a prefill issues per layer as
  * cpy(q -> [D, M, H]), matmul(K^T, q), scale, soft_max under the causal mask, matmul(V, p), cpy(-> [D, H, M])
  * (CudaMatMul src/cuda.rs:867-992, scale and soft_max src/cuda.rs:1597-1663 and 1257-1356, cpy src/cuda.rs:1382-1595),
