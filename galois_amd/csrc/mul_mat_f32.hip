@@ -92,25 +92,27 @@ __global__ __launch_bounds__(kThreads) void mul_mat_f32_ncols(const AT *__restri
 // wave-load covers 64 / LPR rows, and a wave keeps U wave-loads in flight before it reduces any.
 // Rows are numbered with the batch index fastest when that is the smaller stride, so that the rows
 // of one wave-load (and of neighbouring waves) are neighbours in memory.
-template <int LPR, int U, typename AT>
+// IT: what rows are counted in; 32 bits wherever they suffice (16 heads of 64, 79 rows 5.3 -> 3.2 us: a 64-bit division is about a
+// hundred instructions, and a row took four).
+template <int LPR, int U, typename AT, typename IT>
 __global__ __launch_bounds__(kThreads) void mul_vec_f32_krows(const AT *__restrict__ a, const float *__restrict__ b,
                                                               float *__restrict__ dst, int N, int ne12, int r2,
                                                               int64_t a_s1, int64_t a_s2, int batch_fastest) {
     constexpr int RPL = 64 / LPR, K = LPR * 4;
     const int lane = threadIdx.x & 63;
     const int sub = lane / LPR, kl = lane % LPR;
-    const int64_t R = (int64_t)N * ne12;
-    const int64_t r0 = ((int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6)) * (RPL * U);
+    const IT R = (IT)N * (IT)ne12, per = batch_fastest ? (IT)ne12 : (IT)N;
+    const IT r0 = ((IT)blockIdx.x * (kThreads / 64) + (IT)(threadIdx.x >> 6)) * (RPL * U);
     if (r0 >= R) return;
     float4 av[U], bv[U];
     int64_t out[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const int64_t r = r0 + u * RPL + sub;
-        const int64_t rc = r < R ? r : R - 1;
-        const int64_t i2 = batch_fastest ? rc % ne12 : rc / N;
-        const int64_t n = batch_fastest ? rc / ne12 : rc % N;
-        av[u] = mm_ld4(a + (i2 / r2) * a_s2 + n * a_s1 + kl * 4);
+        const IT r = r0 + (IT)(u * RPL + sub);
+        const IT rc = r < R ? r : R - 1;
+        const IT hi = rc / per, lo = rc - hi * per;
+        const int64_t i2 = (int64_t)(batch_fastest ? lo : hi), n = (int64_t)(batch_fastest ? hi : lo);
+        av[u] = mm_ld4(a + (int64_t)((int)i2 / r2) * a_s2 + n * a_s1 + kl * 4);
         bv[u] = *reinterpret_cast<const float4 *>(b + i2 * K + kl * 4);
         out[u] = r < R ? i2 * N + n : -1;
     }
@@ -180,6 +182,56 @@ __global__ __launch_bounds__(kThreads) void mul_vec_f32_ncols(const AT *__restri
     }
 }
 
+// The same in one launch for a K of up to a few hundred rows: a workgroup of 16 waves owns 64 columns, a wave's request four
+// rows of them, 512 rows in flight; the waves meet in LDS.  Measured: see kOnceRows.
+template <typename AT>
+__global__ __launch_bounds__(1024) void mul_vec_f32_ncols_once(const AT *__restrict__ a, const float *__restrict__ b,
+                                                               float *__restrict__ dst, int K, int N, int C, int r2, int64_t a_s0, int64_t a_s2) {
+    __shared__ float red[16][64];
+    constexpr int U = 8;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane >> 4;
+    const int c = blockIdx.x * 64 + (lane & 15) * 4;
+    const int cc = c < C ? c : 0;  // C and N are multiples of 4: a lane's four columns stay in one batch slice
+    const int i2 = cc / N, n = cc - i2 * N;
+    const AT *ac = a + (int64_t)(i2 / r2) * a_s2 + n;
+    const float *bc = b + (int64_t)i2 * K;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int k0 = wave * 4 + sub; k0 - wave * 4 - sub < K; k0 += 64 * U) {
+        float4 v[U];
+        float p[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int kc = min(k0 + u * 64, K - 1);
+            v[u] = mm_ld4(ac + (int64_t)kc * a_s0);
+            p[u] = bc[kc];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (k0 + u * 64 < K) {
+                acc.x = __builtin_fmaf(v[u].x, p[u], acc.x);
+                acc.y = __builtin_fmaf(v[u].y, p[u], acc.y);
+                acc.z = __builtin_fmaf(v[u].z, p[u], acc.z);
+                acc.w = __builtin_fmaf(v[u].w, p[u], acc.w);
+            }
+    }
+#pragma unroll
+    for (int off = 16; off < 64; off <<= 1) {
+        acc.x += __shfl_xor(acc.x, off, 64);
+        acc.y += __shfl_xor(acc.y, off, 64);
+        acc.z += __shfl_xor(acc.z, off, 64);
+        acc.w += __shfl_xor(acc.w, off, 64);
+    }
+    if (sub == 0) *reinterpret_cast<float4 *>(&red[wave][lane * 4]) = acc;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        float s = red[0][lane];
+#pragma unroll
+        for (int w = 1; w < 16; w++) s += red[w][lane];
+        const int o = blockIdx.x * 64 + lane;
+        if (o < C) dst[o] = s;
+    }
+}
+
 // Second pass of the split product: adds the slabs in slab order.
 __global__ __launch_bounds__(kThreads) void sum_slabs_f32(const float *__restrict__ part, float *__restrict__ dst,
                                                           int C, int nslabs) {
@@ -202,8 +254,13 @@ void launch_vec_krows(galois_hip_ctx *ctx, const AT *a, const float *b, float *d
                       int64_t a_s1, int64_t a_s2) {
     constexpr int U = 8, rows_per_wg = (kThreads / 64) * (64 / LPR) * U;
     const int64_t R = (int64_t)N * ne12;
-    hipLaunchKernelGGL((mul_vec_f32_krows<LPR, U, AT>), dim3((unsigned)((R + rows_per_wg - 1) / rows_per_wg)),
-                       dim3(kThreads), 0, ctx->stream, a, b, dst, N, ne12, r2, a_s1, a_s2, (int)(a_s2 < a_s1));
+    const dim3 grid((unsigned)((R + rows_per_wg - 1) / rows_per_wg)), block(kThreads);
+    if (R + rows_per_wg < (int64_t)1 << 32)
+        hipLaunchKernelGGL((mul_vec_f32_krows<LPR, U, AT, uint32_t>), grid, block, 0, ctx->stream, a, b, dst, N, ne12, r2, a_s1, a_s2,
+                           (int)(a_s2 < a_s1));
+    else
+        hipLaunchKernelGGL((mul_vec_f32_krows<LPR, U, AT, int64_t>), grid, block, 0, ctx->stream, a, b, dst, N, ne12, r2, a_s1, a_s2,
+                           (int)(a_s2 < a_s1));
 }
 
 }  // namespace
@@ -223,6 +280,9 @@ namespace {
 // Rows of b from which the 32-row tiles of the f32 matrix-core kernel run.  us at 15 rows (scalar) / 16: a along k, 32 slices of
 // 600 x 128 20.7 / 7.4, one of 1024 x 1024 27.7 / 38.8 (one chain of long k, few tiles); along n 55.9 / 6.0 and 410 / 13.5.
 constexpr int kMfmaMinRows = 16;
+// Rows of V up to which V p is one launch (mul_vec_f32_ncols_once) rather than slabs and their sum.  us in two launches / one: 16
+// heads of 64, 79 rows 4.9 / 3.3, 512 5.6 / 3.9, 1024 5.9 / 5.9, 1500 6.7 / 8.2; 32 heads of 128 5.0 / 3.4, 6.1 / 4.4, 7.3 / 6.5, 8.6 / 8.8.
+constexpr int kOnceRows = 1024;
 
 template <typename AT>
 int32_t mul_mat_any(galois_hip_ctx *ctx, const AT *a, const float *b, float *dst, int32_t K, int32_t N, int32_t M,
@@ -267,7 +327,10 @@ int32_t mul_mat_any(galois_hip_ctx *ctx, const AT *a, const float *b, float *dst
         const int nslabs = (K + rows_per_wg - 1) / rows_per_wg;
         const bool fast = vec16 && gh_aligned(dst, 16) && a_s0 % 4 == 0 && N % 4 == 0 && tiles <= 65535 &&
                           (nslabs == 1 || (int64_t)nslabs * C <= GH_PARTIAL_FLOATS) && ctx->scratch != nullptr;
-        if (fast) {
+        if (fast && nslabs > 1 && K <= kOnceRows) {
+            hipLaunchKernelGGL(mul_vec_f32_ncols_once<AT>, dim3((unsigned)((C + 63) / 64)), dim3(1024), 0, ctx->stream, a, b, dst, K, N, (int)C,
+                               r2, a_s0, a_s2);
+        } else if (fast) {
             float *part = (float *)ctx->scratch;
             hipLaunchKernelGGL(mul_vec_f32_ncols<AT>, dim3((unsigned)tiles, nslabs), dim3(kThreads), 0, ctx->stream, a, b,
                                dst, part, K, N, (int)C, r2, a_s0, a_s2, rows_per_wave);
