@@ -88,6 +88,7 @@ PROTOTYPES = {
     "galois_hip_attn_prefill_f32": (i32, [c_ctx, vp, vp, vp, vp, vp, i32, i32, i32, i32, f32]),
     "galois_hip_attn_prefill_f16kv": (i32, [c_ctx, vp, vp, vp, vp, vp, i32, i32, i32, i32, f32]),
     "galois_hip_qkv_attn_decode_f16kv": (i32, [c_ctx, C.POINTER(GemvItem), vp, vp, vp, i32, i32, i32, vp, f32, f32, f32, i32]),
+    "galois_hip_store_i32_pair": (i32, [c_ctx, vp, i32, vp, i32]),
     "galois_hip_llama_step_workspace": (i32, [c_ctx, vp, C.POINTER(C.c_int64)]),
     "galois_hip_llama_step": (i32, [c_ctx, vp, i32, i32]),
     "galois_hip_qkv_attn_decode_launches": (i32, [c_ctx, i32, i32, i32, C.POINTER(i32)]),

@@ -145,7 +145,21 @@ int32_t launch_bcast(galois_hip_ctx *ctx, int op, const float *x, const float *y
 
 }  // namespace
 
+namespace {
+__global__ void store_i32_pair(int32_t *a, int32_t va, int32_t *b, int32_t vb) { *a = va, *b = vb; }
+}  // namespace
+
 extern "C" {
+
+int32_t galois_hip_store_i32_pair(galois_hip_ctx *ctx, int32_t *a, int32_t va, int32_t *b, int32_t vb) {
+    GH_REQUIRE_CTX(ctx);
+    GH_REQUIRE(ctx, a && b, GALOIS_HIP_E_NULL, "store_i32_pair");
+    GH_REQUIRE(ctx, gh_aligned(a, 4) && gh_aligned(b, 4), GALOIS_HIP_E_ALIGN, "store_i32_pair");
+    GH_BIND(ctx);
+    hipLaunchKernelGGL(store_i32_pair, dim3(1), dim3(1), 0, ctx->stream, a, va, b, vb);
+    GH_LAUNCH_CHECK(ctx, "store_i32_pair launch");
+}
+
 
 int32_t galois_hip_add_f32(galois_hip_ctx *ctx, const float *x, const float *y, float *dst, int64_t kx, int64_t ky) {
     return launch_bcast(ctx, EW_ADD, x, y, dst, kx, ky, "add_f32");

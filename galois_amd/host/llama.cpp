@@ -285,8 +285,8 @@ GResult LlamaDecoder::check_inputs(int32_t token, int32_t n_past) const {
 
 GResult LlamaDecoder::set_inputs(int32_t token, int32_t n_past) {
     G_TRY(check_inputs(token, n_past));
-    if (token != last_token_) G_TRY(tok_id_.write(&token, sizeof(token)));  // synchronous copies: only when they change
-    if (n_past != last_pos_) G_TRY(pos_.write(&n_past, sizeof(n_past)));
+    if (token != last_token_ || n_past != last_pos_)
+        G_TRY(dev_.gpu->check(galois_hip_store_i32_pair(dev_.gpu->ctx(), (int32_t *)tok_id_.data(), token, (int32_t *)pos_.data(), n_past)));
     last_token_ = token, last_pos_ = n_past;
     return GError{};
 }

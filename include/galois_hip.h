@@ -374,6 +374,10 @@ int32_t galois_hip_qkv_attn_decode_f16kv(galois_hip_ctx *ctx, const galois_hip_g
 /* How many launches such a call issues on this context (1 or 2): for these sizes, or as the option says. */
 int32_t galois_hip_qkv_attn_decode_launches(galois_hip_ctx *ctx, int32_t n_head, int32_t n_past, int32_t kv_f16, int32_t *n_launches);
 
+/* Two int32 values to two places on the device, in stream order and without a wait: the token and position of a decode step
+ * (two synchronous copies of four bytes take 29 us, this launch 3). */
+int32_t galois_hip_store_i32_pair(galois_hip_ctx *ctx, int32_t *a, int32_t va, int32_t *b, int32_t vb);
+
 /* A decode step of a LLaMA-architecture model -- embedding row, every layer's products, attention, norms and residual adds,
  * final norm and lm head -- in two launches (a deeper model than 40 layers: one more per 40), for a caller that would
  * otherwise issue galois_hip_get_rows_q4_0, galois_hip_qkv_attn_decode_* and galois_hip_dequantize_mul_mat_vec_q4_0_group
