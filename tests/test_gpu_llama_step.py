@@ -112,6 +112,37 @@ def test_steps_repeat_recorded_and_interleaved(gdev):
     dec.close()
 
 
+def test_two_contexts_on_two_threads():
+    """Steps of two contexts at once on one device: the workgroups of each wait only for their own, of lower index, so neither
+    keeps the other from finishing; the bits are those of a step alone."""
+    import threading
+    hp = dict(n_embd=2048, n_head=16, n_ff=5632, n_vocab=8000, n_layer=3, n_ctx=700)
+    devs = [g.Device.gpu(0) for _ in range(2)]
+    decs = [_decoder(d, seed=2 + i, kv_f16=bool(i), **hp)[0] for i, d in enumerate(devs)]
+    want, bad = [], []
+    for i, dec in enumerate(decs):
+        dec.decode(5 + i, 600 + i, 5)
+        want.append(dec.logits().copy())
+
+    def work(i):
+        try:
+            for _ in range(150):
+                decs[i].decode(5 + i, 600 + i, 5)
+                if not np.array_equal(decs[i].logits(), want[i]):
+                    bad.append(i)
+        except g.GError as e:
+            bad.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad[:3]
+    for dec in decs:
+        dec.close()
+
+
 def test_bad_arguments_are_refused_and_leave_the_decoder_usable(gdev):
     dec, hp = _decoder(gdev)
     dec.decode(9, 20, 5)
