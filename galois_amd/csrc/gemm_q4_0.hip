@@ -670,21 +670,29 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
         }
         return;
     }
-    // q | k | v: a pair of columns is a pair of neighbouring lanes, sixteen columns lie in one matrix.  The angles of four rows
-    // of every column tile are requested together (the operands' registers are free now).
+    // q | k | v: a pair of columns is a pair of neighbouring lanes, sixteen columns lie in one matrix.  The angles of a row tile
+    // are requested together, and the next one's before they are used (the operands' registers are free now).
     if (mats.rope != nullptr) {
         const bool odd = lane & 1;
         const int N = mats.N[0];
-#pragma unroll
-        for (int i = 0; i < RT; i++) {
+        float2 angles[2][NF][4];
+        auto request = [&](int i, float2(&cs)[NF][4]) {
             const int mb = m0 + wm * (16 * RT) + i * 16 + 4 * (lane >> 4);
-            float2 cs[NF][4];
 #pragma unroll
-            for (int j = 0; j < NF; j++)
+            for (int j = 0; j < NF; j++) {
+                if (n0 + ncol0 + j * 16 >= 2 * N) break;  // v is not rotated
 #pragma unroll
                 for (int e = 0; e < 4; e++)
                     cs[j][e] = mats.rope[(uint32_t)min(mb + e, M - 1) * 64u + (uint32_t)(((n0 + ncol0 + j * 16 + (lane & 15)) & 127) >> 1)];
+            }
+        };
+        request(0, angles[0]);
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            const int mb = m0 + wm * (16 * RT) + i * 16 + 4 * (lane >> 4);
+            if (i + 1 < RT) request(i + 1, angles[(i + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
+            const float2(&cs)[NF][4] = angles[i & 1];
 #pragma unroll
             for (int j = 0; j < NF; j++) {
                 const int n = n0 + ncol0 + j * 16, t = n / N;  // uniform
