@@ -525,7 +525,8 @@ __device__ __forceinline__ void gemm_drain_a(gemm_a_regs<RT> &r) {
 
 #define GEMM_LDB(dst, ptr) dst = *reinterpret_cast<const half8_t *>(ptr)
 #define GEMM_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0)
-template <int NF, int GN, int RT>
+// ROPE: the launch of q | k | v (mats.rope); a kernel of its own, so that the others keep their registers and code.
+template <int NF, int GN, int RT, bool ROPE>
 __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float16 *__restrict__ Xh,
                                               const gemm_mats &mats, int K, int M, int m0, int n0, int wm, int ncol0,
                                               int nslots, size_t y_off) {
@@ -672,7 +673,7 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
     }
     // q | k | v: a pair of columns is a pair of neighbouring lanes, sixteen columns lie in one matrix.  The angles of a row tile
     // are requested together, and the next one's before they are used (the operands' registers are free now).
-    if (mats.rope != nullptr) {
+    if constexpr (ROPE) {
         const bool odd = lane & 1;
         const int N = mats.N[0];
         float2 angles[2][NF][4];
@@ -745,7 +746,7 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
     }
 }
 
-template <int GN, int RT>
+template <int GN, int RT, bool ROPE>
 __global__ __launch_bounds__(512) void gemm_q4_0_mfma(const gemm_mats mats, const _Float16 *__restrict__ Xh, int K, int M,
                                                       int n_tiles, int m_tiles, int splits, size_t split_stride) {
     extern __shared__ __attribute__((aligned(16))) _Float16 smem[];  // [3] B stage | [2] raw | pad
@@ -765,7 +766,7 @@ __global__ __launch_bounds__(512) void gemm_q4_0_mfma(const gemm_mats mats, cons
     if (wave >= 4)
         gemm_producer<GN>(smem, mats, K, n0, sup0, sup1 - sup0);
     else  // four consumer waves stacked in M, each 16 * RT rows x GN columns; a piece of 256 is 8 KB of a row group's panel
-        gemm_consumer<GN / 16, GN, RT>(smem, Xh + (size_t)sup0 * 4096, mats, K, M, m0, n0, wave, 0, (sup1 - sup0) * 4,
+        gemm_consumer<GN / 16, GN, RT, ROPE>(smem, Xh + (size_t)sup0 * 4096, mats, K, M, m0, n0, wave, 0, (sup1 - sup0) * 4,
                                    (size_t)sp * split_stride);
 }
 
@@ -806,10 +807,11 @@ int32_t gemm_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *
     const size_t lds = gemm_cfg<GN>::LDS_BYTES;
     // the attribute lives with the function on the current device: set per launch (a table lookup), which is right
     // for every device and every thread without any flag of our own
-    hipError_t e = hipFuncSetAttribute((const void *)gemm_q4_0_mfma<GN, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    constexpr bool CAN_ROPE = GN != 64;  // q | k | v never come in shares
+    const auto kernel = CAN_ROPE && mats.rope != nullptr ? gemm_q4_0_mfma<GN, RT, CAN_ROPE> : gemm_q4_0_mfma<GN, RT, false>;
+    hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return gh_hip(ctx, e, "hipFuncSetAttribute(LDS size)");
-    hipLaunchKernelGGL((gemm_q4_0_mfma<GN, RT>), dim3(grid), dim3(512), lds, ctx->stream, mats, Xh, K, M, n_tiles, m_tiles, splits,
-                       split_stride);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds, ctx->stream, mats, Xh, K, M, n_tiles, m_tiles, splits, split_stride);
     return GALOIS_HIP_OK;
 }
 
