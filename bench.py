@@ -366,7 +366,7 @@ def decode_step_bench(dev, reps, with_graph=True, prefill_only=False):
         return res
     for name, fused in (("eager_one_kernel_per_op", 0), ("eager_fused_norm_and_silu", 1), ("eager_grouped_gemv", 2),
                         ("eager_grouped_gemv_fused_attention", 3), ("eager_split_norms", 4),
-                        ("eager_qkv_and_attention_in_one_call", 5)):
+                        ("eager_qkv_and_attention_in_one_call", 5)):  # this model: the whole step as one call
         dec.time_steps(tok, n_past, fused, SETTLE_STEPS)
         ms = min(dec.time_steps(tok, n_past, fused, reps) for _ in range(3)) / reps
         res[name] = {"library_calls": dec.ops_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1)}

@@ -9,12 +9,12 @@
 //   - v_mfma_f32_16x16x32_f16 adds over k in any order as long as both operands agree on it.  Lane (r, kg) of the
 //     weight operand therefore takes the whole 36-byte slot kg of the piece (two blocks of row r, as the
 //     decode kernel's lanes do): one piece = eight instructions, instruction (b, c) of which multiplies the eight weights k
-//     = 8c .. 8c+7 of block b of each lane's slot.  No shuffle, no LDS round trip, the block's scale is in the lane.
+//     = 8c .. 8c+7 of block b of each lane's slot.  No shuffle, the block's scale is in the lane.
 //   - The activation operand is then the 16-byte run c of row r in panel tile 2 kg + b: four contiguous 256-byte pieces a
 //     request, from L2 (every workgroup reads the whole panel: NT rows of tiles share a fragment).
 //   - The result tile has the weight rows down its registers: a lane holds four consecutive columns of Y.
 // Measured (MI355X, us, weights from HBM, against the 256-row tile): see SK_MAX_ROWS.  77 rows of a 3200 x 8640 matrix through
-// the f32 entry point 93 -> 19.8 (the generic kernel before), a prefill of 23 tokens through 32 layers 4705 -> 2871.
+// the f32 entry point 93 -> 17.6 (the generic kernel before), a prefill of 23 tokens through 32 layers 4705 -> 2505.
 // Weights are rounded exactly as in the main kernel ((q - 8) * d, once, to fp16), sums are f32.
 #pragma once
 

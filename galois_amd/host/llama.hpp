@@ -61,7 +61,8 @@ class LlamaDecoder {
     // token's.  n_embd and n_ff must be multiples of 256; caches [n_embd, n_ctx] (not head-major), f32 or f16.
     // Intermediates are sized for the largest n and n_past + n seen so far (this call allocates when they grow).
     GResult prefill(const int32_t *tokens, size_t n, int32_t n_past);
-    size_t ops_per_prefill() const { return n_prefill_ops_; }  // library calls of the last prefill (a call is one or two launches)
+    size_t ops_per_prefill() const { return n_prefill_ops_; }  // calls of the last prefill (one or two launches each; q | k | v that
+                                                               // leave their products rotated count as the two calls they stand for)
     const Tensor &logits() const { return logits_; }
     const LlamaHParams &hparams() const { return hp_; }
     size_t ops_per_step() const { return n_ops_; }  // calls the last decode step's plan consists of (a call is one or two launches; plan 5 may send
