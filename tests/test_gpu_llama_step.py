@@ -9,7 +9,7 @@ from galois_amd import host_api as g
 
 pytestmark = pytest.mark.gpu
 
-BASE = dict(n_vocab=515, n_embd=256, n_head=2, n_layer=2, n_ff=512, n_ctx=160, rms_eps=1e-6, freq_base=10000.0)
+BASE = dict(n_vocab=515, n_embd=512, n_head=4, n_layer=2, n_ff=512, n_ctx=160, rms_eps=1e-6, freq_base=10000.0)
 # both plans round activations to 18 bits of their block and add f32 in other orders: 1e-5 a product, a few of them a layer;
 # an f16 cache row may differ by a unit in the last place where that falls on the other side (2^-11 of one element)
 TOL = {False: 1e-4, True: 4e-4}
@@ -63,13 +63,14 @@ def _row(dec, hp, name, layer, n_past):
     (dict(), (0, 1, 126, 127, 128, 159)),                                        # f32: one split of 128 keys, two
     (dict(kv_f16=True, n_ctx=530), (0, 254, 255, 256, 511, 512, 529)),           # f16: 256 keys a split
     (dict(kv_head_major=True, n_ctx=300), (5, 299)),
-    (dict(n_embd=128, n_head=1, n_ff=64, n_vocab=1), (3,)),                      # the smallest: one slot in down
+    (dict(n_ff=64, n_vocab=1), (3,)),                                            # the smallest: one slot in down
     (dict(n_embd=1664, n_head=13, n_ff=4096, n_vocab=48), (130,)),               # 35 workgroups of 48 rows: 16 over; one chunk
     (dict(n_embd=1024, n_head=8, n_ff=4160, n_vocab=49), (40,)),                 # two chunks, one slot in the second
-    (dict(n_embd=384, n_head=3, n_ff=8256, n_vocab=2000), (60,)),                # three chunks, one slot in the third
+    (dict(n_embd=640, n_head=5, n_ff=8256, n_vocab=2000), (60,)),                # three chunks, one slot in the third
     (dict(n_embd=4096, n_head=32, n_ff=12288, n_layer=1), (100,)),               # the widest
-    (dict(n_head=1, n_embd=128, n_layer=41), (17,)),                             # 41 layers: two launches
-    (dict(n_embd=128, n_head=1, n_ctx=8300), (8190, 8191, 8192)),                # 64 splits of keys; beyond: layer by layer
+    (dict(n_layer=41), (17,)),                                                   # 41 layers: two launches
+    (dict(n_ctx=8300), (8190, 8191, 8192)),                                      # 64 splits of keys; beyond: layer by layer
+    (dict(n_embd=384, n_head=3), (60,)),                                         # narrower than 512: layer by layer
     (dict(n_embd=4224, n_head=33, n_ff=512, n_layer=1), (9,)),                   # wider: layer by layer
 ])
 def test_step_equals_the_launches_it_replaces(gdev, kw, positions):
