@@ -26,6 +26,19 @@ class GemmItem(C.Structure):
     _fields_ = [("W", vp), ("Y", vp), ("N", i32), ("reserved", i32)]
 
 
+class LlamaLayer(C.Structure):
+    """galois_hip_llama_layer of include/galois_hip.h, field for field."""
+    _fields_ = [(n, vp) for n in ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down", "attn_norm", "ffn_norm", "k_cache", "v_cache")]
+
+
+class LlamaModel(C.Structure):
+    """galois_hip_llama_model of include/galois_hip.h, field for field."""
+    _fields_ = ([(n, i32) for n in ("n_embd", "n_head", "n_ff", "n_vocab", "n_layer", "n_ctx", "kv_f16", "head_major_n_ctx")] +
+                [(n, f32) for n in ("rms_eps", "freq_scale", "theta_scale", "scale")] +
+                [(n, vp) for n in ("tok_embd", "output", "out_norm", "logits", "token", "pos")] +
+                [("layers", C.POINTER(LlamaLayer)), ("workspace", vp), ("workspace_bytes", C.c_int64)])
+
+
 # name -> (restype, argtypes); must list every function the header declares
 PROTOTYPES = {
     "galois_hip_abi_version": (i32, []),

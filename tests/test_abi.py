@@ -115,6 +115,38 @@ def test_rust_binding_block_matches_the_header():
     assert c_fields == rust_fields
 
 
+def _struct_fields(body, rust):
+    """[(name, class)] of a struct's body: the C one's declarators, or the Rust one's `pub name: type`."""
+    body = re.sub(r"/\*.*?\*/|//[^\n]*", "", body, flags=re.S)
+    if rust:
+        known = {"i32": "i32", "i64": "i64", "f32": "f32"}
+        pairs = [f.split(":", 1) for f in body.split(",") if ":" in f]
+        return [(n.replace("pub", "").strip(), "ptr" if t.strip().startswith("*") else known[t.strip()]) for n, t in pairs]
+    out = []
+    for decl in filter(None, (d.strip() for d in body.split(";"))):
+        words = re.sub(r"\bconst\b", "", decl).split(None, 1)
+        for n in words[1].split(","):
+            out.append((n.replace("*", "").strip(), "ptr" if "*" in n else {"int32_t": "i32", "int64_t": "i64", "float": "f32"}[words[0]]))
+    return out
+
+
+@pytest.mark.parametrize("c_name, rust_name, ctype", [
+    ("galois_hip_llama_layer", "GaloisHipLlamaLayer", _abi.LlamaLayer), ("galois_hip_llama_model", "GaloisHipLlamaModel", _abi.LlamaModel)])
+def test_structs_of_the_whole_step_agree_in_all_three_languages(tmp_path, c_name, rust_name, ctype):
+    """Names, order and types in the header, in the Rust block and in ctypes; sizes and offsets as the C compiler lays them out."""
+    header, notes = open(HEADER).read(), open(os.path.join(ROOT, "INTEGRATION.md")).read()
+    c = _struct_fields(re.search(r"typedef struct %s \{(.*?)\n\}" % c_name, header, flags=re.S).group(1), False)
+    rust = _struct_fields(re.search(r"pub struct %s \{(.*?)\n\}" % rust_name, notes, flags=re.S).group(1), True)
+    assert c == rust == [(n, _ctypes_class(t)) for n, t in ctype._fields_]
+    src = tmp_path / "layout.c"
+    src.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "galois_hip.h"\nint main(void) {\n' +
+                   "".join('printf("%%zu ", offsetof(%s, %s));\n' % (c_name, n) for n, _ in c) +
+                   'printf("%%zu", sizeof(%s));\nreturn 0;\n}\n' % c_name)
+    subprocess.check_call(["gcc", "-Wall", "-Werror", "-I", os.path.join(ROOT, "include"), str(src), "-o", str(tmp_path / "layout")])
+    got = [int(t) for t in subprocess.check_output([str(tmp_path / "layout")], text=True).split()]
+    assert got == [getattr(ctype, n).offset for n, _ in c] + [C.sizeof(ctype)]
+
+
 def test_status_strings_without_device():
     lib = _abi.load()
     assert lib.galois_hip_status_string(0) == b"ok"
