@@ -770,6 +770,8 @@ extern "C" int32_t galois_hip_llama_step(galois_hip_ctx *ctx, const galois_hip_l
     ds_shape s;
     GH_REQUIRE(ctx, ds_plan(m, s), GALOIS_HIP_E_UNSUPPORTED, "llama_step: heads of 128, n_embd up to 4096, n_ff a multiple of 64 up to 12288, up to 250 layers");
     GH_REQUIRE(ctx, n_past >= 0 && n_past < m->n_ctx && token < m->n_vocab, GALOIS_HIP_E_SHAPE, "llama_step: token below n_vocab, n_past below n_ctx");
+    GH_REQUIRE(ctx, m->head_major_n_ctx == 0 || m->head_major_n_ctx > n_past, GALOIS_HIP_E_SHAPE,
+               "llama_step: head_major_n_ctx is 0 or the capacity of a [n_head][n_ctx][128] cache, above n_past");
     GH_REQUIRE(ctx, m->workspace_bytes >= s.bytes, GALOIS_HIP_E_SHAPE, "llama_step: workspace of galois_hip_llama_step_workspace bytes");
     GH_REQUIRE(ctx, ctx->qkv_attn_launches == 0, GALOIS_HIP_E_UNSUPPORTED, "llama_step: a form of qkv_attn_decode is asked for");
     GH_REQUIRE(ctx, n_past / s.keys < s.S_max, GALOIS_HIP_E_UNSUPPORTED, "llama_step: at most 64 splits of the keys (of 128 in f32, 256 in f16)");

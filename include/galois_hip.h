@@ -398,7 +398,7 @@ typedef struct galois_hip_llama_layer {
 } galois_hip_llama_layer;
 typedef struct galois_hip_llama_model {
     int32_t n_embd, n_head, n_ff, n_vocab, n_layer, n_ctx;
-    int32_t kv_f16, head_major_n_ctx; /* as the attention calls take them */
+    int32_t kv_f16, head_major_n_ctx; /* as the attention calls take them: 0, or the capacity of a head's rows, above n_past */
     float rms_eps, freq_scale, theta_scale, scale;
     const void *tok_embd, *output;    /* Q4_0 [n_vocab][n_embd] */
     const float *out_norm;
