@@ -5,6 +5,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <mutex>
 #include <vector>
 
 #include "../../include/galois_hip.h"
@@ -29,6 +30,9 @@ struct galois_hip_ctx {
     int32_t wait_target_bias;  // added to the count such a wait waits for: test hook (GALOIS_HIP_OPT_WAIT_TARGET_BIAS)
     int32_t qkv_attn_launches; // 1 or 2: the form of qkv_attn_decode whatever the sizes (GALOIS_HIP_OPT_QKV_ATTN_LAUNCHES)
     bool gemv_f32;             // GALOIS_HIP_OPT_GEMV_F32_ARITHMETIC: one-product GEMV in the reference's f32 arithmetic
+    hipEvent_t order_ev;  // gh_order: recorded behind this context's last launch whose workgroups wait for one another, ...
+    bool order_open;      // ... unless one has gone out since
+    bool capture_waits;   // the capture that is open holds such a launch
     bool capturing;   // between graph_begin_capture and graph_end_capture: nothing may allocate or block
     char last_error[256];
 };
@@ -36,7 +40,9 @@ struct galois_hip_ctx {
 // galois_hip_ctx::scratch holds GH_PARTIAL_FLOATS floats of partial sums.
 constexpr int64_t GH_PARTIAL_FLOATS = 1 << 20;
 constexpr int64_t GH_ATTN_HEADS = 65536;
-constexpr int32_t GH_WAIT_SPIN_DEFAULT = 1 << 20;  // polls of a bounded in-launch wait (a poll and its sleep take about a microsecond)
+// Polls of a bounded in-launch wait.  A poll takes 0.6 us or more (a load past the caches; the attention's and its sleep about one):
+// a wait gives up after most of a second at the earliest.
+constexpr int32_t GH_WAIT_SPIN_DEFAULT = 1 << 20;
 
 struct galois_hip_event {
     hipEvent_t ev;
@@ -45,6 +51,7 @@ struct galois_hip_event {
 struct galois_hip_graph {
     hipGraph_t graph;
     hipGraphExec_t exec;
+    bool waits;  // holds a launch that gh_order is for
 };
 
 // Q4_0 block exactly as the reference stores it (src/ggml_quants.rs:140-145).
@@ -96,6 +103,21 @@ size_t gh_block_bytes(int32_t n_cu);
 
 // device.hip: after a wait for the stream, reports (and clears) what kernels left in the context's status word.
 int32_t gh_check_device_status(galois_hip_ctx *ctx);
+
+// device.hip: held around a launch whose workgroups wait for one another inside it (galois_hip_llama_step, the one-launch form of
+// galois_hip_qkv_attn_decode_*).  Such a wait ends because the workgroups of a launch are placed in the order of their index on every
+// XCD, unless what holds the places of an XCD waits as well: of two such grids on one device each may fill XCDs that the other's
+// awaited workgroups are dealt to.  So those of one context follow, on the device, those that another context has sent out before
+// (within a process).  Until a second context sends one out no event is recorded: a program with one pays a lock that nobody holds.
+class gh_order {
+    galois_hip_ctx *ctx_;
+    std::unique_lock<std::mutex> lock_;
+
+   public:
+    int32_t status;  // the launch may go out
+    explicit gh_order(galois_hip_ctx *ctx);
+    void launched();
+};
 
 // attn_decode.hip: looks up the device's copy of the attention's static scratch (the context's device is current).
 int32_t gh_attn_static_init(galois_hip_ctx *ctx);

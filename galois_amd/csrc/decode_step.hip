@@ -12,10 +12,13 @@
 // and that registers hold 55 MB of a layer's 115 to 180.  Measured, us a layer of 4096 / 11008, 32 heads (four launches / this):
 // 2045 f32 keys 52 / 43, 201 f16 keys 42 / 34; of 1024 / 2816, 8 heads, 78 f32 keys 22 / 15.
 //
-// No deadlock: a workgroup waits only for workgroups of lower index, and those are handed out first, so the unfinished
-// workgroup of the lowest index never waits for one that is not running, whatever else runs on the device.  Waits are
-// bounded all the same; one that runs out makes the logits NaN and sets the context's status word, and every later wait
-// of the launch gives up at once.
+// Why the waits end: a workgroup waits only for workgroups of lower index, and each XCD places the workgroups dealt to it (index
+// mod 8) in their order, so the unfinished workgroup of the lowest index runs, or has its place as soon as what holds it ends.
+// That is how the dispatcher behaves, no promise of the programming model; and it takes that what else holds places does not
+// wait in turn for a place this grid holds: grids that do (gh_order) follow one another where they are of one process.
+// Two processes that both send such grids to one device are not ordered.  The waits are bounded for these cases, and for a kernel of
+// others that holds an XCD for longer: one that runs out makes the logits NaN and sets the context's status word, and every
+// later wait of the launch gives up at once.
 //
 // Vectors between stages are pairs {f32 value, tag}, stored as 8 bytes with device scope.  The tag names the step and
 // the layer, so a reader knows from the element itself whether it is the one it waits for: no producer waits for its
@@ -806,6 +809,8 @@ extern "C" int32_t galois_hip_llama_step(galois_hip_ctx *ctx, const galois_hip_l
     a.key_stride = m->head_major_n_ctx ? DS_D : E;
     a.head_stride = m->head_major_n_ctx ? (int64_t)m->head_major_n_ctx * DS_D : DS_D;
     const size_t lds = (size_t)(E > F ? E : F) / 64 * slot_lds<DS_L>::bytes_per_slot;
+    gh_order order(ctx);
+    if (order.status != GALOIS_HIP_OK) return order.status;
     hipLaunchKernelGGL(decode_step_begin, dim3(1), dim3(1024), 0, ctx->stream, (const uint16_t *)m->tok_embd, E, m->n_vocab, a.head, m->token,
                        m->pos, token, n_past, a.x);
     for (int32_t first = 0; first < m->n_layer; first += DS_MAX_LAYERS) {
@@ -822,5 +827,6 @@ extern "C" int32_t galois_hip_llama_step(galois_hip_ctx *ctx, const galois_hip_l
         else
             ds_launch<float>(a, s, blocks, lds, ctx->stream);
     }
+    order.launched();
     GH_LAUNCH_CHECK(ctx, "llama_step launch");
 }

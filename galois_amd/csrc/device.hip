@@ -2,6 +2,62 @@
 // obtains from cudarc).  One context = one device ordinal + one stream.
 #include "common.h"
 
+#include <map>
+
+namespace {
+
+// Per device: the context that sent out the last launch gh_order is for.
+struct order_state {
+    std::mutex mu;
+    galois_hip_ctx *last = nullptr;
+    bool shared = false;  // it has changed: the event is recorded behind every such launch, so that others wait for no more than that
+};
+order_state &order_of(int32_t ordinal) {
+    static std::mutex mu;
+    static std::map<int32_t, order_state> *all = new std::map<int32_t, order_state>;  // for as long as contexts may live
+    std::lock_guard<std::mutex> g(mu);
+    return (*all)[ordinal];
+}
+hipError_t order_record(galois_hip_ctx *ctx) {  // under the device's lock
+    if (!ctx->order_open) return hipSuccess;
+    const hipError_t e = hipEventRecord(ctx->order_ev, ctx->stream);
+    if (e == hipSuccess) ctx->order_open = false;
+    return e;
+}
+// Where nothing can be recorded on the context's stream or waited for on it any more (a capture opens, the context goes): if
+// its launch is the last of the device, it is waited for here.
+hipError_t order_drain(galois_hip_ctx *ctx) {
+    order_state &s = order_of(ctx->ordinal);
+    std::lock_guard<std::mutex> g(s.mu);
+    if (s.last != ctx) return hipSuccess;
+    s.last = nullptr, ctx->order_open = false;
+    return hipStreamSynchronize(ctx->stream);
+}
+
+}  // namespace
+
+gh_order::gh_order(galois_hip_ctx *ctx) : ctx_(ctx), status(GALOIS_HIP_OK) {
+    if (ctx->capturing) return;  // ordered when the graph is launched
+    order_state &s = order_of(ctx->ordinal);
+    lock_ = std::unique_lock<std::mutex>(s.mu);
+    if (s.last == nullptr || s.last == ctx) return;
+    s.shared = true;
+    hipError_t e = order_record(s.last);
+    if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, s.last->order_ev, 0);
+    status = gh_hip(ctx, e, "waiting for another context's launch");
+}
+
+void gh_order::launched() {
+    if (ctx_->capturing) {
+        ctx_->capture_waits = true;
+        return;
+    }
+    order_state &s = order_of(ctx_->ordinal);
+    ctx_->order_open = true;
+    s.last = ctx_;
+    if (s.shared) (void)order_record(ctx_);  // else whoever waits for it records it
+    lock_.unlock();
+}
 
 // Called once the stream has drained.  A kernel whose bounded wait for other workgroups of its launch ran out has
 // set the context's status word (and poisoned its own result with NaN); the workgroups it gave up on may have counted
@@ -81,8 +137,15 @@ int32_t galois_hip_create(int32_t ordinal, galois_hip_ctx **out) {
     ctx->wait_target_bias = 0;
     ctx->qkv_attn_launches = 0;
     ctx->gemv_f32 = false;
+    ctx->order_open = ctx->capture_waits = false;
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
+        delete ctx;
+        return (int32_t)e;
+    }
+    e = hipEventCreateWithFlags(&ctx->order_ev, hipEventDisableTiming);
+    if (e != hipSuccess) {
+        (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return (int32_t)e;
     }
@@ -108,6 +171,7 @@ int32_t galois_hip_create(int32_t ordinal, galois_hip_ctx **out) {
         if (ctx->attn_done) (void)hipFree(ctx->attn_done);
         if (ctx->block) (void)hipFree(ctx->block);
         if (ctx->dev_status) (void)hipHostFree(ctx->dev_status);
+        (void)hipEventDestroy(ctx->order_ev);
         (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return (int32_t)e;
@@ -119,7 +183,9 @@ int32_t galois_hip_create(int32_t ordinal, galois_hip_ctx **out) {
 int32_t galois_hip_destroy(galois_hip_ctx *ctx) {
     GH_REQUIRE_CTX(ctx);
     (void)hipSetDevice(ctx->ordinal);
+    (void)order_drain(ctx);
     (void)hipStreamSynchronize(ctx->stream);
+    (void)hipEventDestroy(ctx->order_ev);
     if (ctx->ws) (void)hipFree(ctx->ws);
     for (void *p : ctx->ws_retired) (void)hipFree(p);
     if (ctx->scratch) (void)hipFree(ctx->scratch);
@@ -311,8 +377,9 @@ int32_t galois_hip_graph_begin_capture(galois_hip_ctx *ctx) {
     GH_REQUIRE_CTX(ctx);
     GH_REQUIRE(ctx, !ctx->capturing, GALOIS_HIP_E_UNSUPPORTED, "graph_begin_capture: a capture is already open");
     GH_BIND(ctx);
-    hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess) ctx->capturing = true;
+    hipError_t e = order_drain(ctx);
+    if (e == hipSuccess) e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
+    if (e == hipSuccess) ctx->capturing = true, ctx->capture_waits = false;
     return gh_hip(ctx, e, "hipStreamBeginCapture");
 }
 
@@ -333,7 +400,7 @@ int32_t galois_hip_graph_end_capture(galois_hip_ctx *ctx, galois_hip_graph **out
         return gh_hip(ctx, e, "hipGraphInstantiate");
     }
     galois_hip_graph *gr = new galois_hip_graph();
-    gr->graph = g, gr->exec = x;
+    gr->graph = g, gr->exec = x, gr->waits = ctx->capture_waits;
     *out = gr;
     return GALOIS_HIP_OK;
 }
@@ -343,7 +410,12 @@ int32_t galois_hip_graph_launch(galois_hip_ctx *ctx, galois_hip_graph *graph) {
     GH_REQUIRE(ctx, graph != nullptr, GALOIS_HIP_E_NULL, "graph_launch");
     GH_REQUIRE(ctx, !ctx->capturing, GALOIS_HIP_E_UNSUPPORTED, "graph_launch inside a capture");
     GH_BIND(ctx);
-    return gh_hip(ctx, hipGraphLaunch(graph->exec, ctx->stream), "hipGraphLaunch");
+    if (!graph->waits) return gh_hip(ctx, hipGraphLaunch(graph->exec, ctx->stream), "hipGraphLaunch");
+    gh_order order(ctx);
+    if (order.status != GALOIS_HIP_OK) return order.status;
+    const hipError_t e = hipGraphLaunch(graph->exec, ctx->stream);
+    order.launched();
+    return gh_hip(ctx, e, "hipGraphLaunch");
 }
 
 int32_t galois_hip_graph_destroy(galois_hip_ctx *ctx, galois_hip_graph *graph) {

@@ -843,6 +843,8 @@ int32_t launch_qkv_attn(galois_hip_ctx *ctx, const galois_hip_gemv_item *items, 
     constexpr int PGMAX = (kChunkSlots * 8 + FA_WAVES * 64 - 1) / (FA_WAVES * 64);
     const bool short_vec = plan.max_slots <= 64;
     if (plan.mode == 1 && short_vec) lds += (size_t)plan.max_slots * 64 * sizeof(float);  // staged, weighted activations
+    gh_order order(ctx);
+    if (order.status != GALOIS_HIP_OK) return order.status;
 #define FA_LAUNCH(PG_, MODE_) \
     hipLaunchKernelGGL((qkv_attn_decode_fused<PG_, MODE_, CT>), grid, block, lds, ctx->stream, a, b)
     if (short_vec) {
@@ -855,6 +857,7 @@ int32_t launch_qkv_attn(galois_hip_ctx *ctx, const galois_hip_gemv_item *items, 
         else FA_LAUNCH(PGMAX, 2);
     }
 #undef FA_LAUNCH
+    order.launched();
     GH_LAUNCH_CHECK(ctx, what);
 }
 

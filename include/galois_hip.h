@@ -389,8 +389,11 @@ int32_t galois_hip_store_i32_pair(galois_hip_ctx *ctx, int32_t *a, int32_t va, i
  *     between their stages -- one such block per model in flight; 0 if the step is not one this call takes.
  *   token >= 0: the token to decode and its position n_past, which are also stored to model->token and model->pos.
  *   token < 0: the token and the rotation's position are read from there when the launch runs (a recorded step).
- * The stages of the step wait for one another inside the launch, with bounded waits: should one run out, the logits are
- * NaN and the next synchronize or *_sync_copy returns GALOIS_HIP_E_DEVICE_WAIT (once). */
+ * The stages of the step wait for one another inside the launch, with bounded waits: should one run out (a kernel of others
+ * that keeps the launch from an eighth of the device for most of a second, or such launches of two processes that hold each
+ * other's places), the logits are NaN and the next synchronize or *_sync_copy returns GALOIS_HIP_E_DEVICE_WAIT (once).  Steps
+ * of several contexts of one process on one device (and the one-launch form of galois_hip_qkv_attn_decode_*) run one after the
+ * other on the device, in the order of the calls; so do graphs that hold them. */
 typedef struct galois_hip_llama_layer {
     const void *wq, *wk, *wv, *wo, *w_gate, *w_up, *w_down; /* Q4_0 */
     const float *attn_norm, *ffn_norm;
