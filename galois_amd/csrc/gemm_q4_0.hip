@@ -808,6 +808,7 @@ int32_t gemm_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *
     // the attribute lives with the function on the current device: set per launch (a table lookup), which is right
     // for every device and every thread without any flag of our own
     constexpr bool CAN_ROPE = GN != 64;  // q | k | v never come in shares
+    GH_REQUIRE(ctx, CAN_ROPE || mats.rope == nullptr, GALOIS_HIP_E_UNSUPPORTED, "matmul: no rotation behind tiles of 64 columns");
     const auto kernel = CAN_ROPE && mats.rope != nullptr ? gemm_q4_0_mfma<GN, RT, CAN_ROPE> : gemm_q4_0_mfma<GN, RT, false>;
     hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return gh_hip(ctx, e, "hipFuncSetAttribute(LDS size)");
