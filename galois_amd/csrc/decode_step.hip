@@ -743,12 +743,13 @@ bool ds_plan(const galois_hip_llama_model *m, ds_shape &s) {
 }
 
 template <typename CT>
-void ds_launch(const ds_args &a, const ds_shape &s, unsigned blocks, size_t lds, hipStream_t stream) {
+hipError_t ds_launch(const ds_args &a, const ds_shape &s, unsigned blocks, size_t lds, hipStream_t stream) {
 #define DS_GO(RD_, NCHD_)                                                                                                        \
     do {                                                                                                                         \
-        (void)hipFuncSetAttribute((const void *)decode_step<CT, RD_, NCHD_>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                  (int)lds);                                                                                     \
-        hipLaunchKernelGGL((decode_step<CT, RD_, NCHD_>), dim3(blocks), dim3(DS_THREADS), lds, stream, a);           \
+        const hipError_t e = hipFuncSetAttribute((const void *)decode_step<CT, RD_, NCHD_>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+        if (e != hipSuccess) return e;                                                                                           \
+        hipLaunchKernelGGL((decode_step<CT, RD_, NCHD_>), dim3(blocks), dim3(DS_THREADS), lds, stream, a);                       \
+        return hipGetLastError();                                                                                                \
     } while (0)
     if (s.nchd == 1) DS_GO(4, 1);
     else if (s.nchd == 2) DS_GO(2, 2);
@@ -813,7 +814,8 @@ extern "C" int32_t galois_hip_llama_step(galois_hip_ctx *ctx, const galois_hip_l
     if (order.status != GALOIS_HIP_OK) return order.status;
     hipLaunchKernelGGL(decode_step_begin, dim3(1), dim3(1024), 0, ctx->stream, (const uint16_t *)m->tok_embd, E, m->n_vocab, a.head, m->token,
                        m->pos, token, n_past, a.x);
-    for (int32_t first = 0; first < m->n_layer; first += DS_MAX_LAYERS) {
+    hipError_t e = hipGetLastError();
+    for (int32_t first = 0; first < m->n_layer && e == hipSuccess; first += DS_MAX_LAYERS) {
         const int32_t n = m->n_layer - first < DS_MAX_LAYERS ? m->n_layer - first : DS_MAX_LAYERS;
         for (int32_t i = 0; i < n; i++) {
             const galois_hip_llama_layer &y = m->layers[first + i];
@@ -822,11 +824,8 @@ extern "C" int32_t galois_hip_llama_step(galois_hip_ctx *ctx, const galois_hip_l
         }
         a.first_layer = first, a.n_layers = n;
         const unsigned blocks = (unsigned)n * (unsigned)a.b_layer + (first + n == m->n_layer ? (unsigned)wgs(a.V, DS_RW) : 0u);
-        if (m->kv_f16)
-            ds_launch<_Float16>(a, s, blocks, lds, ctx->stream);
-        else
-            ds_launch<float>(a, s, blocks, lds, ctx->stream);
+        e = m->kv_f16 ? ds_launch<_Float16>(a, s, blocks, lds, ctx->stream) : ds_launch<float>(a, s, blocks, lds, ctx->stream);
     }
     order.launched();
-    GH_LAUNCH_CHECK(ctx, "llama_step launch");
+    return gh_hip(ctx, e, "llama_step launch");
 }
