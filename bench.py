@@ -349,11 +349,11 @@ def decode_step_bench(dev, reps, with_graph=True, prefill_only=False):
         q4_flop = 2.0 * n_tok * hp["n_layer"] * (4 * e * e + 3 * e * f)
         attn_flop = 2.0 * 2 * n_tok * n_tok * e * hp["n_layer"]     # scores and out over all n_tok keys (the masked half too)
         if not compare:
-            return {"tokens": n_tok, "library_calls": dec.ops_per_prefill(), "ms": round(ms, 3), "tokens_per_s": round(n_tok / ms * 1e3, 0),
+            return {"tokens": n_tok, "library_calls": dec.calls_per_prefill(), "ms": round(ms, 3), "tokens_per_s": round(n_tok / ms * 1e3, 0),
                     "q4_0_flop_over_the_whole_pass_TFLOPs": round(q4_flop / ms / 1e9, 1),
                     "q4_0_flop_over_the_whole_pass_mfma_frac": round(q4_flop / ms / 1e9 / MFMA_F16_PEAK_TFLOPS, 4),
                     "logits_finite": bool(np.all(np.isfinite(got)))}
-        return {"tokens": n_tok, "library_calls": dec.ops_per_prefill(), "ms": round(ms, 3), "tokens_per_s": round(n_tok / ms * 1e3, 0),
+        return {"tokens": n_tok, "library_calls": dec.calls_per_prefill(), "ms": round(ms, 3), "tokens_per_s": round(n_tok / ms * 1e3, 0),
                 "q4_0_flop_over_the_whole_pass_TFLOPs": round(q4_flop / ms / 1e9, 1),
                 "q4_0_flop_over_the_whole_pass_mfma_frac": round(q4_flop / ms / 1e9 / MFMA_F16_PEAK_TFLOPS, 4),
                 "q4_0_flop": q4_flop, "attention_flop": attn_flop,
@@ -366,21 +366,21 @@ def decode_step_bench(dev, reps, with_graph=True, prefill_only=False):
         return res
     for name, fused in (("eager_one_kernel_per_op", 0), ("eager_fused_norm_and_silu", 1), ("eager_grouped_gemv", 2),
                         ("eager_grouped_gemv_fused_attention", 3), ("eager_split_norms", 4),
-                        ("eager_qkv_and_attention_in_one_call", 5)):  # this model: the whole step as one call
+                        ("eager_whole_step_in_one_grid", 5)):
         dec.time_steps(tok, n_past, fused, SETTLE_STEPS)
         ms = min(dec.time_steps(tok, n_past, fused, reps) for _ in range(3)) / reps
-        res[name] = {"library_calls": dec.ops_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1)}
+        res[name] = {"library_calls": dec.calls_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1)}
         plan_logits[fused] = dec.logits().astype(np.float64)
     if not with_graph:
         res["prefill_512_tokens"] = prefill(dec)
         dec.close()
         return res
     graph_logits = {}
-    for name, fused in (("hip_graph_split_norms", 4), ("hip_graph_qkv_and_attention_in_one_call", 5)):
+    for name, fused in (("hip_graph_split_norms", 4), ("hip_graph_whole_step_in_one_grid", 5)):
         dec.capture(tok, n_past, fused)
         dec.time_replays(SETTLE_STEPS)
         ms = min(dec.time_replays(reps) for _ in range(3)) / reps
-        res[name] = {"library_calls": dec.ops_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1),
+        res[name] = {"library_calls": dec.calls_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1),
                      "GBps": round((weight_bytes + kv_bytes) / ms / 1e6, 1),
                      "hbm_frac": round((weight_bytes + kv_bytes) / ms / 1e6 / HBM_PEAK_GBPS, 4)}
         graph_logits[name] = dec.logits().astype(np.float64)
@@ -391,7 +391,7 @@ def decode_step_bench(dev, reps, with_graph=True, prefill_only=False):
     res["logits_vs_one_kernel_per_op"] = {
         "grouped_gemv_fused_attention": cross(plan_logits[3], plan_logits[0]),
         "split_norms": cross(plan_logits[4], plan_logits[0]),
-        "qkv_and_attention_in_one_call": cross(plan_logits[5], plan_logits[0]),
+        "whole_step_in_one_grid": cross(plan_logits[5], plan_logits[0]),
         **{k: cross(v, plan_logits[0]) for k, v in graph_logits.items()}}
     res["logits_within_1e-4"] = bool(all(v["max_rel"] < 1e-4 and v["l2_rel"] < 1e-4
                                          for v in res["logits_vs_one_kernel_per_op"].values()))
@@ -401,10 +401,10 @@ def decode_step_bench(dev, reps, with_graph=True, prefill_only=False):
     # the same step with the caches kept [n_head][n_ctx][head_dim]: a head's keys contiguous (same weights, same cache
     # contents: the logits are compared with the one-kernel-per-op plan of the [n_ctx][n_embd] decoder above)
     dec, _ = make_decoder(False, True)
-    for name, fused in (("eager_split_norms_head_major_kv", 4), ("eager_qkv_and_attention_in_one_call_head_major_kv", 5)):
+    for name, fused in (("eager_split_norms_head_major_kv", 4), ("eager_whole_step_in_one_grid_head_major_kv", 5)):
         dec.time_steps(tok, n_past, fused, SETTLE_STEPS)
         ms = min(dec.time_steps(tok, n_past, fused, reps) for _ in range(3)) / reps
-        res[name] = {"library_calls": dec.ops_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1),
+        res[name] = {"library_calls": dec.calls_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1),
                      "GBps": round((weight_bytes + kv_bytes) / ms / 1e6, 1),
                      "hbm_frac": round((weight_bytes + kv_bytes) / ms / 1e6 / HBM_PEAK_GBPS, 4),
                      "logits_vs_one_kernel_per_op": cross(dec.logits().astype(np.float64), plan_logits[0])}
@@ -412,11 +412,11 @@ def decode_step_bench(dev, reps, with_graph=True, prefill_only=False):
     # the same step with the KV cache in f16 (the form the reference keeps it in on the GPU): half the cache bytes
     dec, _ = make_decoder(True)
     b16 = weight_bytes + kv_bytes // 2
-    for name, fused in (("eager_split_norms_f16_kv", 4), ("eager_qkv_and_attention_in_one_call_f16_kv", 5)):
+    for name, fused in (("eager_split_norms_f16_kv", 4), ("eager_whole_step_in_one_grid_f16_kv", 5)):
         dec.time_steps(tok, n_past, fused, SETTLE_STEPS)
         ms = min(dec.time_steps(tok, n_past, fused, reps) for _ in range(3)) / reps
         res[name] = {
-            "library_calls": dec.ops_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1),
+            "library_calls": dec.calls_per_step(), "ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1),
             "algorithmic_bytes_per_token": b16, "GBps": round(b16 / ms / 1e6, 1),
             "hbm_frac": round(b16 / ms / 1e6 / HBM_PEAK_GBPS, 4),
             "logits_finite": bool(np.all(np.isfinite(dec.logits())))}

@@ -186,6 +186,8 @@ void *galois_host_llama_tensor(void *m, const char *name, int layer) {
 }
 void *galois_host_llama_logits(void *m) { return (void *)&((LlamaDecoder *)m)->logits(); }
 size_t galois_host_llama_ops_per_step(void *m) { return ((LlamaDecoder *)m)->ops_per_step(); }
+size_t galois_host_llama_calls_per_step(void *m) { return ((LlamaDecoder *)m)->calls_per_step(); }
+size_t galois_host_llama_calls_per_prefill(void *m) { return ((LlamaDecoder *)m)->calls_per_prefill(); }
 int galois_host_llama_decode(void *m, int32_t token, int32_t n_past, int fused) {
     GResult r = ((LlamaDecoder *)m)->decode(token, n_past, fused);
     return r.ok() ? 0 : fail(r);

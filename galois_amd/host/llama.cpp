@@ -277,6 +277,7 @@ GResult LlamaDecoder::whole_step(int32_t token, int32_t n_past, bool *taken) {
     G_TRY(dev_.gpu->check(st));
     *taken = true;
     n_ops_ = 2 + 4 * layers_.size();  // what the step consists of, as it is counted where its calls go out one by one
+    n_calls_ = 1;
     return GError{};
 }
 
@@ -464,7 +465,7 @@ GResult LlamaDecoder::step(int32_t n_past, int fused) {
         G_TRY(norm(x_, out_norm_, a_));
         G_TRY(galois_matmul(output_, a_, logits_)); ops++;
     }
-    n_ops_ = ops;
+    n_ops_ = n_calls_ = ops;
     return GError{};
 }
 

@@ -61,12 +61,14 @@ class LlamaDecoder {
     // token's.  n_embd and n_ff must be multiples of 256; caches [n_embd, n_ctx] (not head-major), f32 or f16.
     // Intermediates are sized for the largest n and n_past + n seen so far (this call allocates when they grow).
     GResult prefill(const int32_t *tokens, size_t n, int32_t n_past);
-    size_t ops_per_prefill() const { return n_prefill_ops_; }  // calls of the last prefill (one or two launches each; q | k | v that
-                                                               // leave their products rotated count as the two calls they stand for)
+    size_t ops_per_prefill() const { return n_prefill_ops_; }  // what the last prefill consists of: q | k | v that leave their products
+                                                               // rotated count as the two calls they stand for
+    size_t calls_per_prefill() const { return n_prefill_calls_; }  // the library calls it went out as (one or two launches each)
     const Tensor &logits() const { return logits_; }
     const LlamaHParams &hparams() const { return hp_; }
-    size_t ops_per_step() const { return n_ops_; }  // calls the last decode step's plan consists of (a call is one or two launches; plan 5 may send
-                                                  // all of them out as one)
+    size_t ops_per_step() const { return n_ops_; }  // what the last decode step's plan consists of, call by call
+    size_t calls_per_step() const { return n_calls_; }  // the library calls it went out as (one or two launches each): 1 where
+                                                        // galois_hip_llama_step took the whole step
 
    private:
     struct Layer {
@@ -94,7 +96,7 @@ class LlamaDecoder {
     GResult prefill_buffers(size_t n, size_t keys);
     Prefill pf_;
     galois_hip_graph *graph_ = nullptr;
-    size_t n_ops_ = 0, n_prefill_ops_ = 0;
+    size_t n_ops_ = 0, n_calls_ = 0, n_prefill_ops_ = 0, n_prefill_calls_ = 0;
     int32_t last_token_ = -1, last_pos_ = -1;
 };
 

@@ -421,6 +421,7 @@ GResult LlamaDecoder::prefill(const int32_t *tokens, size_t n, int32_t n_past) {
         G_TRY(galois_matmul(output_, a_, logits_)); ops += 3;
     }
     n_prefill_ops_ = ops;
+    n_prefill_calls_ = one_launch ? ops - layers_.size() + 1 : ops;  // q | k | v with their rotation are one call; the angles of all layers another
     return GError{};
 }
 

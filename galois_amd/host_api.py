@@ -62,7 +62,8 @@ def lib():
                 ("galois_host_llama_logits", vp, [vp]), ("galois_host_llama_ops_per_step", sz, [vp]),
                 ("galois_host_llama_decode", C.c_int, [vp, C.c_int32, C.c_int32, C.c_int]),
                 ("galois_host_llama_prefill", C.c_int, [vp, C.POINTER(C.c_int32), sz, C.c_int32]),
-                ("galois_host_llama_ops_per_prefill", sz, [vp]),
+                ("galois_host_llama_ops_per_prefill", sz, [vp]), ("galois_host_llama_calls_per_prefill", sz, [vp]),
+                ("galois_host_llama_calls_per_step", sz, [vp]),
                 ("galois_host_llama_time_prefill", C.c_int, [vp, vp, C.POINTER(C.c_int32), sz, C.c_int32, C.c_int,
                                                              C.POINTER(C.c_float)]),
                 ("galois_host_llama_capture", C.c_int, [vp, C.c_int32, C.c_int32, C.c_int]),
@@ -291,6 +292,10 @@ class LlamaDecoder:
     def ops_per_prefill(self):
         return lib().galois_host_llama_ops_per_prefill(self.h)
 
+    def calls_per_prefill(self):
+        """The library calls the last prefill went out as."""
+        return lib().galois_host_llama_calls_per_prefill(self.h)
+
     def time_prefill(self, tokens, n_past, reps):
         t = np.ascontiguousarray(tokens, np.int32)
         ms = C.c_float()
@@ -311,6 +316,10 @@ class LlamaDecoder:
 
     def ops_per_step(self):
         return lib().galois_host_llama_ops_per_step(self.h)
+
+    def calls_per_step(self):
+        """The library calls the last decode step went out as: 1 where the whole step is one grid."""
+        return lib().galois_host_llama_calls_per_step(self.h)
 
     def time_replays(self, n):
         ms = C.c_float()

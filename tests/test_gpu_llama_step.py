@@ -88,6 +88,31 @@ def test_step_equals_the_launches_it_replaces(gdev, kw, positions):
     dec.close()
 
 
+@pytest.mark.parametrize("kw, n_past, grid", [
+    (dict(), 0, True), (dict(), 159, True), (dict(kv_f16=True, kv_head_major=True), 30, True), (dict(n_ff=64, n_vocab=1), 3, True),
+    (dict(n_embd=4096, n_head=32, n_ff=12288, n_layer=1), 100, True), (dict(n_layer=41), 17, True),
+    (dict(n_ctx=8300), 8191, True), (dict(n_ctx=8300), 8192, False),               # 64 splits of 128 f32 keys, 65
+    (dict(n_ctx=8300, kv_f16=True), 8299, True),
+    (dict(n_embd=384, n_head=3), 60, False),                                       # narrower than 512
+    (dict(n_embd=4224, n_head=33, n_layer=1), 9, False),                           # wider than 4096
+    (dict(n_layer=251, n_embd=512, n_ff=64, n_vocab=8, n_ctx=4), 1, False)])
+def test_which_steps_go_out_in_one_grid(gdev, kw, n_past, grid):
+    dec, hp = _decoder(gdev, **kw)
+    dec.decode(0, n_past, 4)
+    assert dec.calls_per_step() == dec.ops_per_step() == 2 + 5 * hp["n_layer"]
+    dec.decode(0, n_past, 5)
+    assert dec.calls_per_step() == (1 if grid else 2 + 4 * hp["n_layer"])
+    gdev.set_option(4, 2)      # a form of q | k | v and attention is asked for: layer by layer
+    try:
+        dec.decode(0, n_past, 5)
+    finally:
+        gdev.set_option(4, 0)
+    assert dec.calls_per_step() == 2 + 4 * hp["n_layer"]
+    dec.capture(0, n_past, 5)
+    assert dec.calls_per_step() == (1 if grid else 2 + 4 * hp["n_layer"])
+    dec.close()
+
+
 def test_steps_repeat_recorded_and_interleaved(gdev):
     """The same bits every time: eager, from a graph with other steps between the replays, and beside another decoder of
     other sizes in the same context."""
