@@ -6,6 +6,8 @@
 // v_mfma_f32_32x32x16_f16 accumulates in f32.
 #include "common.h"
 
+#include <type_traits>
+
 namespace {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -327,12 +329,19 @@ struct gemm_mats {
     // has both products of an element in its registers and stores silu(gate) * up, as fp16, into the panel of the
     // [N[0], M] operand at swiglu_out.  n_total = 96 * ceil(N[0] / 48) then.
     _Float16 *swiglu_out;
-    // q | k | v of heads of 128, each N[0] columns: what leaves the epilogue of the first two is rotated (rope_custom, mode 0,
-    // n_dims 128).  rope: (cos, sin) of row m and pair i of a head at m * 64 + i; kv_f16: the second and third result are
-    // cache rows in f16, rounded to nearest even from the f32 result.  Null: no rotation.
+};
+
+// q | k | v of heads of 128, each N[0] columns: what leaves the epilogue of the first two is rotated (rope_custom, mode 0,
+// n_dims 128).  rope: (cos, sin) of row m and pair i of a head at m * 64 + i; kv_f16: the second and third result are
+// cache rows in f16, rounded to nearest even from the f32 result.  An argument type of its own, and with it kernels of their own, so
+// that the other products keep their registers, code and arguments (in the same kernels the few-rows products took 0.05 to 0.3 us
+// more, 16 x 4096 x 4096 8.4 -> 8.7).
+struct gemm_mats_rope : gemm_mats {
     const float2 *rope;
     int32_t kv_f16;
 };
+template <typename MATS>
+constexpr bool gemm_has_rope = std::is_same<MATS, gemm_mats_rope>::value;
 
 // The rotation of one element x whose neighbour in its pair is p; odd: x is the pair's second.  The same sequence of
 // roundings as rope_f32: one product, then a fused multiply-add.
@@ -525,10 +534,9 @@ __device__ __forceinline__ void gemm_drain_a(gemm_a_regs<RT> &r) {
 
 #define GEMM_LDB(dst, ptr) dst = *reinterpret_cast<const half8_t *>(ptr)
 #define GEMM_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0)
-// ROPE: the launch of q | k | v (mats.rope); a kernel of its own, so that the others keep their registers and code.
-template <int NF, int GN, int RT, bool ROPE>
+template <int NF, int GN, int RT, typename MATS>
 __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float16 *__restrict__ Xh,
-                                              const gemm_mats &mats, int K, int M, int m0, int n0, int wm, int ncol0,
+                                              const MATS &mats, int K, int M, int m0, int n0, int wm, int ncol0,
                                               int nslots, size_t y_off) {
     // Xh: the panel advanced to the workgroup's first k-block; nslots: its stages; y_off: where its results go,
     // relative to Y (a workgroup that holds one share of k of several writes a partial result)
@@ -673,7 +681,7 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
     }
     // q | k | v: a pair of columns is a pair of neighbouring lanes, sixteen columns lie in one matrix.  The angles of a row tile
     // are requested together, and the next one's before they are used (the operands' registers are free now).
-    if constexpr (ROPE) {
+    if constexpr (gemm_has_rope<MATS>) {
         const bool odd = lane & 1;
         const int N = mats.N[0];
         float2 angles[2][NF][4];
@@ -746,8 +754,8 @@ __device__ __forceinline__ void gemm_consumer(const _Float16 *smem, const _Float
     }
 }
 
-template <int GN, int RT, bool ROPE>
-__global__ __launch_bounds__(512) void gemm_q4_0_mfma(const gemm_mats mats, const _Float16 *__restrict__ Xh, int K, int M,
+template <int GN, int RT, typename MATS>
+__global__ __launch_bounds__(512) void gemm_q4_0_mfma(const MATS mats, const _Float16 *__restrict__ Xh, int K, int M,
                                                       int n_tiles, int m_tiles, int splits, size_t split_stride) {
     extern __shared__ __attribute__((aligned(16))) _Float16 smem[];  // [3] B stage | [2] raw | pad
     // XCD-aware tile order: blockIdx % 8 is the XCD; consecutive tiles (same X panel, same share of k) go to one XCD
@@ -766,7 +774,7 @@ __global__ __launch_bounds__(512) void gemm_q4_0_mfma(const gemm_mats mats, cons
     if (wave >= 4)
         gemm_producer<GN>(smem, mats, K, n0, sup0, sup1 - sup0);
     else  // four consumer waves stacked in M, each 16 * RT rows x GN columns; a piece of 256 is 8 KB of a row group's panel
-        gemm_consumer<GN / 16, GN, RT, ROPE>(smem, Xh + (size_t)sup0 * 4096, mats, K, M, m0, n0, wave, 0, (sup1 - sup0) * 4,
+        gemm_consumer<GN / 16, GN, RT>(smem, Xh + (size_t)sup0 * 4096, mats, K, M, m0, n0, wave, 0, (sup1 - sup0) * 4,
                                    (size_t)sp * split_stride);
 }
 
@@ -797,8 +805,8 @@ __global__ __launch_bounds__(256) void gemm_sum_tail(const float *p, const float
 }
 
 // Launch of one tile width.
-template <int GN, int RT>
-int32_t gemm_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int M, int splits = 1,
+template <int GN, int RT, typename MATS>
+int32_t gemm_launch(galois_hip_ctx *ctx, const MATS &mats, const _Float16 *Xh, int K, int M, int splits = 1,
                     size_t split_stride = 0) {
     const int n_tiles = (mats.n_total + GN - 1) / GN;
     const int m_tiles = (M + 64 * RT - 1) / (64 * RT);
@@ -807,9 +815,7 @@ int32_t gemm_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *
     const size_t lds = gemm_cfg<GN>::LDS_BYTES;
     // the attribute lives with the function on the current device: set per launch (a table lookup), which is right
     // for every device and every thread without any flag of our own
-    constexpr bool CAN_ROPE = GN != 64;  // q | k | v never come in shares
-    GH_REQUIRE(ctx, CAN_ROPE || mats.rope == nullptr, GALOIS_HIP_E_UNSUPPORTED, "matmul: no rotation behind tiles of 64 columns");
-    const auto kernel = CAN_ROPE && mats.rope != nullptr ? gemm_q4_0_mfma<GN, RT, CAN_ROPE> : gemm_q4_0_mfma<GN, RT, false>;
+    const auto kernel = gemm_q4_0_mfma<GN, RT, MATS>;
     hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return gh_hip(ctx, e, "hipFuncSetAttribute(LDS size)");
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds, ctx->stream, mats, Xh, K, M, n_tiles, m_tiles, splits, split_stride);
@@ -847,14 +853,20 @@ gemm_tile gemm_pick(const galois_hip_ctx *ctx, int64_t cols, int64_t M, int gn, 
     return best;
 }
 
-int32_t gemm_launch_tile(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int M, const gemm_tile &t, int splits = 1,
+template <typename MATS>
+int32_t gemm_launch_tile(galois_hip_ctx *ctx, const MATS &mats, const _Float16 *Xh, int K, int M, const gemm_tile &t, int splits = 1,
                          size_t split_stride = 0) {
 #define GEMM_RT(GN_)                                                                                   \
     return t.rt == 4   ? gemm_launch<GN_, 4>(ctx, mats, Xh, K, M, splits, split_stride)                \
            : t.rt == 3 ? gemm_launch<GN_, 3>(ctx, mats, Xh, K, M, splits, split_stride)                \
                        : gemm_launch<GN_, 2>(ctx, mats, Xh, K, M, splits, split_stride)
     if (t.gn == 96) GEMM_RT(96);
-    if (t.gn == 64) GEMM_RT(64);
+    if (t.gn == 64) {
+        if constexpr (gemm_has_rope<MATS>)  // q | k | v never come in shares
+            return gh_fail(ctx, GALOIS_HIP_E_UNSUPPORTED, "matmul: no rotation behind tiles of 64 columns");
+        else
+            GEMM_RT(64);
+    }
     GEMM_RT(48);
 #undef GEMM_RT
 }
@@ -869,7 +881,8 @@ void gemm_concat(gemm_mats &mats, int n_mats) {
     mats.n_total = (int32_t)cols;
 }
 
-int32_t gemm_launch_any(galois_hip_ctx *ctx, gemm_mats mats, int n_mats, const _Float16 *Xh, int K, int M) {
+template <typename MATS>
+int32_t gemm_launch_any(galois_hip_ctx *ctx, MATS mats, int n_mats, const _Float16 *Xh, int K, int M) {
     gemm_concat(mats, n_mats);
     if (M <= SK_MAX_ROWS) return skinny_launch_any(ctx, mats, Xh, K, K / 32, M, true);
     const gemm_tile t96 = gemm_pick(ctx, mats.n_total, M, 96), t48 = gemm_pick(ctx, mats.n_total, M, 48);
@@ -1241,7 +1254,7 @@ extern "C" int32_t galois_hip_mul_mat_q4_0_qkv_rope_f16_panel(galois_hip_ctx *ct
                         gh_aligned(q, 16) && gh_aligned(k_rows, 16) && gh_aligned(v_rows, 16),
                GALOIS_HIP_E_ALIGN, "mul_mat_q4_0_qkv_rope_f16_panel: 16-byte aligned operands");
     GH_BIND(ctx);
-    gemm_mats mats = {};
+    gemm_mats_rope mats = {};
     mats.W[0] = (const uint8_t *)W_q, mats.W[1] = (const uint8_t *)W_k, mats.W[2] = (const uint8_t *)W_v;
     mats.Y[0] = q, mats.Y[1] = (float *)k_rows, mats.Y[2] = (float *)v_rows;
     mats.N[0] = mats.N[1] = mats.N[2] = n_head * head_dim;

@@ -154,7 +154,8 @@ constexpr int sk_occ(int nt, int mt, sk_form form) {
 }
 
 // Where four consecutive columns of row m go: n is a column of the concatenated matrices.
-__device__ __forceinline__ void sk_store4(const gemm_mats &mats, int n, int m, float4_t v) {
+template <typename MATS>
+__device__ __forceinline__ void sk_store4(const MATS &mats, int n, int m, float4_t v) {
     if (n >= mats.n_total) return;
     float *Y = mats.Y[0];
     int N = mats.N[0], first = 0;
@@ -163,7 +164,7 @@ __device__ __forceinline__ void sk_store4(const gemm_mats &mats, int n, int m, f
         const bool ge = n >= mats.col0[t];
         Y = ge ? mats.Y[t] : Y, N = ge ? mats.N[t] : N, first = ge ? mats.col0[t] : first;
     }
-    if (mats.rope != nullptr) {  // q | k | v: every matrix has whole sixteens of columns, its rows are 16-byte aligned
+    if constexpr (gemm_has_rope<MATS>) {  // q | k | v: every matrix has whole sixteens of columns, its rows are 16-byte aligned
         if (n < mats.col0[2]) {
             const float4 cs = *reinterpret_cast<const float4 *>(mats.rope + (size_t)m * 64 + (((n - first) & 127) >> 1));
             const float2 c0 = make_float2(cs.x, cs.y), c1 = make_float2(cs.z, cs.w);
@@ -195,8 +196,8 @@ __device__ __forceinline__ void sk_store4(const gemm_mats &mats, int n, int m, f
 
 // K: the rows' true length (a multiple of 32); kp_blocks: 32-k blocks of a panel row, a multiple of 8, zeros past K.
 // With mats.swiglu_out the first NT / 2 tiles are gate rows and the others the same rows of the up matrix.
-template <int NT, int MT, int KS, sk_form FORM>
-__global__ __launch_bounds__(KS * 64, sk_occ(NT, MT, FORM)) void gemm_q4_0_skinny(const gemm_mats mats, const _Float16 *__restrict__ Xh, int K,
+template <int NT, int MT, int KS, sk_form FORM, typename MATS>
+__global__ __launch_bounds__(KS * 64, sk_occ(NT, MT, FORM)) void gemm_q4_0_skinny(const MATS mats, const _Float16 *__restrict__ Xh, int K,
                                                             int kp_blocks, int M, int n_tiles, int m_blocks) {
     constexpr int SG = sk_steps(MT), GROUPS = 8 / SG;  // an even number of groups a piece
     __shared__ __attribute__((aligned(16))) float4_t part[KS][KS][64];
@@ -339,13 +340,13 @@ __global__ __launch_bounds__(KS * 64, sk_occ(NT, MT, FORM)) void gemm_q4_0_skinn
     }
 }
 
-template <int NT, int MT, int KS, sk_form FORM>
-int32_t skinny_launch(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M) {
+template <int NT, int MT, int KS, sk_form FORM, typename MATS>
+int32_t skinny_launch(galois_hip_ctx *ctx, const MATS &mats, const _Float16 *Xh, int K, int kp_blocks, int M) {
     const int cols_per_tile = mats.swiglu_out ? NT / 2 * 16 : NT * 16;
     const int cols = mats.swiglu_out ? mats.N[0] : mats.n_total;
     const int n_tiles = (cols + cols_per_tile - 1) / cols_per_tile, m_blocks = ((M + 15) / 16 + MT - 1) / MT;
     const dim3 grid((unsigned)((n_tiles + 7) / 8 * 8 * m_blocks));
-    hipLaunchKernelGGL((gemm_q4_0_skinny<NT, MT, KS, FORM>), grid, dim3(KS * 64), 0, ctx->stream, mats, Xh, K, kp_blocks, M,
+    hipLaunchKernelGGL((gemm_q4_0_skinny<NT, MT, KS, FORM, MATS>), grid, dim3(KS * 64), 0, ctx->stream, mats, Xh, K, kp_blocks, M,
                        n_tiles, m_blocks);
     return GALOIS_HIP_OK;
 }
@@ -367,8 +368,8 @@ inline double sk_cost(int nt, int mt, bool runs) {
     return 1.55 * nt + mt * (0.78 + 0.25 * nt);
 }
 
-template <int KS, sk_form FORM>
-int32_t skinny_launch_tiles(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, int nt, int mt) {
+template <int KS, sk_form FORM, typename MATS>
+int32_t skinny_launch_tiles(galois_hip_ctx *ctx, const MATS &mats, const _Float16 *Xh, int K, int kp_blocks, int M, int nt, int mt) {
 #define SK_MT(NT_)                                                                                    \
     switch (mt) {                                                                                     \
         case 1: return skinny_launch<NT_, 1, KS, FORM>(ctx, mats, Xh, K, kp_blocks, M);            \
@@ -426,15 +427,18 @@ inline double skinny_us(const galois_hip_ctx *ctx, int N, int K, int M) {
 }
 
 // KS by K alone (the order of the sums): eight waves for long rows, whose pieces keep them busy.  t: tiles the caller has picked.
-int32_t skinny_launch_any(galois_hip_ctx *ctx, const gemm_mats &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned,
+template <typename MATS>
+int32_t skinny_launch_any(galois_hip_ctx *ctx, const MATS &mats, const _Float16 *Xh, int K, int kp_blocks, int M, bool aligned,
                           sk_tiles t = {0, 0, 0.0, false}) {
     const bool swiglu = mats.swiglu_out != nullptr;
     if (t.nt == 0) t = skinny_pick(ctx, swiglu ? 2 * (int64_t)mats.N[0] : mats.n_total, K, M, swiglu, aligned && K % 256 == 0);
     const sk_form form = !aligned ? SK_BLOCKS : t.runs ? SK_RUNS : SK_SLOTS;
+    constexpr sk_form other = gemm_has_rope<MATS> ? SK_SLOTS : SK_BLOCKS;  // q | k | v with their rotation are aligned
+    GH_REQUIRE(ctx, form != SK_BLOCKS || other == SK_BLOCKS, GALOIS_HIP_E_ALIGN, "matmul: rotation behind unaligned weights");
 #define SK_FORM(KS_)                                                                                                     \
     return form == SK_RUNS    ? skinny_launch_tiles<KS_, SK_RUNS>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)            \
            : form == SK_SLOTS ? skinny_launch_tiles<KS_, SK_SLOTS>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)           \
-                              : skinny_launch_tiles<KS_, SK_BLOCKS>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
+                              : skinny_launch_tiles<KS_, other>(ctx, mats, Xh, K, kp_blocks, M, t.nt, t.mt)
     if (K >= 8192) SK_FORM(8);
     SK_FORM(4);
 #undef SK_FORM
