@@ -144,12 +144,14 @@ __device__ __forceinline__ half8_t sk_operand(const uint32_t (&q)[4], half2_t d)
     return __builtin_bit_cast(half8_t, o);
 }
 
-// Instructions of a piece whose activation fragments are requested together: about eight fragments in flight a wave.
-constexpr int sk_steps(int mt) { return mt <= 1 ? 4 : mt <= 4 ? 2 : 1; }
+// Instructions of a piece whose activation fragments are requested together: about eight fragments in flight a wave.  4 x 4
+// tiles whose weights come in runs have registers for half as many only (with two instructions' they spilled five; 56 x 4096 x 14000 22.5 ->
+// 22.0 us, 64 x 1024 x 16384 11.9 -> 11.1).
+constexpr int sk_steps(int nt, int mt, sk_form form) { return mt <= 1 ? 4 : mt <= (nt == 4 && form == SK_RUNS ? 3 : 4) ? 2 : 1; }
 // Waves per SIMD the registers are kept to: four hide the requests' latency where the tiles allow it (2 x 2 tiles: 138 -> 110
 // registers, gate | up at 23 rows 21.4 -> 20.3 us with weights in the Infinity Cache, 25.2 from HBM).
 constexpr int sk_occ(int nt, int mt, sk_form form) {
-    const int regs = 4 * nt * mt + 8 * sk_steps(mt) * mt + (form == SK_RUNS ? 22 : 19) * nt + 40;
+    const int regs = 4 * nt * mt + 8 * sk_steps(nt, mt, form) * mt + (form == SK_RUNS ? 22 : 19) * nt + 40;
     return regs <= 138 ? 4 : regs <= 175 ? 3 : 2;
 }
 
@@ -199,7 +201,7 @@ __device__ __forceinline__ void sk_store4(const MATS &mats, int n, int m, float4
 template <int NT, int MT, int KS, sk_form FORM, typename MATS>
 __global__ __launch_bounds__(KS * 64, sk_occ(NT, MT, FORM)) void gemm_q4_0_skinny(const MATS mats, const _Float16 *__restrict__ Xh, int K,
                                                             int kp_blocks, int M, int n_tiles, int m_blocks) {
-    constexpr int SG = sk_steps(MT), GROUPS = 8 / SG;  // an even number of groups a piece
+    constexpr int SG = sk_steps(NT, MT, FORM), GROUPS = 8 / SG;  // an even number of groups a piece
     __shared__ __attribute__((aligned(16))) float4_t part[KS][KS][64];
     static_assert(sizeof(part[0]) >= 16 * SK_PIECE, "a wave's tile of weights lies in its share of the sums' LDS");
     // blockIdx % 8 is the XCD: the row blocks of one weight tile follow one another on it, so the second reads its

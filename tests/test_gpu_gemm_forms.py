@@ -55,3 +55,9 @@ def test_wide_products_have_the_bits_of_their_columns(dev, k, n, ms):
         for b in (xb, yb, zb):
             dev.free(b)
     dev.free(wb)
+
+
+@pytest.mark.parametrize("k, n", [(1024, 12288), (2304, 12800), (8192, 16384)])
+def test_four_weight_tiles_by_four_row_tiles(dev, k, n):
+    """49 to 64 rows of 12288 to 16384 columns: the widest tiles a wave has, with four and with eight waves a workgroup."""
+    test_wide_products_have_the_bits_of_their_columns(dev, k, n, (49, 63, 64))
