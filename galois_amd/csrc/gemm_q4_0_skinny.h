@@ -365,8 +365,10 @@ constexpr int SK_MAX_ROWS = 80;
 
 // Time of a workgroup relative to others, us at K = 4096 (fitted within 10 %): what a weight tile costs
 // (its bytes, its dequantisation), what a row tile costs (its fragments) and their products.  runs: by the form of the weights.
-inline double sk_cost(int nt, int mt, bool runs) {
-    if (runs) return nt == 1 ? 2.0 + 1.12 * mt : nt == 2 ? 3.6 + 1.05 * mt : nt == 3 ? 5.0 + 1.3 * mt : 6.5 + 1.72 * mt;
+// One weight tile under many row tiles gains nothing from runs at eight waves (40 x 11008 x 4096: 1 x 3 tiles 22.3 us in slots, 23.1 in
+// runs, 2 x 2 20.4).
+inline double sk_cost(int nt, int mt, bool runs, int K) {
+    if (runs) return nt == 1 ? 2.0 + (K >= 8192 && mt >= 3 ? 1.25 : 1.12) * mt : nt == 2 ? 3.6 + 1.05 * mt : nt == 3 ? 5.0 + 1.3 * mt : 6.5 + 1.72 * mt;
     return 1.55 * nt + mt * (0.78 + 0.25 * nt);
 }
 
@@ -401,19 +403,29 @@ inline sk_tiles skinny_pick(const galois_hip_ctx *ctx, int64_t cols, int K, int 
     for (int m = 1; m <= SK_MAX_MT && m <= t; m++)
         for (int n = swiglu ? 2 : 1; n <= 4; n += swiglu ? 2 : 1) {
             // three tiles a wave fill the device where two leave a second round nearly empty (77 x 3200 x 8640: 180 workgroups
-            // instead of 270 or 135; 12288 columns: 256); short rows are better off in more rounds
-            if (n == 3 && K <= (m == 1 ? 2560 : 512)) continue;
+            // instead of 270 or 135; 12288 columns: 256); not where that splits rows that one workgroup could take, unless they are long and come in
+            // runs (72 x 1408 x 4183 11.8 us as two blocks of 3 x 3 tiles, 11.0 as one of 2 x 5; 74 x 4000 x 5277 17.3 / 16.4; 80 x 768 x 5463 9.7 /
+            // 9.1; but 80 x 2048 x 5632 11.4 / 12.0, 56 x 11008 x 5120 27.0 / 30.9).  Short rows are better off in more rounds (beyond 80 rows up to K = 1216: 177 x 1216 x 6951 16.6 us in
+            // three tiles, 15.9 without; 355 x 608 x 4533 16.0, 14.5), up to sixteen rows the longer the fewer columns there are (us in three tiles / in one: 16 x 3328 x 9216 12.6 / 11.4,
+            // x 12288 13.8 / 13.7; 16 x 3584 x 10240 12.7 / 11.9, x 12288 14.3 / 15.3; 16 x 4096 x 8640 12.7 / 12.1, x 11008 14.3 / 15.7; 16 x 4352 x
+            // 8640 14.0 / 13.1, x 9216 14.8 / 14.9)
+            if (n == 3 && ((m < t && t <= SK_MAX_MT && (!whole || K < 2048)) ||
+                           (m > 1 ? K <= (t <= SK_MAX_MT ? 512 : 1216) : K <= 2560 || (double)cols < (double)cus * (37.0 + (4352 - K) * 3 / 256.0))))
+                continue;
             const int64_t tiles = (cols + 16 * n - 1) / (16 * n), blocks = (t + m - 1) / m;
             // The weight tiles are dealt to eight XCDs (blockIdx % 8), so a launch runs as long as its fullest XCD, which may hold
             // more workgroups than CUs where the device as a whole does not (524 x 8192 x 1792: 28 tiles of nine row blocks,
             // 36 workgroups on four of the XCDs, 52 us against 32 with other tiles).  With very many rows that evens out.
             const int64_t wgs = (t < 64 ? (tiles + 7) / 8 * 8 : tiles) * blocks;
             // Runs pay where a CU has more to do than one workgroup's chain of requests, whose LDS trip they lengthen: long rows
-            // (eight waves), a second workgroup, three or four weight tiles a wave (over 500 sizes 3 to 6 % each; elsewhere -3 to 0 %).
+            // (eight waves), a second workgroup, three or four weight tiles a wave (over 500 sizes 3 to 6 % each; elsewhere -3 to 0 %); not with
+            // two pieces a row, a wave's only one (3 x 512 x 8653 6.9 us in runs, 6.7 in slots).
             // Workgroups that share a CU then overlap a little.
             double rounds = (double)((wgs + cus - 1) / cus);
-            const bool runs = whole && (K >= 8192 || wgs > cus || n >= 3);
-            const double cost = rounds * (runs && K < 8192 && rounds > 1 ? rounds > 2 ? 0.85 : 0.9 : 1.0) * sk_cost(n, m, runs);
+            // Four by four tiles have fewer fragments in flight with runs than with slots, which costs more than it gains where four
+            // waves have long rows (64 x 4608 x 14500 24.3 us in runs, 25.2 in slots, x 7424 35.5 / 34.4; eight waves, x 9472 38.7 / 40.6).
+            const bool runs = whole && K > 512 && (K >= 8192 || wgs > cus || n >= 3) && !(n == 4 && m == 4 && K > 5120 && K < 8192);
+            const double cost = rounds * (runs && K < 8192 && rounds > 1 ? rounds > 2 ? 0.85 : 0.9 : 1.0) * sk_cost(n, m, runs, K);
             if (best.nt == 0 || cost < best.cost) best = {n, m, cost, runs};
         }
     return best;
