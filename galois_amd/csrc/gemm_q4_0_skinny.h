@@ -144,10 +144,13 @@ __device__ __forceinline__ half8_t sk_operand(const uint32_t (&q)[4], half2_t d)
     return __builtin_bit_cast(half8_t, o);
 }
 
-// Instructions of a piece whose activation fragments are requested together: about eight fragments in flight a wave.  4 x 4
-// tiles whose weights come in runs have registers for half as many only (with two instructions' they spilled five; 56 x 4096 x 14000 22.5 ->
-// 22.0 us, 64 x 1024 x 16384 11.9 -> 11.1).
-constexpr int sk_steps(int nt, int mt, sk_form form) { return mt <= 1 ? 4 : mt <= (nt == 4 && form == SK_RUNS ? 3 : 4) ? 2 : 1; }
+// Instructions of a piece whose activation fragments are requested together: about eight fragments in flight a wave.  Two and four
+// weight tiles under four row tiles have half as many where weights come in runs: 4 x 4 spilled five registers with two instructions'
+// (56 x 4096 x 14000 22.5 -> 22.0 us, 64 x 1024 x 16384 11.9 -> 11.1); 2 x 4, chosen from K = 8192 on, took 173, a wave per SIMD less
+// than in slots, and takes 141 (64 x 11008 x 6848 31.8 -> 29.8 us, 52 x 8192 x 6752 24.5 -> 23.2; 28 sizes 4.7 to 6.3 % less).
+constexpr int sk_steps(int nt, int mt, sk_form form) {
+    return mt <= 1 ? 4 : mt <= (nt % 2 == 0 && form == SK_RUNS ? 3 : 4) ? 2 : 1;
+}
 // Waves per SIMD the registers are kept to: four hide the requests' latency where the tiles allow it (2 x 2 tiles: 138 -> 110
 // registers, gate | up at 23 rows 21.4 -> 20.3 us with weights in the Infinity Cache, 25.2 from HBM).
 constexpr int sk_occ(int nt, int mt, sk_form form) {

@@ -26,6 +26,7 @@ def _dequant(b):
     (2304, 8200, (1, 16, 17, 33, 64, 80)),     # nine pieces of 256: waves with two and three
     (256, 12288, (5, 48)),                      # one piece: three of the four waves have none
     (8192, 3000, (3, 40, 77)),                  # eight waves a workgroup, runs at any width
+    (8192, 6752, (52, 64)),                     # tiles of two by four
     (8448, 8209, (20,)),
     (3200, 8640, (2, 77)),                      # rows that are not whole pieces: slots
     (2400, 8640, (18, 50)),                     # an odd number of blocks

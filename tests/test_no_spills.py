@@ -27,20 +27,35 @@ def _code_objects(blob):
         at = blob.find(MAGIC, at + 1)
 
 
-@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
-def test_no_kernel_spills_registers(tmp_path):
+def _kernels(tmp_path):
+    """(name, its entry in the notes) of every kernel of the library."""
     with open(_abi.LIB_PATH, "rb") as f:
         blob = f.read()
-    seen, spilled = 0, {}
     for i, code in enumerate(_code_objects(blob)):
         path = tmp_path / ("%d.co" % i)
         path.write_bytes(code)
         notes = subprocess.check_output([READELF, "--notes", str(path)], text=True)
         for kernel in re.split(r"\n  - (?=\.)", notes)[1:]:
-            name, count = re.search(r"\.name:\s+(\S+)", kernel), re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel)
-            if name and count:
-                seen += 1
-                if int(count.group(1)):
-                    spilled[name.group(1)] = int(count.group(1))
-    assert seen >= 200, "the library's kernels were not found"
+            name = re.search(r"\.name:\s+(\S+)", kernel)
+            if name and ".vgpr_count:" in kernel:
+                yield name.group(1), kernel
+
+
+def _field(kernel, name):
+    return int(re.search(r"\.%s:\s+(\d+)" % name, kernel).group(1))
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_no_kernel_spills_registers(tmp_path):
+    kernels = list(_kernels(tmp_path))
+    assert len(kernels) >= 200, "the library's kernels were not found"
+    spilled = {name: _field(k, "vgpr_spill_count") for name, k in kernels if _field(k, "vgpr_spill_count")}
     assert not spilled, spilled
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_few_rows_tiles_of_two_by_four_keep_three_waves_a_simd(tmp_path):
+    """However the weights arrive: 168 registers are what a SIMD's 512 have for each of three waves (in eights)."""
+    regs = {name: _field(k, "vgpr_count") for name, k in _kernels(tmp_path) if "gemm_q4_0_skinnyILi2ELi4E" in name}
+    assert len(regs) >= 6, regs
+    assert max(regs.values()) <= 168, regs
