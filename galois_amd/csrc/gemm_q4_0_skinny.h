@@ -14,7 +14,7 @@
 //     request, from L2 (every workgroup reads the whole panel: NT rows of tiles share a fragment).
 //   - The result tile has the weight rows down its registers: a lane holds four consecutive columns of Y.
 // Measured (MI355X, us, weights from HBM, against the 256-row tile): see SK_MAX_ROWS.  77 rows of a 3200 x 8640 matrix through
-// the f32 entry point 93 -> 17.6 (the generic kernel before), a prefill of 23 tokens through 32 layers 4705 -> 2505.
+// the f32 entry point 93 -> 17.6 to 17.9 (the generic kernel before), a prefill of 23 tokens through 32 layers 4705 -> 2490.
 // Weights are rounded exactly as in the main kernel ((q - 8) * d, once, to fp16), sums are f32.
 #pragma once
 
