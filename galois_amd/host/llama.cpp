@@ -288,9 +288,19 @@ GResult LlamaDecoder::check_inputs(int32_t token, int32_t n_past) const {
     return GError{};
 }
 
+// Whether token and position are the ones on the device.  Others are refused while a graph of the caller's is recorded: they would be on
+// the device only once it runs, and again whenever it does, and a later step would take them for its own.
+GResult LlamaDecoder::inputs_there(int32_t token, int32_t n_past, bool *there) {
+    *there = token == last_token_ && n_past == last_pos_;
+    if (*there) return GError{};
+    return dev_.gpu->check(galois_hip_htod_sync_copy(dev_.gpu->ctx(), tok_id_.data(), &token, 0));  // no bytes: only whether a capture is open
+}
+
 GResult LlamaDecoder::set_inputs(int32_t token, int32_t n_past) {
+    bool there = false;
     G_TRY(check_inputs(token, n_past));
-    if (token != last_token_ || n_past != last_pos_)
+    G_TRY(inputs_there(token, n_past, &there));
+    if (!there)
         G_TRY(dev_.gpu->check(galois_hip_store_i32_pair(dev_.gpu->ctx(), (int32_t *)tok_id_.data(), token, (int32_t *)pos_.data(), n_past)));
     last_token_ = token, last_pos_ = n_past;
     return GError{};
@@ -472,9 +482,10 @@ GResult LlamaDecoder::step(int32_t n_past, int fused) {
 
 GResult LlamaDecoder::decode(int32_t token, int32_t n_past, int fused) {
     if (fused >= 5) {  // the call stores token and position on the device itself
+        bool there = false, taken = false;
         G_TRY(check_inputs(token, n_past));
-        bool taken = false;
-        G_TRY(whole_step(token, n_past, &taken));
+        G_TRY(inputs_there(token, n_past, &there));
+        G_TRY(whole_step(there ? -1 : token, n_past, &taken));
         if (taken) {
             last_token_ = token, last_pos_ = n_past;
             return GError{};

@@ -75,6 +75,7 @@ class LlamaDecoder {
         Tensor attn_norm, ffn_norm, wq, wk, wv, wo, w_gate, w_up, w_down, k_cache, v_cache;
     };
     GResult check_inputs(int32_t token, int32_t n_past) const;
+    GResult inputs_there(int32_t token, int32_t n_past, bool *there);
     GResult set_inputs(int32_t token, int32_t n_past);
     void step_model(galois_hip_llama_model *m, std::vector<galois_hip_llama_layer> *layers);
     GResult whole_step(int32_t token, int32_t n_past, bool *taken);
